@@ -1,0 +1,406 @@
+"""Timed cases of the routed-expert MoE layer on one GPU, through the entry points that an engine
+calls: g53h_moe on device tensors (include/g53h.h), and the reference-signature glm53f_moe and
+glm53f_mm_batch (include/glm53f.h), the former on host tensors over the HBM expert cache.
+
+A case is a dict of plain values:
+
+  kind    "layer"   one g53h_moe call, every expert resident in HBM
+          "mm"      one glm53f_mm_batch call on device operands
+          "dropin"  one token step or one prompt through `layers` glm53f_moe calls, experts served
+                    by the HBM cache and all resident, activations in host memory
+  layout  how the expert codes lie in HBM: "rowmajor" (as a checkpoint holds them), "tiled"
+          (octet-tiled, bit-exact decode), "mtiled" (MFMA-tiled, matrix-core decode), "int4m"
+          (routed experts int4, MFMA-tiled); for "dropin" the cache's slots, "tiled" or "mtiled"
+  T, E, I, NE, K   tokens, hidden, intermediate, routed experts, experts per token
+  skew    whether expert popularity is Zipf-like instead of uniform
+
+Weights are N(0, 0.02) quantised to E4M3 by the absmax of each 128 x 128 block (int4: by the
+absmax of each 64 columns of a row), activations bf16 values N(0, 1) as a norm layer gives them,
+the router bf16 with logits N(0, 1), as in the repository's configurations. There is always one
+shared expert. Everything follows from the seed, by torch alone.
+"""
+import ctypes as C
+import math
+import os
+import sys
+
+import numpy as np
+import torch
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "glm-5.3-flash-in-c_amd"))
+
+import glm53h  # noqa: E402
+from glm53h import G53hExpert, G53hMat, G53hMoeLayer, Glm53fMat, check  # noqa: E402
+
+ROUTED_SCALE, LIMIT, SIGMA = 2.5, 10.0, 0.02
+POOL = 24               # distinct host experts behind a drop-in cache; keys share them in turn
+PREFETCH = 6            # next-layer experts hinted per decode token, the reference CLI's default
+BIG = dict(E=4096, I=2048, NE=288, K=8)
+
+
+def listed():
+    return [
+        # one sequence being generated, the default expert layout for speed
+        dict(name="decode_mtiled", kind="layer", layout="mtiled", T=1, skew=False, **BIG),
+        # the same where the output must equal the reference's bit for bit
+        dict(name="decode_tiled", kind="layer", layout="tiled", T=1, skew=False, **BIG),
+        # the same with the engine's int4 experts
+        dict(name="decode_int4", kind="layer", layout="int4m", T=1, skew=False, **BIG),
+        # the repository's smallest configuration: a toy model, bound by launches
+        dict(name="small_layer", kind="layer", layout="rowmajor", T=8, skew=False, E=256, I=128, NE=16, K=8),
+        # a handful of sequences generated together, or one with drafted tokens
+        dict(name="batch_5", kind="layer", layout="tiled", T=5, skew=False, **BIG),
+        # batched decode with uneven expert popularity
+        dict(name="batch_64", kind="layer", layout="tiled", T=64, skew=True, **BIG),
+        # a short prompt over experts as a checkpoint holds them
+        dict(name="prompt_150_rowmajor", kind="layer", layout="rowmajor", T=150, skew=False, **BIG),
+        # a longer, ragged prompt on a smaller model
+        dict(name="prompt_701_mid", kind="layer", layout="tiled", T=701, skew=True, E=2048, I=1024, NE=64, K=6),
+        # a full prefill chunk
+        dict(name="prefill_2048", kind="layer", layout="tiled", T=2048, skew=False, **BIG),
+        # a dense FP8 projection of the engine for a few tokens
+        dict(name="mm_24", kind="mm", T=24, rows=4096, cols=2048),
+        # one token step of the C engine: two layers, host activations, cached experts
+        dict(name="dropin_decode", kind="dropin", layout="tiled", T=1, layers=2, skew=True, **BIG),
+        # a prompt through the C engine: one layer, host activations, cached experts
+        dict(name="dropin_prompt_150", kind="dropin", layout="tiled", T=150, layers=1, skew=True, **BIG),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return max(lo, min(hi, int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))))
+
+
+def draw(rng):
+    kind = rng.choice(["decode", "decode", "batch", "batch", "batch", "batch", "small", "mm", "dropin", "dropin"])
+    skew = rng.random() < 0.5
+    if kind == "decode":
+        return dict(kind="layer", layout=rng.choice(["mtiled", "tiled", "int4m", "rowmajor"]), T=1, skew=skew,
+                    E=4096, I=2048, NE=_log_int(rng, 32, 288), K=rng.choice([4, 6, 8, 8, 10]))
+    if kind == "batch":
+        E, inter = rng.choice([(4096, 2048), (4096, 2048), (2048, 1024), (4096, 1024), (1024, 512)])
+        return dict(kind="layer", layout=rng.choice(["tiled", "tiled", "rowmajor"]), T=_log_int(rng, 2, 2000),
+                    skew=skew, E=E, I=inter, NE=_log_int(rng, 24, 288), K=rng.choice([4, 6, 8]))
+    if kind == "small":
+        return dict(kind="layer", layout="rowmajor", T=_log_int(rng, 1, 64), skew=skew, E=rng.choice([256, 384, 1024]),
+                    I=rng.choice([128, 256, 384]), NE=_log_int(rng, 12, 64), K=rng.choice([2, 4, 8]))
+    if kind == "mm":
+        return dict(kind="mm", T=_log_int(rng, 1, 64), rows=_log_int(rng, 100, 4096), cols=_log_int(rng, 100, 4096))
+    return dict(kind="dropin", layout=rng.choice(["tiled", "mtiled"]), T=rng.choice([1, 1, _log_int(rng, 2, 192)]),
+                layers=1, skew=skew, E=4096, I=2048, NE=_log_int(rng, 32, 160), K=8)
+
+
+# ------------------------------------------------------------------ inputs from a seed ----
+def _gen(seed, stream):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(int(seed) * 64 + stream)
+    return g
+
+
+def _fp8(g, n, rows, cols):
+    """n matrices rows x cols as E4M3 codes [n][rows][cols] and block scales."""
+    br, bc = -(-rows // 128), -(-cols // 128)
+    w = torch.randn((n, br, 128, bc, 128), generator=g, device="cuda").mul_(SIGMA)
+    scale = w.abs().amax(dim=(2, 4), keepdim=True).div_(448.0)
+    q = w.div_(scale).clamp_(-448.0, 448.0).to(torch.float8_e4m3fn).view(torch.uint8)
+    q = q.view(n, br * 128, bc * 128)[:, :rows, :cols].contiguous()
+    return q, scale.view(n, br, bc).contiguous()
+
+
+def _int4(g, n, rows, cols):
+    """n matrices rows x cols as packed levels [n][rows][cols / 2] (even column in the low nibble,
+    offset 8) and steps [n][rows][cols / 64]."""
+    w = torch.randn((n, rows, cols // 64, 64), generator=g, device="cuda").mul_(SIGMA)
+    step = w.abs().amax(dim=3, keepdim=True).div_(7.0)
+    lv = w.div_(step).round_().clamp_(-8.0, 7.0).add_(8.0).to(torch.uint8).view(n, rows, cols)
+    return (lv[..., 0::2] | (lv[..., 1::2] << 4)).contiguous(), step.view(n, rows, cols // 64).contiguous()
+
+
+def _experts(case, seed, n, int4=False, stream=8):
+    """n experts in groups: yields (first, [gate, up, down]), each matrix as (codes, scales)."""
+    E, inter = case["E"], case["I"]
+    g, make = _gen(seed, stream), _int4 if int4 else _fp8
+    step = max(1, (1 << 26) // (E * inter))
+    for e in range(0, n, step):
+        m = min(step, n - e)
+        yield e, [make(g, m, inter, E), make(g, m, inter, E), make(g, m, E, inter)]
+
+
+def _routing(case, seed, layer=0):
+    """Router [NE][E] bf16 and selection bias [NE] of a layer."""
+    E, NE = case["E"], case["NE"]
+    g = _gen(seed, 16 + 2 * layer)
+    router = (torch.randn((NE, E), generator=g, device="cuda") / math.sqrt(E)).to(torch.bfloat16)
+    if not case["skew"]:
+        return router, torch.rand(NE, generator=g, device="cuda").mul_(0.2).sub_(0.1)
+    # a bias by popularity rank that makes the selection about min(1, c rank^-1.1)
+    rank = torch.randperm(NE, generator=g, device="cuda").float()
+    return router, torch.where(rank > 0, 0.64 * rank.clamp(min=1.0).pow(-0.53) - 1.04, torch.zeros_like(rank))
+
+
+def _tokens(case, seed, layer=0):
+    g = _gen(seed, 17 + 2 * layer)
+    return torch.randn((case["T"], case["E"]), generator=g, device="cuda").to(torch.bfloat16).float()
+
+
+# ----------------------------------------------------------------------------- prepare ----
+def prepare(case, seed):
+    glm53h.init(0)
+    return {"layer": _prepare_layer, "mm": _prepare_mm, "dropin": _prepare_dropin}[case["kind"]](case, seed)
+
+
+def _mats(case, codes, scales, e, flags, int4):
+    """The descriptor of expert e whose matrices lie in stacked tensors."""
+    shapes = [(case["I"], case["E"]), (case["I"], case["E"]), (case["E"], case["I"])]
+    bc = 64 if int4 else 128
+    return G53hExpert(*[G53hMat(codes[m][e].data_ptr(), scales[m][e].data_ptr(), r, c, 1 if int4 else 128, bc,
+                                -(-c // bc), flags) for m, (r, c) in enumerate(shapes)])
+
+
+def _stack(case, seed, n, layout, stream):
+    """n experts in HBM in the given layout: codes and scales of the three matrices, stacked."""
+    L, E, inter = glm53h.lib(), case["E"], case["I"]
+    int4 = layout == "int4m"
+    shapes, per = [(inter, E), (inter, E), (E, inter)], 2 if int4 else 1
+    codes = [torch.empty((n, r, c // per), dtype=torch.uint8, device="cuda") for r, c in shapes]
+    scales = [torch.empty((n, r, c // 64) if int4 else (n, -(-r // 128), -(-c // 128)), device="cuda")
+              for r, c in shapes]
+    for e, mats in _experts(case, seed, n, int4, stream):
+        for m, (q, s) in enumerate(mats):
+            k, (r, c) = len(q), shapes[m]
+            if layout == "rowmajor":
+                codes[m][e:e + k], scales[m][e:e + k] = q, s
+                continue
+            if not int4:
+                scales[m][e:e + k] = s
+            torch.cuda.synchronize()
+            for i in range(k):
+                dst, src = codes[m][e + i].data_ptr(), q[i].data_ptr()
+                if int4:
+                    check(L.g53h_mtile_i4(dst, scales[m][e + i].data_ptr(), src, s[i].data_ptr(), r, c, 0), "mtile_i4")
+                elif layout == "mtiled":
+                    check(L.g53h_mtile_f8(dst, src, r, c, 0), "mtile_f8")
+                else:
+                    check(L.g53h_tile_f8(dst, src, r, c), "tile_f8")
+            check(L.g53h_sync(), "sync")
+    return codes, scales
+
+
+def _prepare_layer(case, seed):
+    T, E, inter, NE, K, layout = (case[k] for k in ("T", "E", "I", "NE", "K", "layout"))
+    int4 = layout == "int4m"
+    codes, scales = _stack(case, seed, NE, layout, 8)
+    sh_layout = "mtiled" if int4 else layout
+    sh_codes, sh_scales = _stack(case, seed, 1, sh_layout, 9)
+    fp8_flags = {"rowmajor": 0, "tiled": 2, "mtiled": 8}[sh_layout]
+    descs = (G53hExpert * (NE + 1))(*[_mats(case, codes, scales, e, 12 if int4 else fp8_flags, int4) for e in range(NE)],
+                                    _mats(case, sh_codes, sh_scales, 0, fp8_flags, False))
+    table = torch.from_numpy(np.frombuffer(bytes(descs), np.uint8).copy()).cuda()
+    router, bias = _routing(case, seed)
+    x = _tokens(case, seed)
+    out = torch.empty((T, E), device="cuda")
+    idx = torch.empty((T, K), dtype=torch.int32, device="cuda")
+    w = torch.empty((T, K), device="cuda")
+    layer = G53hMoeLayer(hidden=E, inter=inter, n_experts=NE, topk=K, norm_topk=1, routed_scale=ROUTED_SCALE,
+                         swiglu_limit=LIMIT, router=router.data_ptr(), router_dt=1, bias=bias.data_ptr(),
+                         experts=table.data_ptr(), shared=table.data_ptr() + NE * C.sizeof(G53hExpert), block_c=128,
+                         tiled={"rowmajor": 0, "tiled": 1, "mtiled": 2, "int4m": 4}[layout])
+    torch.cuda.synchronize()
+    L = glm53h.lib()
+    args = (out.data_ptr(), x.data_ptr(), T, C.byref(layer), idx.data_ptr(), w.data_ptr())
+    keep = (codes, scales, sh_codes, sh_scales, table, router, bias, x, layer)
+    return dict(kind="layer", call=L.g53h_moe, args=args, out=dict(out=out, idx=idx, w=w), keep=keep)
+
+
+def _prepare_mm(case, seed):
+    T, rows, cols = case["T"], case["rows"], case["cols"]
+    codes, scales = _fp8(_gen(seed, 8), 1, rows, cols)
+    x = torch.randn((T, cols), generator=_gen(seed, 17), device="cuda").to(torch.bfloat16).float()
+    y = torch.empty((T, rows), device="cuda")
+    mat = Glm53fMat(codes.data_ptr(), scales.data_ptr(), glm53h.GLM53F_WF8, rows, cols, 128, 128, -(-cols // 128))
+    torch.cuda.synchronize()
+    return dict(kind="mm", call=glm53h.lib().glm53f_mm_batch, args=(y.data_ptr(), x.data_ptr(), T, C.byref(mat)),
+                out=y, keep=(codes, scales, x, mat))
+
+
+class _Cache:
+    """An HBM expert cache over host experts, with every expert of `layers` layers read in."""
+
+    def __init__(self, case, pool, layers):
+        L, NE, E, inter = glm53h.lib(), case["NE"], case["E"], case["I"]
+        self.cfg = glm53h.Glm53fCfg()
+        self.cfg.hidden, self.cfg.n_layers, self.cfg.n_experts, self.cfg.topk = E, layers, NE, case["K"]
+        self.cfg.n_shared, self.cfg.moe_inter, self.cfg.routed_scale, self.cfg.norm_topk = 1, inter, ROUTED_SCALE, 1
+        self.cfg.swiglu_limit, self.cfg.fp8_block_r, self.cfg.fp8_block_c = LIMIT, 128, 128
+
+        def view(_store, layer, expert, out):
+            q, p = out.contents, pool[(layer * NE + expert) % POOL]
+            q.gate, q.up, q.down = [_host_mat(c, s) for c, s in p]
+            return 0
+
+        self.store = glm53h.G53hStore(glm53h.VIEW_FN(view), glm53h.DONE_FN(), None)
+        self.cache, self.pool, self.open = glm53h.Glm53fCache(), pool, False
+        slot = 3 * E * inter + (2 * (inter // 128) * (E // 128) + (E // 128) * (inter // 128)) * 4 + 8192
+        was = os.environ.pop("GLM53F_CACHE_MFMA", None)
+        if case["layout"] == "mtiled":
+            os.environ["GLM53F_CACHE_MFMA"] = "1"          # read by the cache at its start
+        try:
+            check(L.g53h_cache_init_store(C.byref(self.cache), C.byref(self.store), C.byref(self.cfg),
+                                          slot * (layers * NE + 2), 0, 0), "cache")
+            self.open = True
+        finally:
+            os.environ.pop("GLM53F_CACHE_MFMA", None)
+            if was is not None:
+                os.environ["GLM53F_CACHE_MFMA"] = was
+        src = self.cache.src
+        for layer in range(layers):
+            for e in range(0, NE, 16):
+                ids = (C.c_int * 16)(*range(e, min(e + 16, NE)))
+                src.getmany(C.byref(src), layer, ids, min(16, NE - e))
+        check(L.glm53f_cache_sync(C.byref(self.cache)), "cache sync")
+
+    def __del__(self):
+        if self.open:
+            glm53h.lib().glm53f_cache_free(C.byref(self.cache))
+
+
+def _host_mat(codes, scales):
+    rows, cols = codes.shape
+    return Glm53fMat(codes.data_ptr(), scales.data_ptr(), glm53h.GLM53F_WF8, rows, cols, 128, 128, scales.shape[1])
+
+
+def _host_pool(case, seed, n, stream):
+    """n experts in pinned host memory: [expert][matrix] (codes, scales)."""
+    pool = []
+    for _, mats in _experts(case, seed, n, stream=stream):
+        host = [[t.cpu().pin_memory() for t in m] for m in mats]
+        pool += [[(q[i], s[i]) for q, s in host] for i in range(len(host[0][0]))]
+    return pool
+
+
+def _prepare_dropin(case, seed):
+    T, E, layers = case["T"], case["E"], case["layers"]
+    pool = _host_pool(case, seed, POOL, 8)
+    shared = _host_pool(case, seed, layers, 9)
+    routing = [[t.float().cpu().numpy() for t in _routing(case, seed, layer)] for layer in range(layers)]
+    torch.cuda.synchronize()
+    cache = _Cache(case, pool, layers)
+    ws, xs, outs = [], [], []
+    for layer in range(layers):
+        w = glm53h.Glm53fMoeW()
+        w.gate, w.bias = (a.ctypes.data for a in routing[layer])
+        w.sh_gate, w.sh_up, w.sh_down = [_host_mat(c, s) for c, s in shared[layer]]
+        w.src, w.layer, w.prefetch_n = C.pointer(cache.cache.src), layer, PREFETCH
+        if layer + 1 < layers:
+            w.next_gate, w.next_bias = (a.ctypes.data for a in routing[layer + 1])
+        ws.append(w)
+        xs.append(_tokens(case, seed, layer).cpu().numpy())
+        outs.append(np.zeros((T, E), np.float32))
+    calls = [(o.ctypes.data, x.ctypes.data, C.byref(w), C.byref(cache.cfg), T, None) for o, x, w in zip(outs, xs, ws)]
+    return dict(kind="dropin", call=glm53h.lib().glm53f_moe, calls=calls, out=outs, keep=(cache, shared, routing, ws, xs))
+
+
+# --------------------------------------------------------------------------------- run ----
+def run(state):
+    if state["kind"] == "layer":
+        check(state["call"](*state["args"]), "g53h_moe")
+    elif state["kind"] == "mm":
+        state["call"](*state["args"])
+    else:
+        for args in state["calls"]:
+            state["call"](*args)
+    return state["out"]
+
+
+# -------------------------------------------------------------------------------- work ----
+def _expert_bytes(case, int4=False):
+    n = case["E"] * case["I"]
+    return 3 * (n // 2 + n // 16) if int4 else 3 * (n + n // 4096)
+
+
+def _distinct(case):
+    """Expected distinct routed experts of T tokens."""
+    NE, K, T = case["NE"], case["K"], case["T"]
+    if not case["skew"]:
+        p = [K / NE] * NE
+    else:
+        lo, hi = 0.0, float(NE)
+        for _ in range(60):                                  # c with sum min(1, c rank^-1.1) = K
+            c = (lo + hi) / 2
+            lo, hi = (c, hi) if sum(min(1.0, c * r ** -1.1) for r in range(1, NE + 1)) < K else (lo, c)
+        p = [min(1.0, c * r ** -1.1) for r in range(1, NE + 1)]
+    return sum(1.0 - (1.0 - q) ** T for q in p)
+
+
+def work(case):
+    T = case["T"]
+    if case["kind"] == "mm":
+        rows, cols = case["rows"], case["cols"]
+        return {"bytes": rows * cols + (-(-rows // 128)) * (-(-cols // 128)) * 4 + 4 * T * (rows + cols),
+                "flops": 2.0 * T * rows * cols}
+    E, inter, NE, K = (case[k] for k in ("E", "I", "NE", "K"))
+    n = case.get("layers", 1)
+    one = _distinct(case) * _expert_bytes(case, case["layout"] == "int4m") + _expert_bytes(case)
+    one += NE * E * 2 + NE * 4 + 2 * T * E * 4 + 2 * T * K * 4
+    return {"bytes": n * one, "flops": n * (6.0 * T * (K + 1) * E * inter + 2.0 * T * NE * E)}
+
+
+def tolerance(case):
+    # Paths that promise the reference's bits: the matrix product, single tokens over octet-tiled or
+    # row-major experts, and the small layers' row kernels. The matrix-core paths split activations
+    # into E4M3 planes: three for a single token, measured 4.7e-5 off the result in 64 bits, two for
+    # several tokens (about 8 bits of the SwiGLU's output), measured 6.3e-4 off.
+    if case["kind"] == "mm" or (case["T"] == 1 and case["layout"] in ("tiled", "rowmajor")):
+        return "exact"
+    if case["E"] % 512 or case["I"] % 512:
+        return "exact"
+    return {"rel": 2e-4 if case["T"] == 1 else 2.5e-3}
+
+
+# ------------------------------------------------------------------------------- exact ----
+def _wide(codes, scales, int4=False):
+    """One matrix in 64 bits."""
+    if int4:
+        lv = torch.stack((codes & 15, codes >> 4), dim=2).view(codes.shape[0], -1).double() - 8.0
+        return lv * scales.double().repeat_interleave(64, 1)
+    w = codes.view(torch.float8_e4m3fn).float().double()
+    s = scales.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+    return w * s[:w.shape[0], :w.shape[1]]
+
+
+def _mlp64(x, mats):
+    gate, up, down = mats
+    g = (x @ gate.T).clamp(max=LIMIT)
+    u = (x @ up.T).clamp(-LIMIT, LIMIT)
+    return (g * torch.sigmoid(g) * u) @ down.T
+
+
+def _route64(case, x, router, bias):
+    s = torch.sigmoid(x.double() @ router.double().T)
+    idx = torch.topk(s + bias.double(), case["K"], dim=1).indices
+    w = s.gather(1, idx)
+    return idx, w / w.sum(1, keepdim=True) * ROUTED_SCALE
+
+
+def exact(case, seed):
+    if case["kind"] == "mm":
+        codes, scales = _fp8(_gen(seed, 8), 1, case["rows"], case["cols"])
+        x = torch.randn((case["T"], case["cols"]), generator=_gen(seed, 17), device="cuda").to(torch.bfloat16)
+        return x.double() @ _wide(codes[0], scales[0]).T
+    NE, layers = case["NE"], case.get("layers", 1)
+    dropin, int4 = case["kind"] == "dropin", case["layout"] == "int4m"
+    xs = [_tokens(case, seed, layer).double() for layer in range(layers)]
+    routes = [_route64(case, xs[layer], *_routing(case, seed, layer)) for layer in range(layers)]
+    outs = [torch.zeros_like(x) for x in xs]
+    for e, mats in _experts(case, seed, POOL if dropin else NE, int4):
+        for i in range(len(mats[0][0])):
+            wide = [_wide(q[i], s[i], int4) for q, s in mats]
+            for layer, (x, (idx, w)) in enumerate(zip(xs, routes)):
+                mine = (layer * NE + idx) % POOL == e + i if dropin else idx == e + i
+                t, j = torch.nonzero(mine, as_tuple=True)
+                if len(t):
+                    outs[layer].index_add_(0, t, _mlp64(x[t], wide) * w[t, j, None])
+    for e, mats in _experts(case, seed, layers if dropin else 1, stream=9):
+        for i in range(len(mats[0][0])):
+            outs[e + i] += _mlp64(xs[e + i], [_wide(q[i], s[i]) for q, s in mats])
+    return outs if dropin else dict(out=outs[0], idx=None, w=routes[0][1])
