@@ -319,17 +319,24 @@ def _expert_bytes(case, int4=False):
 
 
 def _distinct(case):
-    """Expected distinct routed experts of T tokens."""
+    """Expected distinct routed experts of T tokens: logits are N(0, 1), so expert e is among the K
+    best when sigmoid(logit) + bias[e] passes the level that K of the NE pass on average."""
     NE, K, T = case["NE"], case["K"], case["T"]
+    bias = [0.64 * r ** -0.53 - 1.04 if r else 0.0 for r in range(NE)]
     if not case["skew"]:
-        p = [K / NE] * NE
-    else:
-        lo, hi = 0.0, float(NE)
-        for _ in range(60):                                  # c with sum min(1, c rank^-1.1) = K
-            c = (lo + hi) / 2
-            lo, hi = (c, hi) if sum(min(1.0, c * r ** -1.1) for r in range(1, NE + 1)) < K else (lo, c)
-        p = [min(1.0, c * r ** -1.1) for r in range(1, NE + 1)]
-    return sum(1.0 - (1.0 - q) ** T for q in p)
+        bias = [0.2 * (e + 0.5) / NE - 0.1 for e in range(NE)]
+
+    def passes(level, b):
+        s = level - b
+        if not 0.0 < s < 1.0:
+            return float(s <= 0.0)
+        return 0.5 * math.erfc(math.log(s / (1.0 - s)) / math.sqrt(2.0))
+
+    lo, hi = -1.1, 1.1
+    for _ in range(40):
+        level = (lo + hi) / 2
+        lo, hi = (level, hi) if sum(passes(level, b) for b in bias) > K else (lo, level)
+    return sum(1.0 - (1.0 - passes(level, b)) ** T for b in bias)
 
 
 def work(case):
