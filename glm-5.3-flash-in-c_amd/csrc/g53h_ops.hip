@@ -20,6 +20,9 @@
 /* ------------------------------------------------------------- FP8 matvec ---- */
 #include "g53h_rowdot.h"
 
+typedef float g53_f2 __attribute__((ext_vector_type(2)));
+typedef uint32_t g53_u4 __attribute__((ext_vector_type(4)));
+
 __device__ float g53_row_dot_i4(const G53hMat &m, int o, const float *x)
 {
     const uint8_t *row = m.w + (size_t)o * (m.cols / 2);
@@ -56,6 +59,146 @@ __global__ void k_mm_f8_generic(float *__restrict__ y, const float *__restrict__
     y[(size_t)t * m.rows + o] = g53_row_dot(m, o, x + (size_t)t * m.cols);
 }
 
+/* The same product for FP8 matrices with 128-column blocks (row-major codes, any rows, columns,
+ * alignment and scale rows), TG tokens at a time. A workgroup owns 64 rows x TG tokens; wave w
+ * takes column blocks w, w + NW, ... and lane r row r, so a weight is decoded once for TG tokens
+ * and x is the same for every lane: scalar loads, requested a group ahead of its products, and no
+ * LDS traffic in the inner loop. A wave loads its block's 64 x 128 codes as whole 128-byte runs (8
+ * lanes a row), a round ahead, and turns them through 4 KB of LDS, 32 rows at a time; 16-byte
+ * pieces are swizzled by row pairs, so that 16 lanes meet no bank twice. Each block's scaled
+ * double sum goes to LDS, and the thread that owns (row, token) adds a round's NW sums in block
+ * order, as the reference does.
+ * Bound by the fp32 chains, one FMA per weight and token: the reference rounds each product into
+ * one of eight chains, so matrix cores do not apply. 4096 x 2048, 24 tokens: 73 us with a
+ * thread per (row, token), 19 us here. AL: codes and columns in multiples of 16 bytes. */
+template <int TG, int NW, bool AL>
+__global__ void __launch_bounds__(64 * NW, 4) k_mm_f8_rows(float *__restrict__ y, const float *__restrict__ x, int T,
+                                                           G53hMat m)
+{
+    static_assert(TG <= NW, "one owner thread per (row, token)");
+    __shared__ __attribute__((aligned(16))) g53_u4 stage[NW][256];
+    __shared__ double pb[2][NW][TG][64];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned ng = (unsigned)(T + TG - 1) / TG;         /* the token groups of a row tile are neighbours */
+    const int r0 = (int)(blockIdx.x / ng) * 64, t0 = (int)(blockIdx.x % ng) * TG;
+    const int cols = m.cols, nb = (cols + 127) >> 7, rounds = (nb + NW - 1) / NW;
+    const int row = min(r0 + lane, m.rows - 1);              /* past the end: computed, not stored */
+    const float *srow = m.s + (size_t)(row / m.br) * m.scols;
+    g53_u4 *st = stage[w];
+    const int key = (lane >> 1) & 7;
+    const int lr = lane >> 3, lp = lane & 7;                 /* this lane's piece of a load: row, 16 bytes */
+    g53_u4 q[8];
+    auto load = [&](int b) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int rr = min(r0 + 8 * j + lr, m.rows - 1), c0 = b * 128 + lp * 16;
+            if constexpr (AL) {                              /* past the last column: its last piece again */
+                q[j] = *(const g53_u4 *)(m.w + (size_t)rr * cols + min(c0, cols - 16));
+            } else {                                         /* the words that hold the piece's bytes */
+                q[j] = g53_u4{0, 0, 0, 0};
+                if (c0 >= cols) continue;
+                const uint8_t *src = m.w + (size_t)rr * cols + c0;
+                const int sh = (int)((uintptr_t)src & 3), left = min(cols - c0, 16);
+                const uint32_t *p = (const uint32_t *)(src - sh);
+                uint32_t v[5];
+#pragma unroll
+                for (int k = 0; k < 5; k++) v[k] = 4 * k < left + sh ? p[k] : 0u;
+                q[j].x = __builtin_amdgcn_alignbyte(v[1], v[0], sh);
+                q[j].y = __builtin_amdgcn_alignbyte(v[2], v[1], sh);
+                q[j].z = __builtin_amdgcn_alignbyte(v[3], v[2], sh);
+                q[j].w = __builtin_amdgcn_alignbyte(v[4], v[3], sh);
+            }
+        }
+    };
+    const float *xt[TG];
+#pragma unroll
+    for (int t = 0; t < TG; t++) xt[t] = x + (size_t)min(t0 + t, T - 1) * cols;
+    double acc = 0.0;
+    if (w < nb) load(w);
+    for (int rd = 0; rd < rounds; rd++) {
+        const int b = rd * NW + w;
+        if (b < nb) {
+            float a[TG][8] = {};
+            float xv[2][TG][8];                              /* x of two neighbouring groups */
+            auto xload = [&](float (&d)[TG][8], int c) {     /* columns c .. c + 7, scalar loads */
+#pragma unroll
+                for (int t = 0; t < TG; t++)
+#pragma unroll
+                    for (int l = 0; l < 8; l++) d[t][l] = xt[t][c + l];
+            };
+            auto group = [&](uint32_t lo, uint32_t hi, const float (&d)[TG][8]) {
+                const g53_f2 f01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)lo, false);
+                const g53_f2 f23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)lo, true);
+                const g53_f2 f45 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hi, false);
+                const g53_f2 f67 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hi, true);
+                const float f[8] = {f01.x, f01.y, f23.x, f23.y, f45.x, f45.y, f67.x, f67.y};
+#pragma unroll
+                for (int t = 0; t < TG; t++)
+#pragma unroll
+                    for (int l = 0; l < 8; l++) a[t][l] = __builtin_fmaf(f[l], d[t][l], a[t][l]);
+            };
+            const int W = min(cols - b * 128, 128);
+            g53_u4 v[8];                                      /* this lane's row of the block */
+#pragma unroll
+            for (int j = 0; j < 8; j++) {                    /* 32 rows at a time */
+                const int rr = 8 * (j & 3) + lr;
+                st[rr * 8 + (lp ^ ((rr >> 1) & 7))] = q[j];
+                if ((j & 3) == 3) {
+#pragma unroll
+                    for (int p = 0; p < 8; p++) {
+                        const g53_u4 u = st[(lane & 31) * 8 + (p ^ key)];
+                        v[p] = j == 3 || lane >= 32 ? u : v[p];
+                    }
+                }
+            }
+            if (b + NW < nb) load(b + NW);
+            if (W == 128) {
+                /* a group's x is requested while the group before it is multiplied */
+                xload(xv[0], b * 128);
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    if (i < 15) xload(xv[(i + 1) & 1], b * 128 + 8 * (i + 1));
+                    __builtin_amdgcn_sched_barrier(0);
+                    group((i & 1) ? v[i >> 1].z : v[i >> 1].x, (i & 1) ? v[i >> 1].w : v[i >> 1].y, xv[i & 1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    if (i * 8 + 8 <= W) {
+                        xload(xv[0], b * 128 + 8 * i);
+                        group((i & 1) ? v[i >> 1].z : v[i >> 1].x, (i & 1) ? v[i >> 1].w : v[i >> 1].y, xv[0]);
+                    }
+            }
+            const int nt = W & 7;                            /* the block's last columns, one by one */
+            uint32_t tw[2] = {0, 0};
+            if (nt)
+#pragma unroll
+                for (int p = 0; p < 8; p++) {
+                    if ((W >> 3) == 2 * p) { tw[0] = v[p].x; tw[1] = v[p].y; }
+                    if ((W >> 3) == 2 * p + 1) { tw[0] = v[p].z; tw[1] = v[p].w; }
+                }
+            const float sc = srow[b];
+#pragma unroll
+            for (int t = 0; t < TG; t++) {
+                double s = (((double)a[t][0] + a[t][4]) + ((double)a[t][2] + a[t][6])) +
+                           (((double)a[t][1] + a[t][5]) + ((double)a[t][3] + a[t][7]));
+                for (int j = 0; j < nt; j++)
+                    s += (double)g53_e4m3_hw((uint8_t)(tw[j >> 2] >> (8 * (j & 3)))) * (double)xt[t][b * 128 + W - nt + j];
+                pb[rd & 1][w][t][lane] = s * (double)sc;
+            }
+        }
+        __syncthreads();
+        if (tid < 64 * TG) {
+#pragma unroll
+            for (int k = 0; k < NW; k++)
+                if (rd * NW + k < nb) acc = acc + pb[rd & 1][k][tid >> 6][lane];
+        }
+    }
+    if (tid < 64 * TG && r0 + lane < m.rows && t0 + (tid >> 6) < T)
+        y[(size_t)(t0 + (tid >> 6)) * m.rows + r0 + lane] = (float)acc;
+}
+
 extern "C" int g53h_mm_f8(float *y, const float *x, int T, const G53hMat *m)
 {
     if (g53h_ready()) return -1;
@@ -66,6 +209,28 @@ extern "C" int g53h_mm_f8(float *y, const float *x, int T, const G53hMat *m)
         return g53h_fail("g53h_mm_f8: bad geometry %dx%d block %dx%d scols %d", m->rows, m->cols,
                          m->br, m->bc, m->scols);
     if (m->flags & G53H_MAT_TILED) return g53h_fail("g53h_mm_f8: octet-tiled codes are read by the decode kernel only");
+    if (m->flags == 0 && m->bc == 128) {
+        /* Two tokens a workgroup share each weight's decode; while single tokens leave every CU at
+         * most one workgroup the call is a chain of latencies instead, and 16 waves, each with its
+         * block's codes in flight, shorten it. Measured, (1 token, 16 waves) against (2, 8): 4096 x
+         * 4096 1 token 10.5 against 14.8 us, 2048 x 4096 4 tokens 12.6 against 15.4; 4096 x 2048 24
+         * tokens 28.6 against 19.1, 4096 x 4096 64 tokens 123 against 64. (3 and 4 tokens: 20 and 31
+         * us at 24, the chains' registers spill.) */
+        const long tiles = (m->rows + 63) / 64;
+        const int al = m->cols % 16 == 0 && ((uintptr_t)m->w & 15) == 0, one = tiles * T <= g53h_num_cus();
+        const long wgs = tiles * (one ? T : (T + 1) / 2);
+        if (wgs > 0x7fffffffL) return g53h_fail("g53h_mm_f8: %d rows x %d tokens", m->rows, T);
+        const dim3 g((unsigned)wgs);
+        hipStream_t st = g53h_stream();
+#define G53_MM(TG, NW, AL) hipLaunchKernelGGL((k_mm_f8_rows<TG, NW, AL>), g, dim3(64 * NW), 0, st, y, x, T, *m)
+        if (one && al) G53_MM(1, 16, true);
+        else if (one) G53_MM(1, 16, false);
+        else if (al) G53_MM(2, 8, true);
+        else G53_MM(2, 8, false);
+#undef G53_MM
+        G53_LAUNCHED("k_mm_f8_rows");
+        return 0;
+    }
     const long n = (long)T * m->rows;
     hipLaunchKernelGGL(k_mm_f8_generic, dim3((unsigned)((n + 127) / 128)), dim3(128), 0,
                        g53h_stream(), y, x, T, *m);

@@ -1,0 +1,41 @@
+"""The row-tile matrix product (g53h_mm_f8 on FP8 matrices with 128-column blocks, replaces
+src/core/glm53f_ops.c:185-228): bit-exact with the oracle at the edges of its tiles of 64 rows,
+128 columns and up to four tokens, and for matrices that are not 16-byte aligned."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import glm53h
+import oracle_lib as O
+from glm53h import DevBuf, G53hMat, check
+from test_gpu_parity import same, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def L():
+    return glm53h.init(0)
+
+
+@pytest.mark.parametrize("rows,cols,br,T,shift", [
+    (1, 5, 128, 1, 0), (64, 128, 128, 1, 0), (63, 127, 128, 2, 0), (65, 129, 16, 3, 0), (128, 136, 128, 4, 8),
+    (200, 1030, 16, 5, 0), (130, 1024, 128, 9, 3), (300, 4096, 128, 2, 1), (4096, 2048, 128, 24, 0),
+    (100, 1152, 128, 7, 0), (64, 2047, 64, 13, 16), (256, 2176, 128, 130, 0), (4100, 131, 128, 5, 0)])
+def test_mm_f8_rows(L, rows, cols, br, T, shift):
+    say("mm rows", rows, cols, br, T, shift)
+    rng = np.random.default_rng(rows * 7 + cols)
+    w = rng.integers(0, 256, rows * cols).astype(np.uint8)
+    w[(w & 0x7f) == 0x7f] ^= 1                       # no NaN codes
+    sc = -(-cols // 128)
+    s = rng.uniform(1e-3, 1e-1, -(-rows // br) * sc).astype(np.float32)
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    wd = DevBuf.from_array(np.concatenate([np.zeros(shift, np.uint8), w]))
+    sd, xd, yd = DevBuf.from_array(s), DevBuf.from_array(x), DevBuf((T * rows + 1) * 4)
+    yd.upload(np.full(T * rows + 1, 7.0, np.float32))
+    m = G53hMat(wd.ptr + shift, sd.ptr, rows, cols, br, 128, sc, 0)
+    check(L.g53h_mm_f8(yd.ptr, xd.ptr, T, C.byref(m)), "mm")
+    got = yd.download(np.float32)
+    assert got[-1] == 7.0                            # nothing past the last row
+    assert same(got[:-1].reshape(T, rows), O.mm_f8(O.oracle(), x, w, s, rows, cols, br, 128))
