@@ -15,12 +15,12 @@
  *   3. k_grp_xq           each token's activations as NPX E4M3 planes with a power-of-two
  *                         token scale: x = 2^-k (q0 + q1 / 16 + q2 / 256 ...). For bf16-valued
  *                         inputs two planes hold x exactly (8 significant bits = 4 + 4).
- *   4. k_grp_gateup       per (tile, 128-row block): gate and up rows of the expert times the
+ *   4. k_grp_gemm<true>   per (tile, 128-row block): gate and up rows of the expert times the
  *                         tile's tokens on v_mfma_scale_f32_32x32x64_f8f6f4, one 128x128 scale
  *                         block per step, the block scale applied to each block's fp32 sum;
  *                         SwiGLU in the epilogue; the activation leaves as NPA E4M3 planes with
  *                         a fixed power-of-two scale (|act| <= max(limit, 0.28) * limit).
- *   5. k_grp_down         per (tile, 256-row block): down rows times the activation planes;
+ *   5. k_grp_gemm<false>  per (tile, 256-row block): down rows times the activation planes;
  *                         contributions to contrib[position][hidden] (zeros for an absent
  *                         expert, the reference's drop path).
  *   6. k_grp_combine      out[t] = (float)(sum_j (double)w[t][j] * contrib[pos(t, j)]) in slot
@@ -55,55 +55,26 @@
 typedef int g53_v8i __attribute__((ext_vector_type(8)));
 typedef float g53_v16f __attribute__((ext_vector_type(16)));
 typedef int g53_v4i __attribute__((ext_vector_type(4)));
-/* global-memory views, so loads are global_load (vector memory only), not flat */
-typedef __attribute__((address_space(1))) const g53_v8i g53_gv8i;
-typedef __attribute__((address_space(1))) const g53_v4i g53_gv4i;
-typedef __attribute__((address_space(1))) const float g53_gflt;
 
-#define G53_GRP_NT    128     /* positions per tile                                        */
-#define G53_GRP_NH    (G53_GRP_NT / 32)   /* 32-position halves of a tile (matrix-core columns) */
-#define G53_GRP_XST   144     /* LDS bytes per token row of a 128-byte slice (16 B padding) */
+#define G53_GRP_NT    64      /* positions per tile                                        */
 #define G53_GRP_MAXT  2048    /* tokens per planning pass                                   */
 #define G53_GRP_NPX   2       /* E4M3 planes of the input activations                       */
 #define G53_GRP_NPA   2       /* E4M3 planes of the SwiGLU activations                      */
 #define G53_GRP_MASKS 12288   /* LDS 64-token masks of the planner (chunks x experts)       */
 #define G53_GRP_NW    8       /* waves of a GEMM workgroup                                   */
-#ifndef G53_GRP_WPC
-#define G53_GRP_WPC   1       /* GEMM workgroups resident per CU                             */
-#endif
-#ifndef G53_GRP_PERS
-#define G53_GRP_PERS  1       /* workgroups per CU in the grid: each loops over its items  */
-#endif
-#ifndef G53_GRP_RS
-#define G53_GRP_RS    2       /* weight blocks in a lane's ring                              */
-#endif
-#ifndef G53_GRP_LXS
-#define G53_GRP_LXS   2       /* activation slices in a thread's ring                        */
-#endif
-#ifndef G53_GRP_NS
-#define G53_GRP_NS    2       /* activation slices in the workgroup's LDS ring               */
-#endif
-
 /* error flags (meta[1]) */
 #define G53_GRP_EIDX  1       /* a routed index outside [0, n_experts)                      */
 #define G53_GRP_EDESC 8       /* an expert descriptor without the expected 128x128 layout   */
-#define G53_GRP_ESPIN 2       /* a wait on the slice ring timed out                          */
 
 /* ------------------------------------------------------------------ planning ---- */
-/* meta[]: [0] tiles, [1] error flags, [2..17] the GEMMs' item counters, then the first item of
- * each XCD's range (9 entries: XCD x takes items [b[x], b[x+1])) for gate/up and for down */
-#define G53_GRP_BGU   18
-#define G53_GRP_BDN   27
+/* meta[]: [0] tiles, [1] error flags, then the first item of each XCD's range (9 entries: XCD x
+ * takes items [b[x], b[x+1])) for gate/up and for down */
+#define G53_GRP_BGU   2
+#define G53_GRP_BDN   11
 
 /* Estimated cost of one row of a segment's items (one item per tile) with n positions, in
- * tenths of the time of a tile of at most 64 positions. Measured item times at 1, 2, 3 and 4
- * 32-position halves were 47, 51, 63 and 70 us: up to two halves the weight stream alone sets
- * the time, beyond that the matrix work adds about a third per half. */
-__device__ __forceinline__ int g53_grp_tile_cost(int n)
-{
-    const int h = (n + 31) / 32;
-    return h <= 2 ? 10 : 10 + 3 * (h - 2) - (h == 4 ? 1 : 0);
-}
+ * tenths of the time of a tile of at most 32 positions (37 us; up to 64 positions 44 us). */
+__device__ __forceinline__ int g53_grp_tile_cost(int n) { return n <= 32 ? 10 : 12; }
 __device__ __forceinline__ int g53_grp_seg_cost(int n)
 {
     const int full = n / G53_GRP_NT, rem = n % G53_GRP_NT;
@@ -169,7 +140,6 @@ k_grp_plan(const int *__restrict__ idx, int T, int K, int NE, int has_sh, int *_
             cc += __shfl(ic, 63);
         }
         if (tid == 0) { off[nseg] = cp; tb[nseg] = ct; pc[nseg] = cc; meta[0] = ct; }
-        if (tid < 16) meta[2 + tid] = 0;         /* the GEMMs' item counters */
     }
     __syncthreads();
     /* each XCD's item range, of equal estimated cost: lanes 0-8 for gate/up, 16-24 for down */
@@ -242,8 +212,6 @@ __device__ __forceinline__ void g53_split_planes(const float (&v)[4], uint32_t (
     }
 }
 
-/* Token t's row of x as NPX planes xq[p][t][E] with scale 2^k, k = 8 - exponent(absmax), so
- * every |x| * 2^k < 256; xinv[t] = 2^-k. Grid T, 256 threads, E a multiple of 16. */
 /* Byte position of column c of a 128-column block in the octet-tiled order: run sigma(c % 8)
  * (sigma is its own inverse), element c / 8 of the run. */
 __device__ __forceinline__ int g53_grp_tpos(int c)
@@ -265,9 +233,13 @@ __device__ __forceinline__ void g53_grp_st4(uint8_t *row, int c0, uint32_t q, in
     for (int k = 0; k < 4; k++) blk[g53_grp_tpos((c0 + k) & 127)] = (uint8_t)(q >> (8 * k));
 }
 
+/* Token t's row of x as NPX planes xq[p][t][E] with scale 2^k, k = 8 - exponent(absmax), so
+ * every |x| * 2^k < 256; 2^-k goes to every position of the token (pos_of[t][ns], -1: none).
+ * Grid T, 256 threads, E a multiple of 16. */
 template <int NP>
 __global__ void __launch_bounds__(256)
-k_grp_xq(const float *__restrict__ x, int E, int T, uint8_t *__restrict__ xq, float *__restrict__ xinv, int tiled)
+k_grp_xq(const float *__restrict__ x, int E, int T, uint8_t *__restrict__ xq, float *__restrict__ xinvp,
+         const int *__restrict__ pos_of, int ps, int ns, int tiled)
 {
     __shared__ float red[4];
     const int t = blockIdx.x, tid = threadIdx.x;
@@ -285,7 +257,10 @@ k_grp_xq(const float *__restrict__ x, int E, int T, uint8_t *__restrict__ xq, fl
     if (m > 0.0f && m <= 3.0e38f) (void)frexpf(m, &ex);          /* m < 2^ex */
     const int k = 8 - ex;
     const float sc = ldexpf(1.0f, k);
-    if (tid == 0) xinv[t] = ldexpf(1.0f, -k);
+    for (int j = tid; j < ns; j += 256) {
+        const int p = pos_of[t * ps + j];
+        if (p >= 0) xinvp[p] = ldexpf(1.0f, -k);
+    }
     for (int i = tid * 4; i < E; i += 1024) {
         const float4 v = *(const float4 *)(xr + i);
         const float s[4] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc};
@@ -297,188 +272,89 @@ k_grp_xq(const float *__restrict__ x, int E, int T, uint8_t *__restrict__ xq, fl
 }
 
 /* ------------------------------------------------------------- grouped GEMM ---- */
-/* A workgroup = NW waves; wave w owns 32 rows of A (rows chosen by the caller) and both
- * 32-position halves of a 64-position tile. Two workgroups share a CU, so one's matrix work
- * overlaps the other's waits at its per-block barrier. The K loop walks 128-byte scale blocks.
- * Per block kb a thread issues, in this order, its 16-byte pieces of the activation slice
- * kb + LX (a ring of LX register slots) and its lane's 64 weight bytes of block kb + R - 1 (a
- * ring of R slots), runs block kb on the matrix cores from LDS slice kb, then stores slice
- * kb + 1 to the other LDS buffer. Loads complete in issue order, so that store waits for the
- * weights up to block kb + LX - 1 only, issued LX + 1 blocks earlier. */
-template <int NP, int NH>
-__device__ __forceinline__ void g53_grp_block(g53_v16f (&acc)[G53_GRP_NH], const g53_v8i &w0, const g53_v8i &w1,
-                                              const uint8_t *xb, int c0b, int c1b)
+/* Both GEMMs share one pipeline. A workgroup is 8 waves and stays for the whole launch, one per
+ * CU; it walks its items (256 weight rows x one tile) as one stream of steps of 128 weight columns.
+ * A step's operands - 256 rows x 128 codes, and the tile's positions x 128 codes x 2 planes - go
+ * straight to LDS (global_load_lds, 1 KB a wave instruction), into a ring of three slots, two steps
+ * ahead, across item boundaries: no registers hold loads in flight, every code is fetched as part
+ * of a whole 128-byte run, and one barrier per step hands a slot over. The waits count loads by
+ * hand, so the loads are inline assembly: the compiler would wait for every LDS load before any
+ * LDS read. Everything else a step needs comes by scalar loads, which have a counter of their own.
+ *
+ * LDS rows are 128 bytes, 16-byte piece c of row r at piece c ^ ((r / 2) % 8): the 16 lanes of one
+ * LDS access read piece c of 16 consecutive rows and meet no bank twice.
+ *
+ * Wave w multiplies 64 of the 256 rows (row group w % 4: two matrix-core tiles) by the 32 positions
+ * of half w / 4, so a tile of up to 32 positions occupies one wave of each SIMD.
+ */
+#define G53_GRP_SA   (256 * 128)                      /* a slot's weight rows                     */
+#define G53_GRP_PL   (G53_GRP_NT * 128)               /* one plane of the slot's positions        */
+#define G53_GRP_SLOT (G53_GRP_SA + 2 * G53_GRP_PL)
+#define G53_GRP_NS   3
+static_assert(G53_GRP_NT == 64 && G53_GRP_NPX == 2 && G53_GRP_NPA == 2 && G53_GRP_NW == 8, "slot and wave layout");
+
+/* A value every lane reads alike from memory that no kernel of this launch writes: a scalar load. */
+template <class V>
+__device__ __forceinline__ V g53_sld(const V *p)
 {
-    const float c0 = __int_as_float(c0b), c1 = __int_as_float(c1b);
-#pragma unroll
-    for (int h = 0; h < NH; h++) {
-        g53_v16f b = {};
-#pragma unroll
-        for (int p = 0; p < NP; p++) {
-#pragma unroll
-            for (int s = 0; s < 2; s++) {
-                const g53_v8i x = *(const g53_v8i *)(xb + p * G53_GRP_NT * G53_GRP_XST + h * 32 * G53_GRP_XST + s * 32);
-                b = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(s ? w1 : w0, x, b, 0, 0, 0, 127, 0, 127 - 4 * p);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[h][r] = fmaf(b[r], r < 8 ? c0 : c1, acc[h][r]);
-        /* pin the half's arithmetic here: the compiler would otherwise sink the pure matrix
-         * arithmetic past the ring waits to the loop's end and keep every block's operands live */
-        asm volatile("" : "+v"(acc[h]));
-    }
+    return *(const __attribute__((address_space(4))) V *)(uintptr_t)p;
 }
 
-#ifdef G53_GRP_KTRACE
-__device__ uint64_t *g53_ktrace;     /* diagnostic builds only: per-block timestamps */
-extern "C" int g53h_set_grouped_ktrace(void *p)
+/* A wave's four octets of weight rows (1 KB each, 16 bytes per lane at base + v0 .. v3) to LDS bytes
+ * lds, lds + 1024, ...; nt: streamed once. M0 holds the LDS address and must be written ahead of the
+ * load that uses it. */
+#define G53_DMA_ROWS(NT)                                                                                       \
+    asm volatile("s_mov_b32 m0, %5\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %4" NT                            \
+                 "\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %1, %4" NT                 \
+                 "\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %2, %4" NT                 \
+                 "\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %3, %4" NT                 \
+                 :: "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(base), "s"(lds) : "memory", "m0", "scc")
+__device__ __forceinline__ void g53_dma_rows(const uint32_t (&v)[4], const uint8_t *base, uint32_t lds)
 {
-    return hipMemcpyToSymbol(HIP_SYMBOL(g53_ktrace), &p, sizeof p) == hipSuccess ? 0 : -1;
+    G53_DMA_ROWS("");
 }
-#endif
-
-/* LDS counters of the slice ring: relaxed workgroup-scope atomics (a wave's LDS operations
- * execute in order, so a count added after a wave's slice stores is seen after them), and a
- * bounded sleep-poll that reports a timeout instead of hanging. */
-#define G53_CBAR() asm volatile("" ::: "memory")
-__device__ __forceinline__ void g53_grp_lds_add(int *p, int v)
+__device__ __forceinline__ void g53_dma_rows_nt(const uint32_t (&v)[4], const uint8_t *base, uint32_t lds)
 {
-    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    G53_DMA_ROWS(" nt");
 }
-__device__ __forceinline__ int g53_grp_wait(int *p, int want)
+#undef G53_DMA_ROWS
+/* 16 bytes per lane from base + off to LDS byte lds + 16 * lane. */
+__device__ __forceinline__ void g53_dma16(uint32_t off, const uint8_t *base, uint32_t lds)
 {
-    int spins = 0;
-    while (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < want) {
-        if (++spins > (1 << 22)) return 1;
-        __builtin_amdgcn_s_sleep(1);
-    }
-    G53_CBAR();
-    return 0;
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
 }
-
-/* The activation slice loader of a workgroup of NW waves: a slice is G53_GRP_NT positions x
- * 128 bytes x NP planes, 16-byte pieces; thread t takes piece t % 8 of positions
- * t / 8 + j * 8 * NW. */
-template <int NW>
-struct G53GrpLd {
-    static constexpr int RPT = G53_GRP_NT * 8 / (64 * NW);   /* positions per thread    */
-    const uint8_t *src[RPT];                           /* source rows (+ 16 * piece)     */
-    int dst[RPT];                                      /* LDS offsets in a slice         */
-};
-
-/* acc[h][r] += scale_r * (A_rows x B_tile-half-h), h < NH, over NKB blocks of 128 bytes.
- *   arow    this lane's weight row + (l / 32) * 64 (block 0), kst bytes to the next block
- *           (128 row-major, 1024 octet-tiled)
- *   s0, s1  scale rows for C registers 0-7 and 8-15 (one float per block)
- *   ld      this thread's slice loader; plane p of a source row at + p * xps
- *   NH      32-position halves the tile has (positions beyond the tile's count are padding) */
-template <int NW, int NP, int NKB, int NH>
-__device__ __forceinline__ void g53_grp_kloop(g53_v16f (&acc)[G53_GRP_NH], const uint8_t *arow, int kst, const float *s0,
-                                              const float *s1, const G53GrpLd<NW> &ld, size_t xps, uint8_t *xs,
-                                              int *flags, int &spin_err, int lane)
+/* 4 bytes per lane from p to LDS byte lds + 4 * lane. */
+__device__ __forceinline__ void g53_dma4(const float *p, uint32_t lds)
 {
-    constexpr int SL = NP * G53_GRP_NT * G53_GRP_XST;           /* one slice in LDS        */
-    constexpr int PL = G53_GRP_NT * G53_GRP_XST;                /* one plane of a slice    */
-    /* only the rows the NH halves read are loaded: positions >= 32 * NH are never used */
-    constexpr int RPT0 = G53GrpLd<NW>::RPT, RPN = (NH * 32 + 8 * NW - 1) / (8 * NW);
-    constexpr int RPT = RPN < RPT0 ? RPN : RPT0;
-    constexpr int LX = G53_GRP_LXS;                             /* slice slots             */
-    constexpr int R0 = G53_GRP_RS;                              /* weight slots            */
-    constexpr int R = NKB < R0 ? NKB : R0;
-    constexpr int NS = G53_GRP_NS;                              /* LDS slice slots         */
-    static_assert(NKB % R == 0 && R % LX == 0 && R % NS == 0, "ring sizes");
-    int *ready = flags, *freed = flags + NS;
-    static_assert(NKB <= 64, "one scale per lane");
-    static_assert(NP == 2 || NP == 3, "two or three planes");
-    const uint8_t *xrd = xs + (lane >> 5) * 64 + (lane & 31) * G53_GRP_XST;
-    /* the block scales of the wave's rows, lane k holding block k's (loaded once, before any
-     * weight load, so no later wait on them waits for weights) */
-    const float sv0 = lane < NKB ? ((g53_gflt *)s0)[lane] : 0.0f, sv1 = lane < NKB ? ((g53_gflt *)s1)[lane] : 0.0f;
-    g53_v8i a[R][2];
-    g53_v4i xr[LX][RPT][3];
-    typedef const __attribute__((address_space(1))) uint8_t *gptr;
-    const gptr ag = (gptr)arow;
-    gptr xg[RPT];
-#pragma unroll
-    for (int j = 0; j < RPT; j++) xg[j] = (gptr)ld.src[j];
-#define G53_LDA(sl, k) do { a[sl][0] = *(g53_gv8i *)(ag + (size_t)(k) * kst); a[sl][1] = *(g53_gv8i *)(ag + (size_t)(k) * kst + 32); } while (0)
-#define G53_LDX(sl, k) do { _Pragma("unroll") for (int j = 0; j < RPT; j++) {                                  \
-                                xr[sl][j][0] = *(g53_gv4i *)(xg[j] + (k) * 128);                               \
-                                xr[sl][j][1] = *(g53_gv4i *)(xg[j] + xps + (k) * 128);                         \
-                                if (NP == 3) xr[sl][j][2] = *(g53_gv4i *)(xg[j] + 2 * xps + (k) * 128); } } while (0)
-#define G53_STX(sl, buf) do { _Pragma("unroll") for (int j = 0; j < RPT; j++) {                                \
-                                  uint8_t *d_ = xs + (buf) * SL + ld.dst[j];                                   \
-                                  *(g53_v4i *)d_ = xr[sl][j][0]; *(g53_v4i *)(d_ + PL) = xr[sl][j][1];         \
-                                  if (NP == 3) *(g53_v4i *)(d_ + 2 * PL) = xr[sl][j][2]; } } while (0)
-    /* prologue: slices 0 .. LX-1 (slice 0 to LDS), then the weights of blocks 0 .. R-2 */
-#pragma unroll
-    for (int k = 0; k < LX; k++) G53_LDX(k, k < NKB ? k : NKB - 1);
-#pragma unroll
-    for (int k = 0; k < R - 1; k++) G53_LDA(k, k);
-    G53_STX(0, 0);
-    G53_CBAR();
-    if (lane == 0) g53_grp_lds_add(&ready[0], 1);
-    /* Block kb: issue slice kb+LX and weights kb+R-1; store slice kb+1 into its slot once every
-     * wave has finished the block that slot held (freed), and count it ready; wait until every
-     * wave has stored slice kb (ready), multiply, count it freed. No workgroup barrier: waves
-     * drift up to NS-1 blocks apart. Loads past the end re-read the last block. */
-#pragma nounroll
-    for (int kb0 = 0; kb0 < NKB; kb0 += R) {
-#pragma unroll
-        for (int u = 0; u < R; u++) {
-            const int kb = kb0 + u;
-            const int kx = kb + LX < NKB ? kb + LX : NKB - 1;
-            const int ka = kb + R - 1 < NKB ? kb + R - 1 : NKB - 1;
-#ifdef G53_GRP_KTRACE
-            uint64_t kt0 = __builtin_amdgcn_s_memrealtime(), kt1 = 0, kt2 = 0;
-#endif
-            G53_LDX(u % LX, kx);
-            G53_LDA((u + R - 1) % R, ka);
-            if (kb + 1 < NKB) {
-                const int sn = (u + 1) % NS;
-                spin_err |= g53_grp_wait(&freed[sn], NW * ((kb + 1) / NS));
-                G53_STX((u + 1) % LX, sn);
-                G53_CBAR();
-                if (lane == 0) g53_grp_lds_add(&ready[sn], 1);
-            }
-#ifdef G53_GRP_KTRACE
-            kt1 = __builtin_amdgcn_s_memrealtime();
-#endif
-            spin_err |= g53_grp_wait(&ready[u % NS], NW * (kb / NS + 1));
-#ifdef G53_GRP_KTRACE
-            kt2 = __builtin_amdgcn_s_memrealtime();
-#endif
-            g53_grp_block<NP, NH>(acc, a[u][0], a[u][1], xrd + (u % NS) * SL,
-                                   __builtin_amdgcn_readlane(__float_as_int(sv0), kb),
-                                   __builtin_amdgcn_readlane(__float_as_int(sv1), kb));
-            G53_CBAR();
-            if (lane == 0) g53_grp_lds_add(&freed[u % NS], 1);
-#ifdef G53_GRP_KTRACE
-            if (g53_ktrace && lane == 0 && NKB == 32) {   /* the gate/up kernel */
-                uint64_t *o = g53_ktrace + (((size_t)blockIdx.x * NW + (threadIdx.x >> 6)) * 32 + kb) * 4;
-                o[0] = kt0; o[1] = kt1; o[2] = kt2; o[3] = __builtin_amdgcn_s_memrealtime();
-            }
-#endif
-            __builtin_amdgcn_sched_barrier(0);   /* keep the blocks in program order */
-        }
-    }
-#undef G53_LDA
-#undef G53_LDX
-#undef G53_STX
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 4\n\tglobal_load_lds_dword %0, off"
+                 :: "v"(p), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void g53_grp_bar()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 }
 
 /* A descriptor with the layout the grouped kernels assume (octet-tiled iff the pass is). */
-__device__ __forceinline__ bool g53_grp_desc_ok(const G53hExpert &x, int E, int I, int tiled)
+__device__ __forceinline__ bool g53_grp_mat_ok(const G53hMat *m, int rows, int cols, int tiled)
 {
-    const int want = tiled ? G53H_MAT_TILED : 0;
-    return !((x.gate.flags | x.up.flags | x.down.flags) & G53H_MAT_I4) &&
-           (x.gate.flags & G53H_MAT_TILED) == want && (x.up.flags & G53H_MAT_TILED) == want &&
-           (x.down.flags & G53H_MAT_TILED) == want &&
-           x.gate.br == 128 && x.gate.bc == 128 && x.gate.rows == I && x.gate.cols == E &&
-           x.up.br == 128 && x.up.bc == 128 && x.up.rows == I && x.up.cols == E &&
-           x.down.br == 128 && x.down.bc == 128 && x.down.rows == E && x.down.cols == I &&
-           x.gate.scols >= E / 128 && x.up.scols >= E / 128 && x.down.scols >= I / 128;
+    const int fl = g53_sld(&m->flags);
+    return !(fl & G53H_MAT_I4) && (fl & G53H_MAT_TILED) == (tiled ? G53H_MAT_TILED : 0) && g53_sld(&m->br) == 128 &&
+           g53_sld(&m->bc) == 128 && g53_sld(&m->rows) == rows && g53_sld(&m->cols) == cols &&
+           g53_sld(&m->scols) >= cols / 128;
 }
+__device__ __forceinline__ bool g53_grp_desc_ok(const G53hExpert *x, int E, int I, int tiled)
+{
+    return g53_grp_mat_ok(&x->gate, I, E, tiled) && g53_grp_mat_ok(&x->up, I, E, tiled) &&
+           g53_grp_mat_ok(&x->down, E, I, tiled);
+}
+
+template <int N>
+struct G53Int {
+    static constexpr int value = N;
+};
 
 struct G53GrpArgs {
     const G53hExpert *experts;     /* [NE]                                               */
@@ -487,9 +363,9 @@ struct G53GrpArgs {
                                       segment | tiles of the segment << 16}                */
     const int *meta;               /* [0] tile count, [1] error flags                    */
     int *meta_w;
-    const int *tok_of;             /* position -> token                                  */
+    const int *tok_of;             /* position -> token (readable 8 past the last)       */
     const uint8_t *xq;             /* [NPX][T][E]                                        */
-    const float *xinv;             /* [T]                                                */
+    const float *xinvp;            /* [P]: the token scale of each position              */
     uint8_t *aq;                   /* [NPA][P][I]                                        */
     float *contrib;                /* [P][E]                                             */
     int T, P, E, I, NE;
@@ -497,51 +373,13 @@ struct G53GrpArgs {
     int tiled;                     /* 1: experts octet-tiled, planes in the tiled column order */
     int partial;                   /* 1: experts without weights are outside this batch and
                                       left alone, unless marked dropped (gate.flags & G53H_MAT_DROPPED)    */
-    int *ctr;                      /* [16] item counters: 0-7 gate/up, 8-15 down; each
-                                      kernel starts with its own at zero and clears the
-                                      other kernel's                                      */
-    uint64_t *trace;               /* optional: [grid][8] timestamps of each workgroup    */
+    uint64_t *trace;               /* optional: [items][32] timestamps of each gate/up item  */
 };
 
-/* Diagnostics: 100 MHz timestamps of an item's phases into a.trace[item * 8 + k] when it is set
- * (gti: the item's number). */
-#define G53_GTRACE(k, v) do { if (a.trace && threadIdx.x == 0) a.trace[(size_t)gti * 32 + (k)] = (v); } while (0)
-#define G53_GTRACE_W(k, v) do { if (a.trace && (threadIdx.x & 63) == 0) a.trace[(size_t)gti * 32 + (k)] = (v); } while (0)
-
-/* Item loc of the workgroup's group: the dispatcher deals workgroups round-robin over the 8
- * XCDs, so the workgroups of XCD x (blockIdx.x % 8 == x) share the items blo .. bhi - 1 (a
- * range of equal estimated cost, from the planner), which they claim in order from the
- * group's counter. Items are numbered segment by segment, and inside a segment row block by
- * row block, all tiles of a block in a row: the tiles of one expert that re-read the same
- * weight rows run next to each other on one XCD and find them in its L2. Returns false past
- * the group's last item. */
-__device__ __forceinline__ bool g53_grp_item(const int4 *tiles, int blo, int bhi, int MB, int loc, int4 &tl, int &mb)
-{
-    const int item = blo + loc;
-    if (item >= bhi) return false;
-    const int w = tiles[item / MB].w;                    /* a tile of the item's segment */
-    const int ts0 = w & 0xffff, nts = w >> 16;
-    const int q = item - ts0 * MB;
-    mb = q / nts;
-    tl = tiles[ts0 + q % nts];
-    return true;
-}
-
-/* Claim the group's next item (a relaxed device-scope counter, one claim per item, issued an
- * item ahead so that its latency hides behind the current item). */
-__device__ __forceinline__ int g53_grp_claim(int *ctr)
-{
-    return __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-/* Gate/up + SwiGLU for (tile, block mb of 16*NW intermediate rows). Wave w: A rows 0-15 = gate
- * rows mb*16*NW + w*16 + 0..15, rows 16-31 = the up rows of the same indices, so C registers r
- * and r + 8 of a lane are gate and up of one intermediate row and one position. */
 /* The clamped SwiGLU of src/core/glm53f_ops.c:486-494 (gate clamped from above, up both ways)
  * with the hardware exponential: the result is rounded to two E4M3 planes (about 8 significant
- * bits) right after, so the reference's expf to the last bit buys nothing here, and the exact
- * table method's LDS lookups queue behind the K loop's operand reads of the other waves (about
- * 3 us per 32 positions). Infinities and NaN follow the reference: sigmoid(-inf) = 0. */
+ * bits) right after, so the reference's expf to the last bit buys nothing here. Infinities and
+ * NaN follow the reference: sigmoid(-inf) = 0. */
 __device__ __forceinline__ float g53_grp_swiglu(float g, float u, float limit)
 {
     const float gi = g > limit ? limit : g;
@@ -549,200 +387,348 @@ __device__ __forceinline__ float g53_grp_swiglu(float g, float u, float limit)
     return gi * __frcp_rn(1.0f + __expf(-gi)) * ui;
 }
 
-template <int NW, int NKB>
-__global__ void __launch_bounds__(64 * NW, G53_GRP_WPC) k_grp_gateup(G53GrpArgs a)
+/* A wave's operands of one step: up to two matrix-core tiles of 32 weight rows, and 32 positions
+ * in two planes, two K steps each. */
+struct G53GrpOps {
+    g53_v8i a[2][2], x[2][2];                                /* [tile][K step], [plane][K step] */
+    float c0, c1;                                            /* block scales of C registers 0-7, 8-15 */
+};
+/* Fragment k (0-3 positions, 4-7 weights) of a step's operands from the slot at sl: a4 and x4 are
+ * the lane's four 16-byte pieces (two K steps of two) of its weight row and of its position, the
+ * second tile's rows DA bytes further. */
+template <int DA, int k>
+__device__ __forceinline__ void g53_grp_fetch(G53GrpOps &o, const uint8_t *sl, const int (&a4)[4], const int (&x4)[4])
 {
-    __shared__ __attribute__((aligned(16))) uint8_t xs[G53_GRP_NS * G53_GRP_NPX * G53_GRP_NT * G53_GRP_XST];
-    __shared__ __attribute__((aligned(16))) uint8_t ao[G53_GRP_NPA * G53_GRP_NT * 128];   /* the item's planes */
-    __shared__ float xil[G53_GRP_NT];                    /* the tile's token scales          */
-    __shared__ int flags[2 * G53_GRP_NS];
-    __shared__ int claim[2];
-    static_assert(16 * NW == 128, "an item is one 128-row scale block");
-    int *ctr = a.ctr + (blockIdx.x & 7);
-    if (threadIdx.x == 0) claim[0] = g53_grp_claim(ctr);
-    if (blockIdx.x == 0 && threadIdx.x < 8) a.ctr[8 + threadIdx.x] = 0;   /* the down kernel's */
-    const int blo = a.meta[G53_GRP_BGU + (blockIdx.x & 7)], bhi = a.meta[G53_GRP_BGU + (blockIdx.x & 7) + 1];
-    for (int kk = 0;; kk++) {
-        __syncthreads();                     /* claim[] written; the previous item is done with LDS */
-        int4 tl;
-        int mb;
-        const uint64_t t_item = __builtin_amdgcn_s_memrealtime();
-        if (!g53_grp_item(a.tiles, blo, bhi, a.I / (16 * NW), claim[kk & 1], tl, mb)) break;
-        const int gti = blo + claim[kk & 1];
-        G53_GTRACE(0, t_item);
-        int nxt = 0;
-        if (threadIdx.x == 0) nxt = g53_grp_claim(ctr);
-        G53_GTRACE(4, (uint64_t)__smid() << 32 | (uint32_t)(tl.y << 8 | tl.z));
-        G53_GTRACE(5, (uint64_t)blockIdx.x << 32 | (uint32_t)(tl.x << 8 | mb));
-        const G53hExpert *ex = tl.x < a.NE ? &a.experts[tl.x] : a.shared;
-        const bool usable = ex && ex->gate.w != nullptr && g53_grp_desc_ok(*ex, a.E, a.I, a.tiled);
-        if (!usable) {                                       /* absent expert: down writes zeros */
-            if (ex && ex->gate.w && threadIdx.x == 0) atomicOr(&a.meta_w[1], G53_GRP_EDESC);
-            if (threadIdx.x == 0) claim[(kk + 1) & 1] = nxt;
-            continue;
-        }
-        const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-        const int n = tl.z, pos0 = tl.y;
-        G53GrpLd<NW> ld;
+    constexpr int s = k & 1, m = (k >> 1) & 1;
+    const uint8_t *b0 = sl + (k < 4 ? x4[2 * s] + m * G53_GRP_PL : a4[2 * s] + m * DA);
+    const uint8_t *b1 = sl + (k < 4 ? x4[2 * s + 1] + m * G53_GRP_PL : a4[2 * s + 1] + m * DA);
+    const g53_v4i lo = *(const g53_v4i *)b0, hi = *(const g53_v4i *)b1;
+    (k < 4 ? o.x[m][s] : o.a[m][s]) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+/* The two tiles' products in turn (two independent chains); between<m>() goes in after matrix
+ * instruction m (0-7): a wave issues in order, and 64 cycles of matrix work hide the LDS reads and
+ * loads that would otherwise be issued before it. */
+template <class F>
+__device__ __forceinline__ void g53_grp_mul(g53_v16f (&acc)[2], const G53GrpOps &o, F &&between)
+{
+    g53_v16f b[2] = {};
+#define G53_MUL(m)                                                                                             \
+    b[m & 1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(o.a[m & 1][(m >> 1) & 1], o.x[m >> 2][(m >> 1) & 1], \
+                                                               b[m & 1], 0, 0, 0, 127, 0, 127 - 4 * (m >> 2)); \
+    __builtin_amdgcn_sched_barrier(0);                                                                         \
+    between(G53Int<m>{});                                                                                      \
+    __builtin_amdgcn_sched_barrier(0)
+    G53_MUL(0); G53_MUL(1); G53_MUL(2); G53_MUL(3); G53_MUL(4); G53_MUL(5); G53_MUL(6); G53_MUL(7);
+#undef G53_MUL
 #pragma unroll
-        for (int j = 0; j < G53GrpLd<NW>::RPT; j++) {
-            const int lp = (tid >> 3) + j * 8 * NW, piece = tid & 7;
-            ld.src[j] = a.xq + (size_t)a.tok_of[pos0 + (lp < n ? lp : 0)] * a.E + piece * 16;
-            ld.dst[j] = lp * G53_GRP_XST + piece * 16;
-        }
-        const size_t xps = (size_t)a.T * a.E;
-        /* this lane's weight row */
-        const int i = lane & 31, g = lane >> 5;
-        const int r0 = mb * 16 * NW + w * 16;                /* first intermediate row of the wave */
-        const G53hMat &m = i < 16 ? ex->gate : ex->up;
-        const int wr = r0 + (i & 15);
-        const uint8_t *arow = a.tiled ? m.w + (size_t)(wr >> 3) * NKB * 1024 + (wr & 7) * 128 + g * 64
-                                      : m.w + (size_t)wr * a.E + g * 64;
-        const int kst = a.tiled ? 1024 : 128;
-        const float *s0 = (const float *)ex->gate.s + (size_t)(r0 / 128) * ex->gate.scols;
-        const float *s1 = (const float *)ex->up.s + (size_t)(r0 / 128) * ex->up.scols;
-        g53_v16f acc[G53_GRP_NH] = {};
-        /* the token scales of the tile's positions into LDS before the weights stream (read in
-         * registers at the end, the compiler would load them there, behind the weights) */
-        if (tid < n) xil[tid] = a.xinv[a.tok_of[pos0 + tid]];
-        G53_GTRACE(1, __builtin_amdgcn_s_memrealtime());
-        if (threadIdx.x < 2 * G53_GRP_NS) flags[threadIdx.x] = 0;
-        if (threadIdx.x == 0) claim[(kk + 1) & 1] = nxt;
-        __syncthreads();
-        float xi[G53_GRP_NH];                                /* this lane's positions' scales */
+    for (int f = 0; f < 2; f++)
 #pragma unroll
-        for (int h = 0; h < G53_GRP_NH; h++) xi[h] = xil[h * 32 + i];
-        int spin_err = 0;
-        switch ((n + 31) >> 5) {
-        case 1: g53_grp_kloop<NW, G53_GRP_NPX, NKB, 1>(acc, arow, kst, s0, s1, ld, xps, xs, flags, spin_err, lane); break;
-        case 2: g53_grp_kloop<NW, G53_GRP_NPX, NKB, 2>(acc, arow, kst, s0, s1, ld, xps, xs, flags, spin_err, lane); break;
-        case 3: g53_grp_kloop<NW, G53_GRP_NPX, NKB, 3>(acc, arow, kst, s0, s1, ld, xps, xs, flags, spin_err, lane); break;
-        default: g53_grp_kloop<NW, G53_GRP_NPX, NKB, 4>(acc, arow, kst, s0, s1, ld, xps, xs, flags, spin_err, lane); break;
-        }
-        if (spin_err && lane == 0) atomicOr(&a.meta_w[1], G53_GRP_ESPIN);
-        G53_GTRACE(2, __builtin_amdgcn_s_memrealtime());
-        G53_GTRACE_W(8 + w, __builtin_amdgcn_s_memrealtime());
-        /* epilogue: SwiGLU; the activation planes of the item's 128 rows go to LDS in their final
-         * byte order (the tiled order within the 128-column block when the pass is tiled), then
-         * leave as whole 16-byte pieces: a lane's own bytes are scattered over 64 positions, and
-         * storing them one by one from each lane costs the address unit about 3 us per 32
-         * positions */
-#pragma unroll
-        for (int h = 0; h < G53_GRP_NH; h++) {
-            const int j = h * 32 + i;
-            if (j >= n) continue;
-            uint32_t pk[2][G53_GRP_NPA];
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                float v[4];
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int r = q * 4 + k;
-                    v[k] = g53_grp_swiglu(acc[h][r] * xi[h], acc[h][r + 8] * xi[h], a.limit) * a.aq_scale;
-                }
-                g53_split_planes<G53_GRP_NPA>(v, pk[q]);
-            }
-            /* C register q * 4 + k holds local row w * 16 + q * 8 + g * 4 + k of the block */
-#pragma unroll
-            for (int p = 0; p < G53_GRP_NPA; p++) {
-                uint8_t *d = ao + (p * G53_GRP_NT + j) * 128;
-                if (a.tiled) {          /* rows of q = 0 and 1 are neighbouring bytes of one run */
-#pragma unroll
-                    for (int k = 0; k < 4; k++)
-                        *(uint16_t *)(d + (g53_grp_tpos(g * 4 + k) & ~15) + 2 * w) =
-                            (uint16_t)(((pk[0][p] >> (8 * k)) & 0xffu) | (((pk[1][p] >> (8 * k)) & 0xffu) << 8));
-                } else {
-                    *(uint32_t *)(d + w * 16 + g * 4) = pk[0][p];
-                    *(uint32_t *)(d + w * 16 + 8 + g * 4) = pk[1][p];
-                }
-            }
-        }
-        __syncthreads();
-        for (int c = tid; c < n * G53_GRP_NPA * 8; c += 64 * NW) {
-            const int p = c / (n * 8), jq = c - p * n * 8, j = jq >> 3, piece = jq & 7;
-            *(g53_v4i *)(a.aq + ((size_t)p * a.P + pos0 + j) * a.I + mb * 128 + piece * 16) =
-                *(const g53_v4i *)(ao + (p * G53_GRP_NT + j) * 128 + piece * 16);
-        }
-        G53_GTRACE(3, __builtin_amdgcn_s_memrealtime());
-        G53_GTRACE_W(16 + w, __builtin_amdgcn_s_memrealtime());
-    }
+        for (int r = 0; r < 16; r++) acc[f][r] = fmaf(b[f][r], r < 8 ? o.c0 : o.c1, acc[f][r]);
 }
 
-/* Down for (tile, block mb of 32*NW rows): wave w owns rows mb*32*NW + w*32 + 0..31 of the down
- * matrix (inside one 128-row scale block), the tile's activation planes are the B operand. */
-template <int NW, int NKB>
-__global__ void __launch_bounds__(64 * NW, G53_GRP_WPC) k_grp_down(G53GrpArgs a)
+/* The items of a launch. The dispatcher deals workgroups round-robin over the 8 XCDs, so the
+ * workgroups of XCD x (blockIdx.x % 8 == x) share the items [blo, bhi) (a range of equal estimated
+ * cost, from the planner) and take them in turn. Items are numbered segment by segment, and inside
+ * a segment row block by row block, all tiles of a block in a row: the tiles of one expert that
+ * re-read the same weight rows run side by side on one XCD and find them in its L2. */
+struct G53GrpItem {
+    int4 tl;                       /* the tile; tl.z == 0: no item                       */
+    int mb, many;                  /* row block; whether other tiles share its rows      */
+    int num;
+    const G53hExpert *ex;
+};
+
+/* GATEUP: gate/up rows and SwiGLU for (tile, 128 intermediate rows): LDS rows 0-127 are the gate
+ * rows, 128-255 the up rows of the same indices, and a wave's 32 rows are 16 gate rows and the same
+ * 16 up rows, so C registers r and r + 8 of a lane are gate and up of one row and position; the
+ * activations leave as E4M3 planes. Otherwise: 256 down rows times the activation planes into the
+ * contributions.
+ *
+ * Bound by HBM while tiles hold at most 32 positions: 32 KB of codes a step and CU. Hidden 4096,
+ * inter 2048, 288 experts, gate/up: 150 tokens over 202 experts 613 -> 540 us (6.3 TB/s; a stream of
+ * the same bytes and nothing else reaches 6.2, non-temporal 6.6), 64 tokens 436 -> 410 us. (Weights in
+ * registers, fetched in 16-byte pieces of 32 rows, two blocks in flight behind the positions' loads,
+ * gave the first figures.) 2048 tokens: 1124 -> 1100 us: 453 tiles, of which most hold 33 - 64
+ * positions; a step then takes about 1900 cycles (1024 of matrix instructions a SIMD, which the LDS
+ * reads, the scaling and the barrier do not overlap whole) at the 1.6 GHz that the card's power
+ * allows, and no wave waits for memory. */
+template <bool GATEUP>
+__global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
 {
-    __shared__ __attribute__((aligned(16))) uint8_t xs[G53_GRP_NS * G53_GRP_NPA * G53_GRP_NT * G53_GRP_XST];
-    __shared__ int flags[2 * G53_GRP_NS];
-    __shared__ int claim[2];
-    constexpr int MR = 32 * NW;
-    int *ctr = a.ctr + 8 + (blockIdx.x & 7);
-    if (threadIdx.x == 0) claim[0] = g53_grp_claim(ctr);
-    if (blockIdx.x == 0 && threadIdx.x < 8) a.ctr[threadIdx.x] = 0;        /* the gate/up kernel's */
-    const int blo = a.meta[G53_GRP_BDN + (blockIdx.x & 7)], bhi = a.meta[G53_GRP_BDN + (blockIdx.x & 7) + 1];
-    for (int kk = 0;; kk++) {
-        __syncthreads();                     /* claim[] written; the previous item is done with LDS */
-        int4 tl;
-        int mb;
-        if (!g53_grp_item(a.tiles, blo, bhi, a.E / MR, claim[kk & 1], tl, mb)) break;
-        int nxt = 0;
-        if (threadIdx.x == 0) nxt = g53_grp_claim(ctr);
-        const G53hExpert *ex = tl.x < a.NE ? &a.experts[tl.x] : a.shared;
-        const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-        const int n = tl.z, pos0 = tl.y;
-        const int i = lane & 31, g = lane >> 5;
-        const bool present = ex && ex->gate.w != nullptr;
-        if (!present && a.partial && !(ex && (ex->gate.flags & G53H_MAT_DROPPED))) {   /* another batch */
-            if (tid == 0) claim[(kk + 1) & 1] = nxt;
-            continue;
-        }
-        const bool ok = present && g53_grp_desc_ok(*ex, a.E, a.I, a.tiled);
-        if (!ok) {                                           /* zero contributions */
-            for (int q = tid; q < n * (MR / 4); q += 64 * NW) {
-                const int j = q / (MR / 4), c = (q % (MR / 4)) * 4;
-                *(float4 *)(a.contrib + (size_t)(pos0 + j) * a.E + mb * MR + c) = make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-            if (tid == 0) claim[(kk + 1) & 1] = nxt;
-            continue;
-        }
-        G53GrpLd<NW> ld;
+    __shared__ __attribute__((aligned(1024))) uint8_t ring[G53_GRP_NS * G53_GRP_SLOT];
+    __shared__ float xil[2][64];                             /* the items' token scales ...      */
+    __shared__ float scl[2][64];                             /* ... and block scales: two rows   */
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 31, g = lane >> 5;
+    const int K = GATEUP ? a.E : a.I, MB = GATEUP ? a.I / 128 : a.E / 256, nkb = K / 128;
+    const int nper = (int)(gridDim.x >> 3), bnd = (GATEUP ? G53_GRP_BGU : G53_GRP_BDN) + (int)(blockIdx.x & 7);
+    const int bhi = g53_sld(a.meta + bnd + 1);
+    int loc = g53_sld(a.meta + bnd) + (int)(blockIdx.x >> 3);
+    const uint32_t lring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)ring;
+    const uint32_t lxil = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float *)&xil[0][0];
+    const uint32_t lscl = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float *)&scl[0][0];
+
+    /* this lane's part of a load instruction: row lane / 8 of eight, piece lane % 8 of LDS */
+    const int lr = lane >> 3, lp = lane & 7;
+    uint32_t voa[4];                                         /* the wave's four octets of weight rows */
 #pragma unroll
-        for (int j = 0; j < G53GrpLd<NW>::RPT; j++) {
-            const int lp = (tid >> 3) + j * 8 * NW, piece = tid & 7;
-            ld.src[j] = a.aq + (size_t)(pos0 + (lp < n ? lp : 0)) * a.I + piece * 16;
-            ld.dst[j] = lp * G53_GRP_XST + piece * 16;
-        }
-        const size_t xps = (size_t)a.P * a.I;
-        const int r0 = mb * MR + w * 32;
-        const int wr = r0 + i;
-        const uint8_t *arow = a.tiled ? ex->down.w + (size_t)(wr >> 3) * NKB * 1024 + (wr & 7) * 128 + g * 64
-                                      : ex->down.w + (size_t)wr * a.I + g * 64;
-        const int kst = a.tiled ? 1024 : 128;
-        const float *s0 = (const float *)ex->down.s + (size_t)(r0 / 128) * ex->down.scols;
-        g53_v16f acc[G53_GRP_NH] = {};
-        if (threadIdx.x < 2 * G53_GRP_NS) flags[threadIdx.x] = 0;
-        if (threadIdx.x == 0) claim[(kk + 1) & 1] = nxt;
-        __syncthreads();
-        int spin_err = 0;
-        switch ((n + 31) >> 5) {
-        case 1: g53_grp_kloop<NW, G53_GRP_NPA, NKB, 1>(acc, arow, kst, s0, s0, ld, xps, xs, flags, spin_err, lane); break;
-        case 2: g53_grp_kloop<NW, G53_GRP_NPA, NKB, 2>(acc, arow, kst, s0, s0, ld, xps, xs, flags, spin_err, lane); break;
-        case 3: g53_grp_kloop<NW, G53_GRP_NPA, NKB, 3>(acc, arow, kst, s0, s0, ld, xps, xs, flags, spin_err, lane); break;
-        default: g53_grp_kloop<NW, G53_GRP_NPA, NKB, 4>(acc, arow, kst, s0, s0, ld, xps, xs, flags, spin_err, lane); break;
-        }
-        if (spin_err && lane == 0) atomicOr(&a.meta_w[1], G53_GRP_ESPIN);
-#pragma unroll
-        for (int h = 0; h < G53_GRP_NH; h++) {
-            const int j = h * 32 + i;
-            if (j >= n) continue;
-            float *dst = a.contrib + (size_t)(pos0 + j) * a.E + r0 + g * 4;
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                *(float4 *)(dst + q * 8) = make_float4(acc[h][q * 4] * a.aq_inv, acc[h][q * 4 + 1] * a.aq_inv,
-                                                       acc[h][q * 4 + 2] * a.aq_inv, acc[h][q * 4 + 3] * a.aq_inv);
-        }
+    for (int o = 0; o < 4; o++) {
+        const int c = lp ^ ((4 * (o & 1) + (lane >> 4)) & 7);
+        voa[o] = (uint32_t)(8 * o * K + (a.tiled ? lr * 128 + c * 16 : lr * K + c * 16));
     }
+    const uint32_t vox = (uint32_t)((lp ^ ((4 * (w & 1) + (lane >> 4)) & 7)) * 16);
+    const int kst = a.tiled ? 1024 : 128;
+    const size_t xps = GATEUP ? (size_t)a.T * a.E : (size_t)a.P * a.I;
+    auto item_at = [&](int n) {
+        G53GrpItem it;
+        const int w0 = g53_sld(&a.tiles[n / MB].w);          /* a tile of the item's segment */
+        const int ts0 = w0 & 0xffff, nts = w0 >> 16, q = n - ts0 * MB;
+        it.mb = q / nts;
+        it.many = nts > 1;
+        const int *t = (const int *)(a.tiles + ts0 + q % nts);
+        it.tl = make_int4(g53_sld(t), g53_sld(t + 1), g53_sld(t + 2), 0);
+        it.num = n;
+        it.ex = it.tl.x < a.NE ? a.experts + it.tl.x : a.shared;
+        return it;
+    };
+    /* the workgroup's next item whose expert can be multiplied; the others are dealt with here */
+    auto next_item = [&]() {
+        for (;; loc += nper) {
+            if (loc >= bhi) return G53GrpItem{make_int4(0, 0, 0, 0), 0, 0, 0, nullptr};
+            G53GrpItem it = item_at(loc);
+            const G53hExpert *ex = it.ex;
+            const bool present = ex && g53_sld(&ex->gate.w) != nullptr;
+            if (present && g53_grp_desc_ok(ex, a.E, a.I, a.tiled)) {
+                loc += nper;
+                return it;
+            }
+            if (GATEUP) {                                    /* the down launch writes its zeros */
+                if (present && tid == 0) atomicOr(&a.meta_w[1], G53_GRP_EDESC);
+            } else if (present || !a.partial || (ex && (g53_sld(&ex->gate.flags) & G53H_MAT_DROPPED))) {
+                for (int q = tid; q < it.tl.z * 64; q += 64 * G53_GRP_NW)
+                    *(float4 *)(a.contrib + (size_t)(it.tl.y + (q >> 6)) * a.E + it.mb * 256 + (q & 63) * 4) =
+                        make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+        }
+    };
+
+    /* an item as requests need it: its bases, and this lane's positions in the planes */
+    struct Bound {
+        const uint8_t *pa, *px;
+        uint32_t vx[2];
+        int mode;                                            /* 0 streamed, 1 shared by tiles, 2 unaligned */
+    };
+    auto bind = [&](const G53GrpItem &it) {
+        Bound r;
+        const int n = it.tl.z, row = (w & 3) * 8;
+        const uint8_t *m;
+        if (GATEUP) {
+            m = w < 4 ? g53_sld(&it.ex->gate.w) : g53_sld(&it.ex->up.w);
+            r.pa = m + (size_t)(it.mb * 128 + (w & 3) * 32) * K;
+            r.px = a.xq;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                int tk = 0;
+#pragma unroll
+                for (int q = 0; q < 8; q++) {                /* past the tile's end: its first position */
+                    const int rr = row + 32 * h + q, v = g53_sld(a.tok_of + it.tl.y + (rr < n ? rr : 0));
+                    tk = lr == q ? v : tk;
+                }
+                r.vx[h] = (uint32_t)((w >> 2) * xps + (size_t)tk * K) + vox;
+            }
+        } else {
+            m = g53_sld(&it.ex->down.w);
+            r.pa = m + (size_t)(it.mb * 256 + w * 32) * K;
+            r.px = a.aq + (size_t)it.tl.y * K;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int rr = row + 32 * h + lr;
+                r.vx[h] = (uint32_t)((w >> 2) * xps + (size_t)(rr < n ? rr : 0) * K) + vox;
+            }
+        }
+        r.mode = ((uintptr_t)m & 15) ? 2 : it.many;
+        return r;
+    };
+    /* request the block at r.pa / r.px into a slot (LDS byte so) and step to the next block */
+    auto request = [&](Bound &r, uint32_t so) {
+        const uint32_t ls = lring + so + w * 4096, lx = lring + so + G53_GRP_SA + (w >> 2) * G53_GRP_PL + (w & 3) * 1024;
+        /* rows that one tile reads are streamed past the caches: 540 against 567 us at 150 tokens
+         * (gate/up); rows that several tiles read come from L2 for all but the first */
+        if (r.mode == 0) g53_dma_rows_nt(voa, r.pa, ls);
+        else if (r.mode == 1) g53_dma_rows(voa, r.pa, ls);
+        else {                                               /* codes that are not 16-byte aligned: by registers */
+#pragma unroll
+            for (int o = 0; o < 4; o++) {
+                g53_v4i v;
+                __builtin_memcpy(&v, r.pa + voa[o], 16);
+                *(g53_v4i *)(ring + so + w * 4096 + o * 1024 + lane * 16) = v;
+            }
+        }
+        g53_dma16(r.vx[0], r.px, lx);
+        g53_dma16(r.vx[1], r.px, lx + 4096);
+        /* with fewer than six loads the steps' waits would not count right: this wave's all land here */
+        if (r.mode == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        r.pa += kst;
+        r.px += 128;
+    };
+    auto scales = [&](const G53GrpItem &it, int par) {       /* the item's scales, by waves 0 and 1 */
+        if (GATEUP && w == 0) g53_dma4(a.xinvp + it.tl.y + min(lane, it.tl.z - 1), lxil + par * 256);
+        if (w == 1) {                                        /* rows: gate and up, or the item's two of down */
+            const G53hExpert *ex = it.ex;
+            const float *r0, *r1;
+            if (GATEUP) {
+                r0 = g53_sld(&ex->gate.s) + (size_t)it.mb * g53_sld(&ex->gate.scols);
+                r1 = g53_sld(&ex->up.s) + (size_t)it.mb * g53_sld(&ex->up.scols);
+            } else {
+                r0 = g53_sld(&ex->down.s) + (size_t)(2 * it.mb) * g53_sld(&ex->down.scols);
+                r1 = r0 + g53_sld(&ex->down.scols);
+            }
+            g53_dma4((g ? r1 : r0) + min(i, nkb - 1), lscl + par * 256);
+        }
+    };
+    /* this wave's first row in an item (gate/up: intermediate row) and its half of the positions;
+     * its lanes' operand pieces in a slot */
+    const int rw = (w & 3) * (GATEUP ? 32 : 64), half = w >> 2;
+    int a4[4], x4[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int po = ((4 * g + q) ^ ((i >> 1) & 7)) * 16;
+        a4[q] = (GATEUP ? rw + (i & 15) + (i & 16) * 8 : rw + i) * 128 + po;
+        x4[q] = G53_GRP_SA + (half * 32 + i) * 128 + po;
+    }
+    /* fragment k of the operands of block kb of the item of parity pr from a slot (8: its scales) */
+    auto fetch = [&](auto k, G53GrpOps &o, int kb, int pr, uint32_t so) {
+        if constexpr (decltype(k)::value == 8) {
+            o.c0 = scl[pr][GATEUP ? kb : (w & 2) * 16 + kb];
+            o.c1 = GATEUP ? scl[pr][32 + kb] : o.c0;
+        } else {
+            g53_grp_fetch<(GATEUP ? 16 : 32) * 128, decltype(k)::value>(o, ring + so, a4, x4);
+        }
+    };
+    auto fetch_all = [&](G53GrpOps &o, int kb, int pr, uint32_t so) {
+        fetch(G53Int<0>{}, o, kb, pr, so); fetch(G53Int<1>{}, o, kb, pr, so); fetch(G53Int<2>{}, o, kb, pr, so);
+        fetch(G53Int<3>{}, o, kb, pr, so); fetch(G53Int<4>{}, o, kb, pr, so); fetch(G53Int<5>{}, o, kb, pr, so);
+        fetch(G53Int<6>{}, o, kb, pr, so); fetch(G53Int<7>{}, o, kb, pr, so); fetch(G53Int<8>{}, o, kb, pr, so);
+    };
+
+    G53GrpItem cur = next_item();
+    if (cur.tl.z == 0) return;
+    Bound bd = bind(cur);
+    G53GrpOps ops[2];
+    int par = 0;
+    uint32_t so = 0;                                         /* slot of the step being multiplied */
+    scales(cur, 0);
+    request(bd, 0);
+    request(bd, G53_GRP_SLOT);
+    request(bd, 2 * G53_GRP_SLOT);
+    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    g53_grp_bar();
+    fetch_all(ops[0], 0, 0, 0);
+    for (;;) {
+        const int n = cur.tl.z, pos0 = cur.tl.y;
+        if (GATEUP && a.trace && tid == 0) {
+            uint64_t *tr = a.trace + (size_t)cur.num * 32;
+            tr[0] = __builtin_amdgcn_s_memrealtime();
+            tr[4] = (uint64_t)__smid() << 32 | (uint32_t)(pos0 << 8 | n);
+            tr[5] = (uint64_t)blockIdx.x << 32 | (uint32_t)(cur.tl.x << 8 | cur.mb);
+        }
+        const G53GrpItem nx = next_item();
+        /* past the last item, its own blocks are requested again, so that every step is alike */
+        const Bound nb = bind(nx.tl.z ? nx : cur);
+        const bool act = half * 32 < n, actn = half * 32 < nx.tl.z;
+        g53_v16f acc[2] = {};
+        /* A step: the next step's six loads have landed - this wave's by the wait, every wave's by
+         * the barrier, which also ends every wave's reads of the step being multiplied, so its slot
+         * is requested again, three steps ahead; the next step's operands leave LDS while this
+         * step's, read a step ago, are multiplied. Waves without positions only load. */
+        auto step = [&](int kb, G53GrpOps &o, G53GrpOps &on) {
+            asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+            g53_grp_bar();
+            if (kb == nkb - 3) {
+                bd = nb;
+                if (nx.tl.z) scales(nx, par ^ 1);
+            }
+            const uint32_t rs = so;
+            so = so == 2 * G53_GRP_SLOT ? 0u : so + G53_GRP_SLOT;
+            const bool last = kb + 1 == nkb;
+            const int kn = last ? 0 : kb + 1, pn = last ? par ^ 1 : par;
+            if (act)
+                g53_grp_mul(acc, o, [&](auto m) {
+                    fetch(m, on, kn, pn, so);
+                    if constexpr (decltype(m)::value == 0) request(bd, rs);
+                    if constexpr (decltype(m)::value == 7) fetch(G53Int<8>{}, on, kn, pn, so);
+                });
+            else {
+                request(bd, rs);
+                if (last && actn) fetch_all(on, kn, pn, so);
+            }
+        };
+        for (int kb = 0; kb < nkb; kb += 2) {
+            step(kb, ops[0], ops[1]);
+            step(kb + 1, ops[1], ops[0]);
+        }
+        if (GATEUP && a.trace && tid == 0) a.trace[(size_t)cur.num * 32 + 2] = __builtin_amdgcn_s_memrealtime();
+        const int j = half * 32 + i;                         /* this lane's position */
+        if (GATEUP) {
+            /* SwiGLU; the activation planes of the item's 128 rows are put together in the slot
+             * whose operands have been read, in their final byte order (the tiled order within the 128-column
+             * block when the pass is tiled), and leave as whole 16-byte pieces */
+            uint8_t *ao = ring + so;
+            const float xi = xil[par][j];
+            g53_grp_bar();                                   /* every wave is done with the slot */
+#pragma unroll
+            for (int f = 0; f < 2; f++) {
+                if (j >= n) continue;
+                uint32_t pk[2][G53_GRP_NPA];
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    float v[4];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const int r = q * 4 + k;
+                        v[k] = g53_grp_swiglu(acc[f][r] * xi, acc[f][r + 8] * xi, a.limit) * a.aq_scale;
+                    }
+                    g53_split_planes<G53_GRP_NPA>(v, pk[q]);
+                }
+                /* C register q * 4 + k holds row rb + q * 8 + g * 4 + k of the block */
+                const int rb = rw + f * 16;
+#pragma unroll
+                for (int p = 0; p < G53_GRP_NPA; p++) {
+                    uint8_t *d = ao + (p * G53_GRP_NT + j) * 128;
+                    if (a.tiled) {          /* rows of q = 0 and 1 are neighbouring bytes of one run */
+#pragma unroll
+                        for (int k = 0; k < 4; k++)
+                            *(uint16_t *)(d + (g53_grp_tpos(g * 4 + k) & ~15) + (rb >> 3)) =
+                                (uint16_t)(((pk[0][p] >> (8 * k)) & 0xffu) | (((pk[1][p] >> (8 * k)) & 0xffu) << 8));
+                    } else {
+                        *(uint32_t *)(d + rb + g * 4) = pk[0][p];
+                        *(uint32_t *)(d + rb + 8 + g * 4) = pk[1][p];
+                    }
+                }
+            }
+            g53_grp_bar();
+            for (int c = tid; c < n * G53_GRP_NPA * 8; c += 64 * G53_GRP_NW) {
+                const int p = c / (n * 8), jq = c - p * n * 8, jj = jq >> 3, piece = jq & 7;
+                *(g53_v4i *)(a.aq + ((size_t)p * a.P + pos0 + jj) * a.I + cur.mb * 128 + piece * 16) =
+                    *(const g53_v4i *)(ao + (p * G53_GRP_NT + jj) * 128 + piece * 16);
+            }
+            if (a.trace && tid == 0) a.trace[(size_t)cur.num * 32 + 3] = __builtin_amdgcn_s_memrealtime();
+        } else {
+#pragma unroll
+            for (int f = 0; f < 2; f++) {
+                if (j >= n) continue;
+                float *dst = a.contrib + (size_t)(pos0 + j) * a.E + cur.mb * 256 + rw + f * 32 + g * 4;
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    *(float4 *)(dst + q * 8) = make_float4(acc[f][q * 4] * a.aq_inv, acc[f][q * 4 + 1] * a.aq_inv,
+                                                           acc[f][q * 4 + 2] * a.aq_inv, acc[f][q * 4 + 3] * a.aq_inv);
+            }
+        }
+        if (nx.tl.z == 0) break;
+        cur = nx;
+        par ^= 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         /* no load may outlive the workgroup's LDS */
 }
 
 /* out[t][d] = (float)(sum_j (double)w[t][j] * (double)contrib[pos(t,j)][d]) (+ shared, float):
@@ -854,7 +840,7 @@ static int g53_grp_plan_pass(const float *x, int tc, const G53hMoeLayer *L, cons
     int *pos_of = (int *)p;   p += al256((size_t)tc * (K + 1) * 4);
     int4 *tiles = (int4 *)p;  p += al256((size_t)maxtiles * 16);
     uint8_t *xq = (uint8_t *)p; p += al256((size_t)G53_GRP_NPX * tc * E);
-    float *xinv = (float *)p; p += al256((size_t)tc * 4);
+    float *xinvp = (float *)p; p += al256((size_t)P * 4);
     uint8_t *aq = (uint8_t *)p; p += al256((size_t)G53_GRP_NPA * P * I);
     float *contrib = (float *)p;
     const int nch = (tc + 63) / 64;
@@ -862,9 +848,10 @@ static int g53_grp_plan_pass(const float *x, int tc, const G53hMoeLayer *L, cons
     if (lds > 160 * 1024) return g53h_fail("g53h_moe_grouped: %zu bytes of planner LDS", lds);
     if (lds > 65536) G53_TRY(hipFuncSetAttribute((const void *)k_grp_plan, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k_grp_plan, dim3(1), dim3(1024), lds, st, idx, tc, K, NE, hs, tok_of, pos_of, tiles, meta,
-                       I / (16 * G53_GRP_NW), E / (32 * G53_GRP_NW));
+                       I / 128, E / 256);
     G53_LAUNCHED("k_grp_plan");
-    hipLaunchKernelGGL(k_grp_xq<G53_GRP_NPX>, dim3(tc), dim3(256), 0, st, x, E, tc, xq, xinv, L->tiled ? 1 : 0);
+    hipLaunchKernelGGL(k_grp_xq<G53_GRP_NPX>, dim3(tc), dim3(256), 0, st, x, E, tc, xq, xinvp, pos_of, K + 1, K + hs,
+                       L->tiled ? 1 : 0);
     G53_LAUNCHED("k_grp_xq");
     g53h_prof_mark(G53_PROF_GROUPED);
     float bound = L->swiglu_limit > 0.28f ? L->swiglu_limit : 0.28f;
@@ -872,8 +859,8 @@ static int g53_grp_plan_pass(const float *x, int tc, const G53hMoeLayer *L, cons
     int ex = 0;
     (void)frexpf(bound, &ex);                      /* |act| <= bound < 2^ex */
     G53GrpArgs &a = g_pass.a;
-    a.experts = L->experts; a.shared = L->shared; a.tiles = tiles; a.meta = meta; a.meta_w = meta; a.ctr = meta + 2;
-    a.tok_of = tok_of; a.xq = xq; a.xinv = xinv; a.aq = aq; a.contrib = contrib;
+    a.experts = L->experts; a.shared = L->shared; a.tiles = tiles; a.meta = meta; a.meta_w = meta;
+    a.tok_of = tok_of; a.xq = xq; a.xinvp = xinvp; a.aq = aq; a.contrib = contrib;
     a.T = tc; a.P = P; a.E = E; a.I = I; a.NE = NE;
     a.limit = L->swiglu_limit; a.aq_scale = ldexpf(1.0f, 8 - ex); a.aq_inv = ldexpf(1.0f, ex - 8);
     a.partial = 0;
@@ -890,25 +877,13 @@ static int g53_grp_run_pass(const G53hExpert *experts, const G53hExpert *shared,
     a.experts = experts; a.shared = shared; a.partial = partial;
     const int E = a.E, I = a.I, maxtiles = g_pass.maxtiles;
     hipStream_t st = g53h_stream();
-    constexpr int NW = G53_GRP_NW;
-    unsigned g1 = (unsigned)((maxtiles * (I / (16 * NW)) + 7) / 8 * 8);
-    unsigned g2 = (unsigned)((maxtiles * (E / (32 * NW))) + 7) / 8 * 8;
-#if G53_GRP_PERS
-    {
-        const unsigned cap = (unsigned)(g53h_num_cus() * G53_GRP_WPC * G53_GRP_PERS) / 8 * 8;
-        if (cap >= 8) { g1 = g1 < cap ? g1 : cap; g2 = g2 < cap ? g2 : cap; }
-    }
-#endif
-#define G53_GU(N) case N: hipLaunchKernelGGL((k_grp_gateup<NW, N>), dim3(g1), dim3(64 * NW), 0, st, a); break
-#define G53_DN(N) case N: hipLaunchKernelGGL((k_grp_down<NW, N>), dim3(g2), dim3(64 * NW), 0, st, a); break
-    switch (E / 128) { G53_GU(4); G53_GU(8); G53_GU(16); G53_GU(32);
-                       default: return g53h_fail("g53h_moe_grouped: hidden %d", E); }
+    const unsigned cap = (unsigned)g53h_num_cus() / 8 * 8;
+    unsigned g1 = (unsigned)(maxtiles * (I / 128) + 7) / 8 * 8, g2 = (unsigned)(maxtiles * (E / 256) + 7) / 8 * 8;
+    if (cap >= 8) { g1 = g1 < cap ? g1 : cap; g2 = g2 < cap ? g2 : cap; }
+    hipLaunchKernelGGL((k_grp_gemm<true>), dim3(g1), dim3(64 * G53_GRP_NW), 0, st, a);
     G53_LAUNCHED("k_grp_gateup");
     g53h_prof_mark(G53_PROF_GATEUP);
-    switch (I / 128) { G53_DN(4); G53_DN(8); G53_DN(16); G53_DN(32);
-                       default: return g53h_fail("g53h_moe_grouped: inter %d", I); }
-#undef G53_GU
-#undef G53_DN
+    hipLaunchKernelGGL((k_grp_gemm<false>), dim3(g2), dim3(64 * G53_GRP_NW), 0, st, a);
     G53_LAUNCHED("k_grp_down");
     g53h_prof_mark(G53_PROF_DOWN);
     return 0;
@@ -941,7 +916,7 @@ static size_t g53_grp_ws(const G53hMoeLayer *L, int tc)
     const size_t P = (size_t)tc * K + (size_t)hs * tc;
     const int maxtiles = (tc * K + G53_GRP_NT - 1) / G53_GRP_NT + NE + hs * ((tc + G53_GRP_NT - 1) / G53_GRP_NT);
     return al256(P * 4) + al256((size_t)tc * (K + 1) * 4) + al256((size_t)maxtiles * 16) +
-           al256((size_t)G53_GRP_NPX * tc * E) + al256((size_t)tc * 4) + al256((size_t)G53_GRP_NPA * P * I) +
+           al256((size_t)G53_GRP_NPX * tc * E) + al256(P * 4) + al256((size_t)G53_GRP_NPA * P * I) +
            al256(P * E * 4);
 }
 

@@ -225,7 +225,7 @@ int g53h_moe_combine(float *out_d, const float *contrib_d, const float *w_d, int
  * g53h_moe takes this path for T >= 2 when g53h_set_grouped is on (the default; it returns the
  * previous setting) and the layer qualifies; otherwise the exact per-token kernels.
  * g53h_grouped_errors waits for the stream and returns, then clears, the grouped kernels' flags
- * (1: a routed index out of range, 2: a wait between waves timed out, 8: an expert descriptor
+ * (1: a routed index out of range, 8: an expert descriptor
  * without the 128x128 layout). */
 int g53h_moe_grouped(float *out_d, const float *x_d, int T, const G53hMoeLayer *L, int *idx_d,
                      float *w_d);

@@ -1,0 +1,61 @@
+"""The grouped GEMMs' step pipeline at the edges of its tiles (32 and 64 positions), of its shortest
+and longest items (4 to 32 steps), over both code layouts and over codes that are not 16-byte
+aligned (replaces src/core/glm53f_ops.c:376-444 in :1144-1342). Every expert is chosen by every
+token, so a tile's positions are the batch's tokens. Bar: routing bit-exact, outputs within the
+path's tolerance of the oracle."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import glm53h
+import glm53h.synth as S
+from glm53h import DevBuf, G53hExpert, G53hMat, check
+from test_gpu_grouped import oracle_out, run, say, within
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def L():
+    return glm53h.init(0)
+
+
+@pytest.mark.parametrize("E,inter,T,tiled", [
+    (512, 512, 2, True), (512, 512, 32, False), (512, 1024, 33, True), (1024, 512, 64, False),
+    (1024, 1024, 65, True), (2048, 512, 97, False), (512, 2048, 129, True), (4096, 512, 31, True),
+    (512, 4096, 63, False)])
+def test_grouped_tile_edges(L, E, inter, T, tiled):
+    say("tile edges", E, inter, T, tiled)
+    sp = S.LayerSpec(E=E, I=inter, NE=3, K=3, router_sigma=0.02)
+    layer = S.DeviceLayer.build(sp, tiled=tiled)
+    x = S.x_host(sp, T, batch=1)
+    out, idx, w = run(layer, x, 1, "g53h_moe_grouped")
+    want, wi, ww = oracle_out(layer, x, idx)
+    assert np.array_equal(idx, wi) and np.array_equal(w.view(np.uint32), ww.view(np.uint32))
+    within(out, want, f"E={E} I={inter} T={T}")
+
+
+@pytest.mark.parametrize("shift,T,tiled", [(1, 5, False), (4, 40, True), (8, 130, False)])
+def test_grouped_unaligned_codes(L, shift, T, tiled):
+    """The second expert's codes at an address that is not a multiple of 16, the others aligned: the
+    result is bit for bit that of the aligned layer."""
+    say("unaligned codes", shift, T, tiled)
+    sp = S.LayerSpec(E=1024, I=512, NE=4, K=3, router_sigma=0.02)
+    layer = S.DeviceLayer.build(sp, tiled=tiled)
+    x = S.x_host(sp, T, batch=2)
+    want, wi, _ = run(layer, x, 1, "g53h_moe_grouped")
+    keep = []
+
+    def moved(m):
+        b = DevBuf(m.rows * m.cols + 16)
+        check(L.g53h_d2d(b.ptr + shift, m.w, m.rows * m.cols), "d2d")
+        keep.append(b)
+        return G53hMat(b.ptr + shift, m.s, m.rows, m.cols, m.br, m.bc, m.scols, m.flags)
+
+    e = layer.experts[1]
+    layer.experts[1] = G53hExpert(moved(e.gate), moved(e.up), moved(e.down))
+    layer.table.upload(np.frombuffer(bytes(layer.experts), np.uint8))
+    out, idx, _ = run(layer, x, 1, "g53h_moe_grouped")
+    assert np.array_equal(idx, wi)
+    assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
