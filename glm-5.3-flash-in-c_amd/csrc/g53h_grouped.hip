@@ -337,11 +337,13 @@ __device__ __forceinline__ void g53_grp_bar()
     asm volatile("" ::: "memory");
 }
 
-/* A descriptor with the layout the grouped kernels assume (octet-tiled iff the pass is). */
+/* A descriptor with the layout the grouped kernels assume: octet-tiled iff the pass is, or
+ * MFMA-tiled in an MFMA-tiled pass. */
 __device__ __forceinline__ bool g53_grp_mat_ok(const G53hMat *m, int rows, int cols, int tiled)
 {
     const int fl = g53_sld(&m->flags);
-    return !(fl & G53H_MAT_I4) && (fl & G53H_MAT_TILED) == (tiled ? G53H_MAT_TILED : 0) && g53_sld(&m->br) == 128 &&
+    const int want = tiled == 2 ? G53H_MAT_MTILED : tiled ? G53H_MAT_TILED : 0;
+    return !(fl & G53H_MAT_I4) && (fl & (tiled == 2 ? G53H_MAT_MTILED : G53H_MAT_TILED)) == want && g53_sld(&m->br) == 128 &&
            g53_sld(&m->bc) == 128 && g53_sld(&m->rows) == rows && g53_sld(&m->cols) == cols &&
            g53_sld(&m->scols) >= cols / 128;
 }
@@ -370,7 +372,8 @@ struct G53GrpArgs {
     float *contrib;                /* [P][E]                                             */
     int T, P, E, I, NE;
     float limit, aq_scale, aq_inv;
-    int tiled;                     /* 1: experts octet-tiled, planes in the tiled column order */
+    int tiled;                     /* 1: experts octet-tiled, planes in the tiled column order;
+                                      2: experts MFMA-tiled, planes in column order        */
     int partial;                   /* 1: experts without weights are outside this batch and
                                       left alone, unless marked dropped (gate.flags & G53H_MAT_DROPPED)    */
     uint64_t *trace;               /* optional: [items][32] timestamps of each gate/up item  */
@@ -474,7 +477,9 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
 #pragma unroll
     for (int o = 0; o < 4; o++) {
         const int c = lp ^ ((4 * (o & 1) + (lane >> 4)) & 7);
-        voa[o] = (uint32_t)(8 * o * K + (a.tiled ? lr * 128 + c * 16 : lr * K + c * 16));
+        /* piece c of row lr: of a row's 128 bytes, or of an MFMA-tiled unit its columns 16 c .. */
+        voa[o] = (uint32_t)(8 * o * K + (a.tiled == 2 ? (c & 1) * 512 + (c >> 1) * 128 + lr * 16
+                                         : a.tiled ? lr * 128 + c * 16 : lr * K + c * 16));
     }
     const uint32_t vox = (uint32_t)((lp ^ ((4 * (w & 1) + (lane >> 4)) & 7)) * 16);
     const int kst = a.tiled ? 1024 : 128;
@@ -695,7 +700,7 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
 #pragma unroll
                 for (int p = 0; p < G53_GRP_NPA; p++) {
                     uint8_t *d = ao + (p * G53_GRP_NT + j) * 128;
-                    if (a.tiled) {          /* rows of q = 0 and 1 are neighbouring bytes of one run */
+                    if (a.tiled == 1) {     /* rows of q = 0 and 1 are neighbouring bytes of one run */
 #pragma unroll
                         for (int k = 0; k < 4; k++)
                             *(uint16_t *)(d + (g53_grp_tpos(g * 4 + k) & ~15) + (rb >> 3)) =
@@ -829,7 +834,8 @@ struct G53GrpPass {
 };
 static G53GrpPass g_pass;
 
-static int g53_grp_plan_pass(const float *x, int tc, const G53hMoeLayer *L, const int *idx, char *ws, int *meta)
+/* layout: 0 row-major, 1 octet-tiled, 2 MFMA-tiled experts. */
+static int g53_grp_plan_pass(const float *x, int tc, const G53hMoeLayer *L, const int *idx, char *ws, int *meta, int layout)
 {
     const int E = L->hidden, I = L->inter, K = L->topk, NE = L->n_experts, hs = L->shared ? 1 : 0;
     const int P = tc * K + hs * tc;
@@ -851,7 +857,7 @@ static int g53_grp_plan_pass(const float *x, int tc, const G53hMoeLayer *L, cons
                        I / 128, E / 256);
     G53_LAUNCHED("k_grp_plan");
     hipLaunchKernelGGL(k_grp_xq<G53_GRP_NPX>, dim3(tc), dim3(256), 0, st, x, E, tc, xq, xinvp, pos_of, K + 1, K + hs,
-                       L->tiled ? 1 : 0);
+                       layout == 1);
     G53_LAUNCHED("k_grp_xq");
     g53h_prof_mark(G53_PROF_GROUPED);
     float bound = L->swiglu_limit > 0.28f ? L->swiglu_limit : 0.28f;
@@ -864,7 +870,7 @@ static int g53_grp_plan_pass(const float *x, int tc, const G53hMoeLayer *L, cons
     a.T = tc; a.P = P; a.E = E; a.I = I; a.NE = NE;
     a.limit = L->swiglu_limit; a.aq_scale = ldexpf(1.0f, 8 - ex); a.aq_inv = ldexpf(1.0f, ex - 8);
     a.partial = 0;
-    a.tiled = L->tiled ? 1 : 0;
+    a.tiled = layout;
     a.trace = g_grp_trace;
     g_pass.active = 1; g_pass.tc = tc; g_pass.K = K; g_pass.hs = hs; g_pass.maxtiles = maxtiles;
     g_pass.pos_of = pos_of; g_pass.meta = meta; g_pass.contrib = contrib;
@@ -905,7 +911,7 @@ static int g53_grp_combine_pass(float *out, const float *wts)
 static int g53_grp_chunk(float *out, const float *x, int tc, const G53hMoeLayer *L, const int *idx,
                          const float *wts, char *ws, int *meta)
 {
-    if (g53_grp_plan_pass(x, tc, L, idx, ws, meta) || g53_grp_run_pass(L->experts, L->shared, 0)) return -1;
+    if (g53_grp_plan_pass(x, tc, L, idx, ws, meta, L->tiled ? 1 : 0) || g53_grp_run_pass(L->experts, L->shared, 0)) return -1;
     return g53_grp_combine_pass(out, wts);
 }
 
@@ -964,13 +970,23 @@ static int g53_grp_tcmax(int NE)
     return tcmax > G53_GRP_MAXT ? G53_GRP_MAXT : tcmax;
 }
 
+/* HBM that routing and one planning pass of T tokens may take (the workspace grows by a quarter more
+ * than asked, the router's partial sums are at most 8 doubles a score). */
+extern "C" size_t g53h_grouped_bytes(const G53hMoeLayer *L, int T)
+{
+    const size_t scores = (size_t)T * L->n_experts;
+    return g53_grp_ws(L, T) / 4 * 5 + scores * (2 * sizeof(float) + 8 * sizeof(double)) + (2u << 20);
+}
+
 extern "C" int g53h_grouped_max_tokens(const G53hMoeLayer *L)
 {
     if (!g_grp_mode || !g53_grp_shapes_ok(L)) return 0;
     return g53_grp_tcmax(L->n_experts);
 }
 
-extern "C" int g53h_grouped_begin(const float *x, int T, const G53hMoeLayer *L, const int *idx)
+/* g53h_grouped_begin for experts of a given layout: also MFMA-tiled ones (2), which the drop-in's
+ * cache may hold. */
+extern "C" int g53h_grouped_begin_layout(const float *x, int T, const G53hMoeLayer *L, const int *idx, int layout)
 {
     if (g53h_ready()) return -1;
     if (!g53_grp_shapes_ok(L)) return g53h_fail("g53h_grouped_begin: layer shapes not supported");
@@ -981,14 +997,19 @@ extern "C" int g53h_grouped_begin(const float *x, int T, const G53hMoeLayer *L, 
     }
     char *ws = (char *)g53h_workspace(g53_grp_ws(L, T));
     if (!ws) return -1;
-    return g53_grp_plan_pass(x, T, L, idx, ws, g_grp_err + 16);
+    return g53_grp_plan_pass(x, T, L, idx, ws, g_grp_err + 16, layout);
+}
+
+extern "C" int g53h_grouped_begin(const float *x, int T, const G53hMoeLayer *L, const int *idx)
+{
+    return g53h_grouped_begin_layout(x, T, L, idx, L && L->tiled ? 1 : 0);
 }
 
 extern "C" int g53h_grouped_batch(const G53hMoeLayer *L)
 {
     if (!g_pass.active) return g53h_fail("g53h_grouped_batch: no pass begun");
-    if (L && (L->tiled ? 1 : 0) != g_pass.a.tiled)
-        return g53h_fail("g53h_grouped_batch: the pass was planned for %s experts", g_pass.a.tiled ? "octet-tiled" : "row-major");
+    if (L && (g_pass.a.tiled == 2 ? L->tiled : L->tiled ? 1 : 0) != g_pass.a.tiled)
+        return g53h_fail("g53h_grouped_batch: the pass was planned for %s experts", g_pass.a.tiled == 2 ? "MFMA-tiled" : g_pass.a.tiled ? "octet-tiled" : "row-major");
     if (!L || L->n_experts != g_pass.a.NE || L->hidden != g_pass.a.E || L->inter != g_pass.a.I)
         return g53h_fail("g53h_grouped_batch: another layer than the pass's");
     if (L->shared && !g_pass.hs) return g53h_fail("g53h_grouped_batch: the pass was planned without a shared expert");

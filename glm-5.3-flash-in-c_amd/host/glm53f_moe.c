@@ -1317,6 +1317,196 @@ static void moe_chunk(float *out, const float *x, const Glm53fMoeW *w, const Glm
     errors_check(errs, w->layer, K);
 }
 
+/* ------------------------------------------------ several tokens through the HBM cache ---- */
+size_t g53h_grouped_bytes(const G53hMoeLayer *L, int T);
+int g53h_grouped_begin_layout(const float *x_d, int T, const G53hMoeLayer *L, const int *idx_d, int layout);
+
+static void *g_pin_ids;
+static size_t g_pin_ids_n;
+static int *g_held;                     /* the pass's gets, in order */
+static size_t g_held_n;
+
+static int *held_room(size_t n)
+{
+    if (n <= g_held_n) return g_held;
+    int *p = (int *)realloc(g_held, n * sizeof *p);
+    if (!p) { fprintf(stderr, "glm53f: FATAL, out of host memory\n"); abort(); }
+    g_held = p;
+    g_held_n = n;
+    return p;
+}
+
+/* A run of whole chunks (T tokens, T % 64 != 1) whose experts this library's HBM cache holds tiled:
+ * one routing, then the reference's calls chunk by chunk in its order (hints, getmany, gets; moe_chunk
+ * above), then one grouped pass over all T tokens, so that an expert several chunks name is read
+ * once, and the releases. Every expert stays held until the pass is queued, so the caller makes
+ * sure that the cache has slots for all of them: what it evicts for a get is then the same as if
+ * each had been released at once, since a held expert was used later than any that is not.
+ * 150 tokens over 225 experts: 6.7 ms by chunks of 64 and batches of 8 experts with a wait for the
+ * stream each, 1.36 ms so. */
+static void moe_cached(float *out, const float *x, const Glm53fMoeW *w, const Glm53fCfg *c, int T, int with_shared,
+                       int kind)
+{
+    const int E = c->hidden, K = c->topk, NE = c->n_experts, nch = (T + G53_MOE_CHUNK - 1) / G53_MOE_CHUNK;
+    Glm53fExpertSrc *src = w->src;
+    const float *xd = stage_in(&g_xin, x, (size_t)T * E);
+    int *idx_d = (int *)buf_get(&g_idx, ((size_t)T * K + 1) * sizeof(int));
+    float *w_d = (float *)buf_get(&g_w, (size_t)T * K * sizeof(float));
+    int dt = 0;
+    const void *gate = resident_router(w->gate, (size_t)NE * E, &dt);
+    const float *bias = (const float *)resident(w->bias, (size_t)NE * sizeof(float));
+    int *flag_d = idx_d + (size_t)T * K;
+    if (g53h_memset(flag_d, 0, sizeof(int)) ||
+        g53h_router(idx_d, w_d, xd, T, gate, dt, bias, NE, E, K, c->norm_topk, c->routed_scale, flag_d))
+        g53_die("glm53f_router");
+    int *ids = (int *)pinned(&g_pin_ids, &g_pin_ids_n, ((size_t)T * K + 1) * sizeof(int));
+    if (g53h_d2h(ids, idx_d, ((size_t)T * K + 1) * sizeof(int))) g53_die("glm53f_moe routing");
+    if (ids[(size_t)T * K]) {
+        fprintf(stderr, "glm53f: FATAL, router selection (NaN scores) is below %d, above the limit of %d.\n", K, K);
+        abort();
+    }
+    read_switches();
+    const int prefetch = w->prefetch_n > 0 && src->hint != NULL && !g_prefill_off;
+    G53hExpert *table_d = (G53hExpert *)buf_get(&g_table, (size_t)(NE + 1) * sizeof(G53hExpert));
+    G53hExpert *table = (G53hExpert *)pinned(&g_pin_tab, &g_pin_tab_n, (size_t)(NE + 1) * sizeof(G53hExpert));
+    memset(table, 0, (size_t)(NE + 1) * sizeof(G53hExpert));
+    int *held = held_room((size_t)nch * NE), nh = 0, drops = 0;
+    unsigned char *dropped = NULL;                   /* [chunk][expert], once a get has failed */
+    for (int ch = 0; ch < nch; ch++) {
+        const int c0 = ch * G53_MOE_CHUNK, m = T - c0 < G53_MOE_CHUNK ? T - c0 : G53_MOE_CHUNK;
+        int uniq[1024], nu = 0;
+        unsigned char seen[1024];
+        memset(seen, 0, (size_t)NE);
+        for (int i = c0 * K; i < (c0 + m) * K; i++)
+            if (!seen[ids[i]]) { seen[ids[i]] = 1; uniq[nu++] = ids[i]; }
+        if (prefetch) {
+            src->hint(src, w->layer, uniq, nu);
+            int per = g_prefill_pred >= 0 ? g_prefill_pred : w->prefetch_n;
+            if (per > 2 * GLM53F_MAX_TOPK) per = 2 * GLM53F_MAX_TOPK;
+            if (per > NE) per = NE;
+            if (w->next_gate && per > 0 && (w->prefill_next || g_prefill_pred >= 0)) {
+                static int pred[64 * 2 * GLM53F_MAX_TOPK];
+                const int np = predict_next(pred, xd + (size_t)c0 * E, w, c, m, per);
+                src->hint(src, w->layer + 1, pred, np);
+            }
+        }
+        for (int g0 = 0; g0 < nu; g0 += G53_MOE_BATCH) {
+            const int gn = nu - g0 < G53_MOE_BATCH ? nu - g0 : G53_MOE_BATCH;
+            if (!prefetch && src->getmany) src->getmany(src, w->layer, uniq + g0, gn);
+            for (int u = g0; u < g0 + gn; u++) {
+                const int e = uniq[u];
+                Glm53fExpertQ q;
+                memset(&q, 0, sizeof q);
+                if (src->get(src, w->layer, e, &q) != 0) {
+                    glm53f_expert_drops++;
+                    fprintf(stderr, "EXPERT DROP: layer %d expert %d failed to load; this output is CORRUPT\n",
+                            w->layer, e);
+                    if (!dropped && !(dropped = (unsigned char *)calloc((size_t)nch, (size_t)NE))) {
+                        fprintf(stderr, "glm53f: FATAL, out of host memory\n");
+                        abort();
+                    }
+                    dropped[(size_t)ch * NE + e] = 1;
+                    drops++;
+                    continue;
+                }
+                check_expert_shape(&q, c, w->layer, e);
+                held[nh++] = e;
+                table[e].gate = view_mat_f8(&q.gate);
+                table[e].up = view_mat_f8(&q.up);
+                table[e].down = view_mat_f8(&q.down);
+            }
+        }
+    }
+    if (with_shared) {
+        table[NE].gate = dev_mat_resident_tiled_as(&w->sh_gate, "shared gate", kind == 2);
+        table[NE].up = dev_mat_resident_tiled_as(&w->sh_up, "shared up", kind == 2);
+        table[NE].down = dev_mat_resident_tiled_as(&w->sh_down, "shared down", kind == 2);
+    }
+    G53hMoeLayer L;
+    memset(&L, 0, sizeof L);
+    L.hidden = E; L.inter = c->moe_inter; L.n_experts = NE; L.topk = K; L.norm_topk = c->norm_topk;
+    L.routed_scale = c->routed_scale; L.swiglu_limit = c->swiglu_limit;
+    L.experts = table_d; L.shared = with_shared ? table_d + NE : NULL; L.block_c = 128; L.tiled = kind;
+    const int odev = g53h_is_device_ptr(out);
+    float *od = odev ? out : (float *)buf_get(&g_out, (size_t)T * E * sizeof(float));
+    /* one pass over all tokens; chunk by chunk when a get failed, whose zero is its own chunk's */
+    const int step = drops ? G53_MOE_CHUNK : T;
+    for (int c0 = 0; c0 < T; c0 += step) {
+        const int m = T - c0 < step ? T - c0 : step;
+        G53hExpert *t = table;
+        if (drops) {
+            t = (G53hExpert *)malloc((size_t)(NE + 1) * sizeof *t);
+            if (!t) { fprintf(stderr, "glm53f: FATAL, out of host memory\n"); abort(); }
+            memcpy(t, table, (size_t)(NE + 1) * sizeof *t);
+            for (int e = 0; e < NE; e++)
+                if (dropped[(size_t)(c0 / G53_MOE_CHUNK) * NE + e]) {
+                    memset(&t[e], 0, sizeof t[e]);
+                    t[e].gate.flags = G53H_MAT_DROPPED;
+                }
+        }
+        if (drops ? g53h_h2d(table_d, t, (size_t)(NE + 1) * sizeof *t)
+                  : g53h_h2d_async(table_d, t, (size_t)(NE + 1) * sizeof *t))
+            g53_die("glm53f_moe");
+        if (drops) free(t);
+        if (g53h_grouped_begin_layout(xd + (size_t)c0 * E, m, &L, idx_d + (size_t)c0 * K, kind) ||
+            g53h_grouped_batch(&L) || g53h_grouped_end(od + (size_t)c0 * E, w_d + (size_t)c0 * K))
+            g53_die("glm53f_moe");
+    }
+    free(dropped);
+    if (src->release)
+        for (int i = 0; i < nh; i++) src->release(src, w->layer, held[i]);
+    int *errs = errors_enqueue();
+    if (!odev) {
+        if (g53h_d2h(out, od, (size_t)T * E * sizeof(float))) g53_die("glm53f_moe");
+    } else if (g53h_sync()) {
+        g53_die("glm53f_moe");
+    }
+    errors_check(errs, w->layer, K);
+}
+
+/* How many of T tokens moe_cached takes at a time: 0 when it does not apply (another source, a cache
+ * whose slots are row-major or int4, a layer the grouped kernels do not take, too few slots). Slots are
+ * enough when, beside every expert that the pass may name, they have room for the reads that hints may
+ * land meanwhile (in flight, queued, and of the next layer where the pass predicts it): then a get
+ * always finds a slot that none of these holds, and all such slots were used before them. */
+static int cached_tokens(const Glm53fMoeW *w, const Glm53fCfg *c, int T, int with_shared, int *kind)
+{
+    *kind = g53h_cache_slot_kind(w->src);
+    if (T < 2 || (*kind != 1 && *kind != 2)) return 0;
+    if (with_shared) {
+        if (!shared_tileable(w)) return 0;
+        /* an HBM shared expert: the chunks of an MFMA-tiled cache take it as it is */
+        if (*kind == 2 && (g53h_is_device_ptr(w->sh_gate.w) || g53h_is_device_ptr(w->sh_up.w) ||
+                           g53h_is_device_ptr(w->sh_down.w)))
+            return 0;
+    }
+    const Glm53fCache *cache = (const Glm53fCache *)w->src;
+    G53hMoeLayer L;
+    memset(&L, 0, sizeof L);
+    L.hidden = c->hidden; L.inter = c->moe_inter; L.n_experts = c->n_experts; L.topk = c->topk;
+    L.swiglu_limit = c->swiglu_limit; L.block_c = 128;
+    int most = g53h_grouped_max_tokens(&L) / G53_MOE_CHUNK * G53_MOE_CHUNK;
+    if (most > T) most = T;
+    if (most < T && most < G53_MOE_CHUNK) return 0;
+    /* a pass's buffers must fit beside what the caller keeps in HBM; shorter passes where they do not,
+     * chunks (which need the least) in the end. Asked once per size: the buffers are kept. */
+    static size_t granted = 0;
+    L.shared = with_shared ? (const G53hExpert *)&L : NULL;
+    for (;; most = most / 2 / G53_MOE_CHUNK * G53_MOE_CHUNK) {
+        if (most < 2) return 0;
+        const size_t need = g53h_grouped_bytes(&L, most) + (size_t)2 * most * c->hidden * sizeof(float);
+        if (need <= granted) break;
+        size_t free_b = 0, total_b = 0;
+        if (g53h_mem_info(&free_b, &total_b)) return 0;
+        if (need + ((size_t)64 << 20) <= free_b) { granted = need; break; }
+        if (most <= G53_MOE_CHUNK) return 0;
+    }
+    const long named = (long)most * c->topk < c->n_experts ? (long)most * c->topk : c->n_experts;
+    read_switches();
+    const long next = w->next_gate && (w->prefill_next || g_prefill_pred >= 0) ? c->n_experts : 0;
+    return named + next + cache->n_io + cache->qlen <= cache->nslot ? most : 0;
+}
+
 static void moe_layer(float *out, const float *x, const Glm53fMoeW *w, const Glm53fCfg *c, int T, int with_shared)
 {
     if (T < 1) return;
@@ -1325,8 +1515,16 @@ static void moe_layer(float *out, const float *x, const Glm53fMoeW *w, const Glm
         fprintf(stderr, "glm53f: FATAL, routed experts is %d, above the limit of 1024.\n", c->n_experts);
         abort();
     }
+    int t0 = 0, kind = 0;
+    const int pass = cached_tokens(w, c, T, with_shared, &kind);
+    while (pass && T - t0 > 1) {                     /* a last chunk of one token decodes below */
+        int n = T - t0 < pass ? T - t0 : pass;
+        if (n % G53_MOE_CHUNK == 1) n--;
+        moe_cached(out + (size_t)t0 * c->hidden, x + (size_t)t0 * c->hidden, w, c, n, with_shared, kind);
+        t0 += n;
+    }
     /* chunks of 64 tokens, as src/core/glm53f_ops.c:1344-1362 */
-    for (int t0 = 0; t0 < T; t0 += G53_MOE_CHUNK) {
+    for (; t0 < T; t0 += G53_MOE_CHUNK) {
         const int n = (T - t0) < G53_MOE_CHUNK ? (T - t0) : G53_MOE_CHUNK;
         moe_chunk(out + (size_t)t0 * c->hidden, x + (size_t)t0 * c->hidden, w, c, n, with_shared);
     }

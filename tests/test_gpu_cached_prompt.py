@@ -1,0 +1,103 @@
+"""Several tokens through the HBM cache (glm53f_moe, T >= 2; src/core/glm53f_ops.c:1144-1362): a cache
+with slots for every expert a pass may name is multiplied in one grouped pass, a smaller one chunk by
+chunk and batch by batch. Both make the reference's calls, so the outputs are equal bit for bit, as are
+the counts of gets, with octet-tiled and MFMA-tiled slots, hints on and off, and a get that fails."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import glm53h
+import glm53h.synth as S
+import oracle_lib as O
+from glm53h import check
+from test_gpu_cache import make_cfg
+from test_gpu_grouped import within
+from test_gpu_parity import fmat, say
+
+pytestmark = pytest.mark.gpu
+NP = 6
+
+
+@pytest.fixture(scope="module")
+def L():
+    return glm53h.init(0)
+
+
+@pytest.fixture(scope="module")
+def layer():
+    sp = S.spec(2, NE=24, seed=5)
+    pool = [S.expert_host(sp, p) for p in range(NP)]
+    return sp, pool, S.router_host(sp), S.bias_host(sp), S.expert_host(sp, "shared")
+
+
+def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True):
+    sp, pool, W, B, sh = layer
+    cf = make_cfg(sp)
+    cf.n_layers = 1
+
+    def view(_st, _layer, e, out):
+        if e in fails:
+            return -1
+        q = out.contents
+        q.gate, q.up, q.down = [fmat(w, s, r, c, 128, 128) for (w, s), (r, c) in
+                                zip(pool[e % NP], [(sp.I, sp.E), (sp.I, sp.E), (sp.E, sp.I)])]
+        return 0
+
+    st = glm53h.G53hStore(glm53h.VIEW_FN(view), glm53h.DONE_FN(), None)
+    c, probe = glm53h.Glm53fCache(), glm53h.Glm53fCache()
+    check(L.g53h_cache_init_store(C.byref(probe), C.byref(st), C.byref(cf), 1 << 30, 0, 0), "cache")
+    budget = probe.slot_bytes * slots
+    L.glm53f_cache_free(C.byref(probe))
+    check(L.g53h_cache_init_store(C.byref(c), C.byref(st), C.byref(cf), budget, n_io, 0), "cache")
+    w = glm53h.Glm53fMoeW()
+    w.gate, w.bias, w.src, w.prefetch_n = W.ctypes.data, B.ctypes.data, C.pointer(c.src), prefetch_n
+    (gw, gs), (uw, us), (dw, ds) = sh
+    w.sh_gate, w.sh_up = fmat(gw, gs, sp.I, sp.E, 128, 128), fmat(uw, us, sp.I, sp.E, 128, 128)
+    w.sh_down = fmat(dw, ds, sp.E, sp.I, 128, 128)
+    drops = C.c_long.in_dll(L, "glm53f_expert_drops")
+    was, outs = drops.value, []
+    try:
+        for _ in range(2):                           # the second call finds what fits resident
+            out = np.zeros(x.shape, np.float32)
+            (L.glm53f_moe if shared else L.glm53f_moe_routed)(out.ctypes.data, x.ctypes.data, C.byref(w), C.byref(cf),
+                                                              x.shape[0], None)
+            outs.append(out)
+        check(L.glm53f_cache_sync(C.byref(c)), "sync")
+        gets, pins = c.hits + c.misses, sum(c.pins[i] for i in range(c.nslot))
+    finally:
+        L.glm53f_cache_free(C.byref(c))
+        L.glm53f_forget_host_weights()
+    assert pins == 0                                 # everything was released
+    lost, drops.value = drops.value - was, was
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    return outs[0], gets, lost
+
+
+@pytest.mark.parametrize("T,mfma,n_io,prefetch_n,shared", [
+    (2, False, 0, 0, True), (64, True, 0, 0, True), (65, False, 2, 6, True), (130, True, 2, 6, False),
+    (130, False, 0, 0, True)])
+def test_one_pass_is_the_chunks(L, layer, monkeypatch, T, mfma, n_io, prefetch_n, shared):
+    say("cached prompt", T, "mfma" if mfma else "octet", n_io, prefetch_n, shared)
+    if mfma:
+        monkeypatch.setenv("GLM53F_CACHE_MFMA", "1")
+    sp, pool, W, B, sh = layer
+    x = np.ascontiguousarray(S.x_host(sp, T, batch=4), np.float32)
+    want, gets, _ = run(L, layer, x, sp.NE - 5, shared=shared)              # chunks: too few slots
+    got, gets1, lost = run(L, layer, x, sp.NE + n_io + 64, n_io, prefetch_n, shared=shared)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    assert gets1 == gets and lost == 0
+    sel = [0, T - 1]
+    idx, _ = O.router(O.oracle(), x[sel], sp, W, B)
+    mats = {int(e): pool[int(e) % NP] for e in np.unique(idx)}
+    within(got[sel], O.moe(O.oracle(), x[sel], sp, W, B, mats, sh if shared else None)[0], f"T={T}")
+
+
+def test_failed_get_is_the_chunks_drop(L, layer):
+    say("cached prompt with an expert that cannot be read")
+    sp = layer[0]
+    x = np.ascontiguousarray(S.x_host(sp, 130, batch=6), np.float32)
+    want, _, lost = run(L, layer, x, sp.NE - 5, fails=(3, 17))
+    got, _, lost1 = run(L, layer, x, sp.NE + 64, fails=(3, 17))
+    assert lost1 == lost > 0
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
