@@ -28,6 +28,7 @@
 typedef float g53_f2 __attribute__((ext_vector_type(2)));
 
 #include "g53h_gemv.h"
+#include "g53h_rowdot.h"
 
 /* Work is spread over the whole GPU in grid-stride order: at step j, wave w takes chunk
  * j * nwaves + w, so the waves running together read one contiguous sweep of HBM (regularly
@@ -197,6 +198,110 @@ __global__ void k_combine(float *__restrict__ out, const float *__restrict__ con
     out[i] = o;
 }
 
+/* --------------------------------------------------------------- small layers ---- */
+/* Layers of a few hundred columns are a chain of launches and load latencies. Two kernels, every
+ * row of every (token, slot) at once: lane r of a wave takes row r of 64 and the wave one 128-column
+ * block of it, x (the same for every lane) comes by scalar loads, and the blocks' scaled sums meet in
+ * LDS, where one lane per row adds them in block order. Latency bounds both: 8 tokens of 256 x 128 (16
+ * experts, top-8 and shared) take 4.4 and 7.4 us; the block-lane kernels took 5 and 9.7, and the combine
+ * 4 and one launch more. */
+__device__ __forceinline__ double g53_sml_block(const G53hMat &m, int row, int b, const float *__restrict__ x)
+{
+    if (m.flags || m.bc != 128 || ((uintptr_t)m.w & 15)) {   /* anything else: the whole row with block 0 */
+        if (b) return 0.0;
+        if (!g53_rows_ok(m)) return __builtin_nan("");
+        return (m.flags & G53H_MAT_TILED) && !(m.flags & G53H_MAT_I4) ? g53_row_dot_tiled(m, row, x) : g53_row_dot(m, row, x);
+    }
+    const uint8_t *p = m.w + (size_t)row * m.cols + b * 128;
+    uint4 c[8];
+    g53_ld_blk(c, p);
+    const float sc = ((g53_gf *)m.s)[(size_t)(row / m.br) * m.scols + b];
+    float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const float *xb = x + b * 128;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const uint32_t d[4] = {c[k].x, c[k].y, c[k].z, c[k].w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int e = 16 * k + 4 * i, l = e & 7;
+            const g53_f2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)d[i], false);
+            const g53_f2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)d[i], true);
+            a[l + 0] = __builtin_fmaf(lo[0], xb[e + 0], a[l + 0]);
+            a[l + 1] = __builtin_fmaf(lo[1], xb[e + 1], a[l + 1]);
+            a[l + 2] = __builtin_fmaf(hi[0], xb[e + 2], a[l + 2]);
+            a[l + 3] = __builtin_fmaf(hi[1], xb[e + 3], a[l + 3]);
+        }
+    }
+    const double s = (((double)a[0] + a[4]) + ((double)a[2] + a[6])) +
+                     (((double)a[1] + a[5]) + ((double)a[3] + a[7]));
+    return s * (double)sc;
+}
+
+#define G53_SML_NB   8          /* most blocks of a gate or up row (hidden 1024)              */
+#define G53_SML_TASK 64         /* most (slot, block) pairs of the down kernel                */
+
+/* Gate and up of 64 intermediate rows of one (token, slot), and the SwiGLU. Grid (I / 64, T *
+ * nslots), a wave per block of both rows or half as many. */
+__global__ void __launch_bounds__(1024) k_sml_gateup(float *__restrict__ act, const float *__restrict__ x, int E, int I,
+                                                    int nslots, const G53hExpert *__restrict__ slots, float limit)
+{
+    __shared__ double pb[2 * G53_SML_NB][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ts = blockIdx.y, o = blockIdx.x * 64 + lane, nb = E / 128;
+    const G53hExpert *ex = slots + ts;
+    if (!ex->gate.w) return;                                 /* dropped: the down kernel adds zero */
+    for (int q = w; q < 2 * nb; q += (int)blockDim.x >> 6) {
+        const bool up = q >= nb;
+        pb[q][lane] = g53_sml_block(up ? ex->up : ex->gate, o, up ? q - nb : q, x + (size_t)(ts / nslots) * E);
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    double g = 0.0, u = 0.0;
+    for (int b = 0; b < nb; b++) {
+        g = g + pb[b][lane];
+        u = u + pb[nb + b][lane];
+    }
+    act[(size_t)ts * I + o] = g53_swiglu1((float)g, (float)u, limit);
+}
+
+/* Down of 64 rows of every slot of one token, combined in top-k order in double, then the shared
+ * expert in float (src/core/glm53f_ops.c:1329-1340). Grid (E / 64, T). */
+__global__ void __launch_bounds__(1024) k_sml_down(float *__restrict__ out, const float *__restrict__ act,
+                                                  const float *__restrict__ wts, int E, int I, int K, int nslots,
+                                                  const G53hExpert *__restrict__ slots)
+{
+    __shared__ double pb[G53_SML_TASK][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = blockIdx.y, d = blockIdx.x * 64 + lane, nb = I / 128;
+    for (int q = w; q < nslots * nb; q += (int)blockDim.x >> 6) {
+        const int s = q / nb, b = q % nb, ts = t * nslots + s;
+        const G53hExpert *ex = slots + ts;
+        pb[q][lane] = ex->gate.w ? g53_sml_block(ex->down, d, b, act + (size_t)ts * I) : 0.0;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    double acc = 0.0;
+    float sh = 0.0f;
+    for (int s = 0; s < nslots; s++) {
+        double c = 0.0;
+        for (int b = 0; b < nb; b++) c = c + pb[s * nb + b][lane];
+        if (s < K) acc = acc + (double)wts[(size_t)t * K + s] * (double)(float)c;
+        else sh = (float)c;
+    }
+    float v = (float)acc;
+    if (nslots > K) v = v + sh;
+    out[(size_t)t * E + d] = v;
+}
+
+/* Waves of a workgroup with n blocks to multiply: one each up to 16 while the launch has few
+ * workgroups, at most 8 in larger ones (64 tokens of a 1024 x 256 layer: 90 us with 16, 77 with 8, 77.5
+ * with 4; 300 tokens of 256 x 128: 51.7, 50.4, 52.9; 8 tokens of it: 17.1 with 16, 18.3 with 8). */
+static int g53_sml_waves(int n, long groups)
+{
+    const int most = groups > 2 * g53h_num_cus() ? 8 : 16;
+    return n < most ? n : most;
+}
+
 /* ------------------------------------------------------------------ dispatch ---- */
 /* Allow a kernel more than the default 64 KB of dynamic LDS (gfx950 has 160 KB per CU). */
 static int g53_lds_attr(const void *fn, size_t bytes)
@@ -233,6 +338,26 @@ static int g53_layer_body(float *out, const float *x, int T, const G53hMoeLayer 
     const int nslots = K + (L->shared ? 1 : 0);
     float *act = (float *)ws;
     hipStream_t st = g53h_stream();
+    /* small layers: every row of every slot at once, the combine in the down kernel. Against the
+     * block-lane kernels and k_combine (16 experts x 256 x 128, top-8 and shared: 1 token 23.6 -> 15.8 us
+     * for the call, 8 tokens 27.0 -> 17.2, 1000 tokens 188 -> 129; 64 experts x 1024 x 256: 25.1 -> 24.3,
+     * 64 tokens 107 -> 77) while a down workgroup has at most 20 blocks: at 64 its few workgroups are
+     * the longer chain (1 token of 1024 x 1024: 27.3 -> 40.7). Against the row-wave kernels as far as the
+     * LDS of the sums goes (40 experts x 384 x 384, 5 tokens: 143 -> 29; 300 x 640 x 128, 33: 585 -> 42). */
+    const int sml_task = nslots * (I / 128);
+    if (fused && L->block_c == 128 && E % 128 == 0 && I % 128 == 0 && E <= 128 * G53_SML_NB &&
+        sml_task <= (g53_fast_ok(L) ? 20 : G53_SML_TASK) && (long)T * (nslots + 1) <= 65535) {
+        const long wg_gu = (long)(I / 64) * T * nslots, wg_dn = (long)(E / 64) * T;
+        hipLaunchKernelGGL(k_sml_gateup, dim3(I / 64, T * nslots), dim3(64 * g53_sml_waves(2 * (E / 128), wg_gu)), 0,
+                           st, act, x, E, I, nslots, slots, L->swiglu_limit);
+        G53_LAUNCHED("k_sml_gateup");
+        g53h_prof_mark(G53_PROF_GATEUP);
+        hipLaunchKernelGGL(k_sml_down, dim3(E / 64, T), dim3(64 * g53_sml_waves(sml_task, wg_dn)), 0, st, out, act,
+                           wts, E, I, K, nslots, slots);
+        G53_LAUNCHED("k_sml_down");
+        g53h_prof_mark(G53_PROF_DOWN);
+        return 0;
+    }
     if (g53_fast_ok(L)) {
         const int nbe = E / 128, nbi = I / 128;
         const int rpw_e = 64 / nbe, rpw_i = 64 / nbi, cus = g53h_num_cus();

@@ -23,34 +23,6 @@
 typedef float g53_f2 __attribute__((ext_vector_type(2)));
 typedef uint32_t g53_u4 __attribute__((ext_vector_type(4)));
 
-__device__ float g53_row_dot_i4(const G53hMat &m, int o, const float *x)
-{
-    const uint8_t *row = m.w + (size_t)o * (m.cols / 2);
-    const float *srow = m.s + (size_t)o * m.scols;
-    double acc = 0.0;
-    for (int g = 0, j0 = 0; j0 < m.cols; g++, j0 += m.bc) {
-        const int j1 = (j0 + m.bc < m.cols) ? j0 + m.bc : m.cols;
-        const double p = g53_group_dot_i4(row, x, j0, j1) * (double)srow[g];
-        acc = acc + p;
-    }
-    return (float)acc;
-}
-
-__device__ float g53_row_dot(const G53hMat &m, int o, const float *x)
-{
-    if (m.flags & G53H_MAT_I4) return g53_row_dot_i4(m, o, x);
-    const uint8_t *row = m.w + (size_t)o * m.cols;
-    const float *srow = m.s + (size_t)(o / m.br) * m.scols;
-    double acc = 0.0;
-    for (int b = 0, j0 = 0; j0 < m.cols; b++, j0 += m.bc) {
-        const int j1 = (j0 + m.bc < m.cols) ? j0 + m.bc : m.cols;
-        const double bsum = g53_block_dot(row, x, j0, j1);
-        const double p = bsum * (double)srow[b];
-        acc = acc + p;
-    }
-    return (float)acc;
-}
-
 __global__ void k_mm_f8_generic(float *__restrict__ y, const float *__restrict__ x, int T, G53hMat m)
 {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -586,6 +558,51 @@ __global__ void __launch_bounds__(256) k_router_select_w(int *__restrict__ idx, 
                          0, experts, shared, slots);
 }
 
+/* Scores and selection of a small bf16 router in one launch, a workgroup per token. 16 lanes take an
+ * expert (lane l of them columns 8 l + 128 i .. + 7, its products added in order, then across the
+ * lanes: exact as in k_router_scores); then the first wave selects. E a multiple of 128. */
+template <int NV>
+__global__ void __launch_bounds__(1024) k_router_small(int *__restrict__ idx, float *__restrict__ w,
+                                                      const float *__restrict__ x, const uint16_t *__restrict__ gate,
+                                                      const float *__restrict__ bias, int NE, int E, int K,
+                                                      int norm_topk, float routed_scale, int *__restrict__ nan_flag,
+                                                      const G53hExpert *__restrict__ experts,
+                                                      const G53hExpert *__restrict__ shared,
+                                                      G53hExpert *__restrict__ slots)
+{
+    __shared__ float score[64 * NV], choice[64 * NV];
+    const int t = blockIdx.x, lane = threadIdx.x & 63, l = threadIdx.x & 15;
+    const float *xt = x + (size_t)t * E + 8 * l;
+    for (int e0 = 0; e0 < NE; e0 += (int)blockDim.x >> 4) {
+        const int e = e0 + (int)(threadIdx.x >> 4);
+        const uint16_t *row = gate + (size_t)(e < NE ? e : NE - 1) * E + 8 * l;
+        double acc = 0.0;
+#pragma unroll 4
+        for (int i = 0; i < E; i += 128) {
+            const uint4 q = *(const uint4 *)(row + i);
+            const float4 x0 = *(const float4 *)(xt + i), x1 = *(const float4 *)(xt + i + 4);
+            const uint32_t d[4] = {q.x, q.y, q.z, q.w};
+            const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                acc += (double)g53_bitsf(d[k] << 16) * (double)xv[2 * k];
+                acc += (double)g53_bitsf(d[k] & 0xffff0000u) * (double)xv[2 * k + 1];
+            }
+        }
+        for (int o = 8; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+        if (l == 0 && e < NE) {
+            const float s = g53_sigmoidf((float)acc);
+            score[e] = s;
+            choice[e] = s + bias[e];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    g53_select_token<NV>(0, lane, idx + (size_t)t * K, w + (size_t)t * K, score, choice, nullptr, 1, bias, 1, NE, K,
+                         norm_topk, routed_scale, nan_flag, 0, experts, shared,
+                         slots ? slots + (size_t)t * (K + (shared ? 1 : 0)) : nullptr);
+}
+
 /* slots[t][j] = experts[idx[t][j]] (j < K), slots[t][K] = *shared: the descriptor table of
  * the expert kernels, for callers that route elsewhere. */
 __global__ void k_resolve_slots(G53hExpert *__restrict__ slots, const G53hExpert *__restrict__ experts,
@@ -641,6 +658,17 @@ int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate
 {
     if (NE < 1 || NE > 1024) return g53h_fail("g53h_router: %d experts (max 1024)", NE);
     if (K < 1 || K > NE || K > GLM53F_MAX_TOPK_DEV) return g53h_fail("g53h_router: topk %d", K);
+    /* a router of at most 128 KB, a workgroup per token: one launch where there were two (us; 16 experts x
+     * 256: 1 token 6.6 -> 5.5, 8 tokens 8.4 -> 5.2, 512 9.4 -> 6.1; 64 x 1024: 8 tokens 9.0 -> 7.9, 512
+     * 14.1 -> 12.4). One token of a larger one is faster over all its experts' workgroups (64 x 1024: 6.6,
+     * here 7.4), many tokens of many experts over the matrix cores (256 x 256, 512 tokens: 10.8, here 15.6). */
+    if (gate_dt == 1 && E % 128 == 0 && (long)NE * E <= (T == 1 ? 8192 : 65536) && NE <= (T == 1 ? 32 : 320) &&
+        T <= 512 && (long)T * NE <= 65536 && (((uintptr_t)x | (uintptr_t)gate) & 15) == 0) {
+        hipLaunchKernelGGL(k_router_small<5>, dim3(T), dim3(NE > 32 ? 1024 : 512), 0, g53h_stream(), idx, w, x,
+                           (const uint16_t *)gate, bias, NE, E, K, norm_topk, routed_scale, nan_flag, experts, shared, slots);
+        G53_LAUNCHED("k_router_small");
+        return 0;
+    }
     float *score = scratch, *choice = scratch + (size_t)T * NE;
     const double *psum = nullptr;                            /* split logits, summed by the selection */
     int nsum = 1;

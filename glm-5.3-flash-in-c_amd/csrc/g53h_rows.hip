@@ -239,14 +239,6 @@ __device__ __forceinline__ double g53_pass(const G53hMat &m, const float *__rest
     return acc;
 }
 
-/* A usable octet-tiled matrix: 128-column blocks and whole row octets (the tiled format's
- * definition); anything else marked tiled is not read. */
-__device__ __forceinline__ bool g53_rows_ok(const G53hMat &m)
-{
-    if (!(m.flags & G53H_MAT_TILED) || (m.flags & G53H_MAT_I4)) return true;
-    return m.bc == 128 && m.cols == 128 * m.scols && (m.rows & 7) == 0 && ((uintptr_t)m.w & 15) == 0;
-}
-
 /* Sizes measured on MI355X (config-2 int4 decode): one wave per workgroup, 4 gate rows (and 4
  * up rows) or 8 down rows per wave keep the kernels at 3 waves per SIMD for the down rows and 2
  * for gate/up; 8-wave workgroups, or 8 gate / 16 down rows per wave, were slower. */

@@ -1,0 +1,130 @@
+"""Small layers (hidden up to 1024, every row of every slot at once) and small routers (scores and
+selection in one launch), at the edges of their rules and over every form of descriptor that they
+accept (replaces src/core/glm53f_ops.c:1144-1342). Bar: bit-exact with the oracle and with the
+row-wave kernels."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import glm53h
+import glm53h.synth as S
+import oracle_lib as O
+from glm53h import DevBuf, G53hExpert, G53hMat, check
+from test_gpu_grouped import oracle_out, run, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def L():
+    return glm53h.init(0)
+
+
+def bits(a):
+    return np.asarray(a, np.float32).view(np.uint32)
+
+
+@pytest.mark.parametrize("E,I,NE,K,T,kw", [
+    (128, 128, 3, 1, 1, {}), (256, 128, 16, 8, 8, {}), (384, 384, 33, 8, 5, {}), (1024, 256, 64, 9, 65, {}),
+    (1024, 128, 12, 4, 200, dict(shared=False)), (640, 896, 9, 8, 3, dict(norm_topk=0)),
+    (256, 128, 20, 3, 70, dict(br=64)), (896, 128, 40, 16, 2, dict(limit=0.0))])
+def test_small_layer_edges(L, E, I, NE, K, T, kw):
+    say("small layer", E, I, NE, K, T, kw)
+    sp = S.LayerSpec(E=E, I=I, NE=NE, K=K, router_sigma=0.02, **kw)
+    layer = S.DeviceLayer.build(sp)
+    x = S.x_host(sp, T, batch=3)
+    out, idx, w = run(layer, x, 0)
+    want, wi, ww = oracle_out(layer, x, idx)
+    assert np.array_equal(idx, wi) and np.array_equal(bits(w), bits(ww))
+    assert np.array_equal(bits(out), bits(want))
+
+
+@pytest.mark.parametrize("T", [1, 7])
+def test_small_layer_descriptors(L, T):
+    """Octet-tiled and unaligned descriptors among row-major ones: the same values, the same result.
+    Then an int4 one, as the row-wave kernels, which a layer without a block width takes."""
+    say("small layer descriptors", T)
+    sp = S.LayerSpec(E=384, I=256, NE=6, K=6, router_sigma=0.02)
+    layer = S.DeviceLayer.build(sp)
+    keep = []
+
+    def tiled(m):
+        b = DevBuf(m.rows * m.cols)
+        check(L.g53h_tile_f8(b.ptr, m.w, m.rows, m.cols), "tile")
+        keep.append(b)
+        return G53hMat(b.ptr, m.s, m.rows, m.cols, m.br, m.bc, m.scols, 2)
+
+    def moved(m):
+        b = DevBuf(m.rows * m.cols + 16)
+        check(L.g53h_d2d(b.ptr + 5, m.w, m.rows * m.cols), "d2d")
+        keep.append(b)
+        return G53hMat(b.ptr + 5, m.s, m.rows, m.cols, m.br, m.bc, m.scols, 0)
+
+    def int4(m):
+        q, st = DevBuf(m.rows * m.cols // 2), DevBuf(m.rows * (m.cols // 64) * 4)
+        check(L.g53h_i4_from_f8(q.ptr, st.ptr, C.byref(m)), "i4")
+        keep.extend((q, st))
+        return G53hMat(q.ptr, st.ptr, m.rows, m.cols, 1, 64, m.cols // 64, 4)
+
+    def put(forms):
+        for e, f in forms:
+            d = layer.experts[e]
+            layer.experts[e] = G53hExpert(f(d.gate), f(d.up), f(d.down))
+        layer.table.upload(np.frombuffer(bytes(layer.experts), np.uint8))
+
+    x = S.x_host(sp, T, batch=4)
+    want = run(layer, x, 0)
+    put(((1, tiled), (2, moved), (sp.NE, tiled)))
+    got = run(layer, x, 0)
+    assert np.array_equal(got[1], want[1]) and np.array_equal(bits(got[0]), bits(want[0]))
+    layer = S.DeviceLayer.build(sp)
+    put(((3, int4),))
+    got = run(layer, x, 0)
+    layer.layer.block_c = 0
+    want = run(layer, x, 0)
+    assert np.array_equal(got[1], want[1]) and np.array_equal(bits(got[0]), bits(want[0]))
+
+
+@pytest.mark.parametrize("T,NE,E,K,shift", [
+    (1, 1, 128, 1, 0), (1, 32, 256, 8, 0), (2, 65, 384, 8, 0), (3, 16, 4096, 16, 0), (512, 128, 512, 4, 0),
+    (200, 320, 128, 10, 0), (512, 129, 128, 3, 0), (5, 33, 256, 8, 1)])
+def test_small_router(L, T, NE, E, K, shift):
+    """Either side of the rule; shift moves x off 16-byte alignment."""
+    say("small router", T, NE, E, K, shift)
+    sp = S.LayerSpec(E=E, I=128, NE=NE, K=K, router_sigma=0.05)
+    rf, bias = S.router_host(sp), S.bias_host(sp)
+    x = S.x_host(sp, T, batch=5)
+    xd = DevBuf(x.nbytes + 16)
+    check(L.g53h_h2d(xd.ptr + 4 * shift, x.ctypes.data, x.nbytes), "h2d")
+    g, b = DevBuf.from_array((rf.view(np.uint32) >> 16).astype(np.uint16)), DevBuf.from_array(bias)
+    idx, w, flag = DevBuf(T * K * 4), DevBuf(T * K * 4), DevBuf(4)
+    flag.zero()
+    check(L.g53h_router(idx.ptr, w.ptr, xd.ptr + 4 * shift, T, g.ptr, 1, b.ptr, NE, E, K, sp.norm_topk,
+                        C.c_float(sp.routed_scale), flag.ptr), "router")
+    wi, ww = O.router(O.oracle(), x, sp, rf, bias)
+    assert np.array_equal(idx.download(np.int32).reshape(T, K), wi)
+    assert np.array_equal(bits(w.download(np.float32).reshape(T, K)), bits(ww))
+    assert flag.download(np.int32)[0] == 0
+
+
+def test_small_router_nan(L):
+    """A token whose scores are NaN raises the flag, the others are as without it."""
+    say("small router NaN")
+    sp = S.LayerSpec(E=256, I=128, NE=16, K=4, router_sigma=0.05)
+    layer = S.DeviceLayer.build(sp)
+    x = S.x_host(sp, 3, batch=6)
+    xn = x.copy()
+    xn[1, 17] = np.nan
+    res = []
+    for v in (x, xn):
+        xd = DevBuf.from_array(v)
+        idx, w, flag = DevBuf(3 * 4 * 4), DevBuf(3 * 4 * 4), DevBuf(4)
+        flag.zero()
+        check(L.g53h_router(idx.ptr, w.ptr, xd.ptr, 3, layer.router.ptr, 1, layer.bias.ptr, 16, 256, 4, 1,
+                            C.c_float(2.5), flag.ptr), "router")
+        res.append((idx.download(np.int32).reshape(3, 4), bits(w.download(np.float32).reshape(3, 4)),
+                    flag.download(np.int32)[0]))
+    assert res[0][2] == 0 and res[1][2] != 0
+    for t in (0, 2):
+        assert np.array_equal(res[0][0][t], res[1][0][t]) and np.array_equal(res[0][1][t], res[1][1][t])
