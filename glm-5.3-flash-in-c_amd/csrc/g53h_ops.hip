@@ -276,15 +276,12 @@ __global__ void __launch_bounds__(64) k_router_scores(float *__restrict__ score,
  * expert's weight) and B[l / 16][l % 16] (a token's x); step s uses column 64w + 16(l/16) + s
  * of the chunk, so a lane reads 32 consecutive router bytes per chunk. Result: lane l, register
  * r holds C[4r + l/16][l % 16]. x chunks are staged in LDS. bf16 router rows, E a multiple of
- * 256. */
+ * 256. The double instruction's rate bounds it from some hundred tokens on, below that the wait for
+ * a chunk, so the next chunk's operands are requested before this one is multiplied (288 experts x
+ * 4096 with the selection, us: 150 tokens 26.3 -> 20.2, 384: 47.3 -> 32.7, 2048: 109.8 -> 103.5, where a
+ * 32 x 32 tile per wave over eight column ranges had been faster than the unpipelined loop). */
 typedef double g53_v4d __attribute__((ext_vector_type(4)));
-#ifndef G53_RM32_S
-#define G53_RM32_S    8         /* column ranges of the large-batch router               */
-#endif
-static_assert(G53_RM32_S >= 1 && G53_RM32_S <= 8, "the selection sums at most 8 column ranges");
-#ifndef G53_RM32_MINT
-#define G53_RM32_MINT 512       /* tokens from which the large-batch router is used       */
-#endif
+typedef float g53_v4f __attribute__((ext_vector_type(4)));
 #define G53_RM_XST 260                                  /* LDS floats per token row       */
 __global__ void __launch_bounds__(256) k_router_mfma(float *__restrict__ score, float *__restrict__ choice,
                                                      const float *__restrict__ x, int T,
@@ -302,20 +299,29 @@ __global__ void __launch_bounds__(256) k_router_mfma(float *__restrict__ score, 
     const float *xl = xs + i * G53_RM_XST + w * 64 + g * 16;
     g53_v4d acc = {0.0, 0.0, 0.0, 0.0};
     const int kb = blockIdx.z * klen;                        /* this workgroup's column range */
+    /* the next chunk's operands come to registers while this one's are multiplied */
+    g53_u4 wv[2];
+    g53_v4f xv[4];
+    const int xc = (threadIdx.x & 63) * 4;
+    auto load = [&](int k0) {
+        wv[0] = *(const g53_u4 *)(wrow + k0);
+        wv[1] = *(const g53_u4 *)(wrow + k0 + 8);
+#pragma unroll
+        for (int q = 0; q < 4; q++) xv[q] = *(const g53_v4f *)(x + (size_t)min(t0 + w + 4 * q, T - 1) * E + k0 + xc);
+    };
+    load(kb);
     for (int k0 = kb; k0 < kb + klen; k0 += 256) {
-        const uint4 wv0 = *(const uint4 *)(wrow + k0), wv1 = *(const uint4 *)(wrow + k0 + 8);
+        const g53_u4 d[2] = {wv[0], wv[1]};
         __syncthreads();
-        for (int q = threadIdx.x; q < 16 * 64; q += 256) {
-            const int tk = q >> 6, c = (q & 63) * 4;
-            const int tt = t0 + tk < T ? t0 + tk : T - 1;
-            *(float4 *)(xs + tk * G53_RM_XST + c) = *(const float4 *)(x + (size_t)tt * E + k0 + c);
-        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) *(g53_v4f *)(xs + (w + 4 * q) * G53_RM_XST + xc) = xv[q];
         __syncthreads();
-        const uint32_t d[8] = {wv0.x, wv0.y, wv0.z, wv0.w, wv1.x, wv1.y, wv1.z, wv1.w};
+        if (k0 + 256 < kb + klen) load(k0 + 256);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)g53_bitsf(d[k] << 16), (double)xl[2 * k], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)g53_bitsf(d[k] & 0xffff0000u), (double)xl[2 * k + 1],
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)g53_bitsf(d[k >> 2][k & 3] << 16), (double)xl[2 * k], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)g53_bitsf(d[k >> 2][k & 3] & 0xffff0000u), (double)xl[2 * k + 1],
                                                        acc, 0, 0, 0);
         }
     }
@@ -335,77 +341,6 @@ __global__ void __launch_bounds__(256) k_router_mfma(float *__restrict__ score, 
             if (choice) choice[(size_t)t * NE + e] = s + bias[e];
         }
     }
-}
-
-/* The same partial sums for large batches: one wave per workgroup owns a 32 x 32 tile
- * (experts e0 = 32 * bx .., tokens t0 = 32 * by ..) over the column range bz * klen .. + klen, as 2 x 2 blocks of v_mfma_f64_16x16x4f64, so that each operand
- * converted to double feeds two instructions. Both operands come straight from memory (L2):
- * per 64-column chunk, lane l reads 16 consecutive columns 16 (l / 16) .. of its two expert rows
- * (l % 16, 16 + l % 16) and of its two token rows; step s of the chunk uses column
- * 16 (l / 16) + s, the same K assignment for A and B. The next chunk's loads are issued before
- * the current chunk's arithmetic. The sums go to psum[bz][t][e]; the selection kernel adds
- * the ranges in column order. bf16 router rows, klen a multiple of 64. */
-__global__ void __launch_bounds__(64) k_router_mfma32(const float *__restrict__ x, int T,
-                                                      const uint16_t *__restrict__ gate, int NE, int E,
-                                                      int klen, int S, double *__restrict__ psum)
-{
-    /* workgroups are dealt round-robin over the 8 XCDs: XCD x takes the contiguous tile range
-     * x * per .., expert tiles fastest, so the expert tiles that read one token tile's
-     * activations share one L2 */
-    const int ET = (NE + 31) >> 5, TT = (T + 31) >> 5, n = ET * TT * S, per = (int)(gridDim.x >> 3);
-    const int j = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-    if (j >= n) return;
-    const int bx = j % ET, by = (j / ET) % TT, bz = j / (ET * TT);
-    const int lane = threadIdx.x, i = lane & 15, g = lane >> 4;
-    const int e0 = bx * 32, t0 = by * 32;
-    const int kb = bz * klen;
-    const uint16_t *wr[2];
-    const float *xr[2];
-#pragma unroll
-    for (int f = 0; f < 2; f++) {
-        const int e = min(e0 + 16 * f + i, NE - 1), t = min(t0 + 16 * f + i, T - 1);   /* past the end: discarded */
-        wr[f] = gate + (size_t)e * E + kb + 16 * g;
-        xr[f] = x + (size_t)t * E + kb + 16 * g;
-    }
-    g53_v4d acc[2][2] = {};
-    uint4 wa[2][2], wb[2][2];
-    float4 xa[2][4], xb[2][4];
-#define G53_RM32_LD(W, X, c) do { _Pragma("unroll") for (int f = 0; f < 2; f++) {                               \
-        W[f][0] = *(const uint4 *)(wr[f] + (c)); W[f][1] = *(const uint4 *)(wr[f] + (c) + 8);                   \
-        _Pragma("unroll") for (int q = 0; q < 4; q++) X[f][q] = *(const float4 *)(xr[f] + (c) + 4 * q); } } while (0)
-#define G53_RM32_MUL(W, X) do {                                                                                 \
-        _Pragma("unroll") for (int s = 0; s < 16; s++) {                                                        \
-            double a[2], b[2];                                                                                  \
-            _Pragma("unroll") for (int f = 0; f < 2; f++) {                                                     \
-                const uint32_t wd = ((const uint32_t *)&W[f][s >> 3])[(s & 7) >> 1];                            \
-                a[f] = (double)g53_bitsf((s & 1) ? (wd & 0xffff0000u) : (wd << 16));                            \
-                b[f] = (double)((const float *)&X[f][s >> 2])[s & 3];                                           \
-            }                                                                                                   \
-            _Pragma("unroll") for (int f = 0; f < 2; f++)                                                       \
-                _Pragma("unroll") for (int h = 0; h < 2; h++)                                                   \
-                    acc[f][h] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[f], b[h], acc[f][h], 0, 0, 0);           \
-        } } while (0)
-    G53_RM32_LD(wa, xa, 0);
-    for (int c = 0; c < klen; c += 128) {
-        if (c + 64 < klen) G53_RM32_LD(wb, xb, c + 64);
-        G53_RM32_MUL(wa, xa);
-        if (c + 64 >= klen) break;
-        if (c + 128 < klen) G53_RM32_LD(wa, xa, c + 128);
-        G53_RM32_MUL(wb, xb);
-    }
-#undef G53_RM32_LD
-#undef G53_RM32_MUL
-#pragma unroll
-    for (int f = 0; f < 2; f++)
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int t = t0 + 16 * h + i;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int e = e0 + 16 * f + 4 * r + g;
-                if (t < T && e < NE) psum[((size_t)bz * T + t) * NE + e] = acc[f][h][r];
-            }
-        }
 }
 
 extern "C" __device__ unsigned __ockl_wfred_max_u32(unsigned);
@@ -659,12 +594,13 @@ int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate
     if (NE < 1 || NE > 1024) return g53h_fail("g53h_router: %d experts (max 1024)", NE);
     if (K < 1 || K > NE || K > GLM53F_MAX_TOPK_DEV) return g53h_fail("g53h_router: topk %d", K);
     /* a router of at most 128 KB, a workgroup per token: one launch where there were two (us; 16 experts x
-     * 256: 1 token 6.6 -> 5.5, 8 tokens 8.4 -> 5.2, 512 9.4 -> 6.1; 64 x 1024: 8 tokens 9.0 -> 7.9, 512
-     * 14.1 -> 12.4). One token of a larger one is faster over all its experts' workgroups (64 x 1024: 6.6,
-     * here 7.4), many tokens of many experts over the matrix cores (256 x 256, 512 tokens: 10.8, here 15.6). */
-    if (gate_dt == 1 && E % 128 == 0 && (long)NE * E <= (T == 1 ? 8192 : 65536) && NE <= (T == 1 ? 32 : 320) &&
-        T <= 512 && (long)T * NE <= 65536 && (((uintptr_t)x | (uintptr_t)gate) & 15) == 0) {
-        hipLaunchKernelGGL(k_router_small<5>, dim3(T), dim3(NE > 32 ? 1024 : 512), 0, g53h_stream(), idx, w, x,
+     * 256: 1 token 6.6 -> 5.5, 8 tokens 8.3 -> 5.2; 64 x 1024: 8 tokens 9.0 -> 7.9; 128 x 512, 256 tokens:
+     * 9.8 -> 8.8). One token of a larger one is faster over all its experts' workgroups (64 x 1024: 6.6,
+     * here 7.4), more than 256 tokens and more experts over the matrix cores (64 x 1024, 320 tokens: 10.2,
+     * here 11.7; 256 x 256, 64 tokens: 9.3, here 9.9). */
+    if (gate_dt == 1 && E % 128 == 0 && (long)NE * E <= (T == 1 ? 8192 : 65536) && NE <= (T == 1 ? 32 : 128) &&
+        T <= 256 && (((uintptr_t)x | (uintptr_t)gate) & 15) == 0) {
+        hipLaunchKernelGGL(k_router_small<2>, dim3(T), dim3(NE > 32 ? 1024 : 512), 0, g53h_stream(), idx, w, x,
                            (const uint16_t *)gate, bias, NE, E, K, norm_topk, routed_scale, nan_flag, experts, shared, slots);
         G53_LAUNCHED("k_router_small");
         return 0;
@@ -672,22 +608,14 @@ int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate
     float *score = scratch, *choice = scratch + (size_t)T * NE;
     const double *psum = nullptr;                            /* split logits, summed by the selection */
     int nsum = 1;
-    if (T >= G53_RM32_MINT && gate_dt == 1 && E % (64 * G53_RM32_S) == 0) {   /* large batches */
-        const int S = G53_RM32_S;
-        double *part = (double *)g53_router_part((size_t)S * T * NE * sizeof(double));
-        if (!part) return -1;
-        const unsigned n32 = (unsigned)(((NE + 31) / 32) * ((T + 31) / 32) * S + 7) / 8 * 8;
-        hipLaunchKernelGGL(k_router_mfma32, dim3(n32), dim3(64), 0, g53h_stream(), x, T, (const uint16_t *)gate, NE,
-                           E, E / S, S, part);
-        G53_LAUNCHED("k_router_mfma32");
-        psum = part;
-        nsum = S;
-    } else if (T >= 2 && gate_dt == 1 && E % 256 == 0) {    /* batches: the matrix-core form */
-        /* few tiles (small T): the columns are split over up to 8 workgroups per tile so that
-         * enough loads are in flight; the partial sums are added in column order after */
+    if (T >= 2 && gate_dt == 1 && E % 256 == 0) {           /* batches: the matrix-core form */
+        /* few tiles (small T): the columns are split over up to 8 workgroups per tile while that gives
+         * at most 10 workgroups per CU; the partial sums are added in column order after (288 experts x
+         * 4096, both launches: 150 tokens 22.7 us at 640 workgroups, 20.2 at 2560; 256: 28.4, 24.4;
+         * 5120 is no faster) */
         const int tiles = ((NE + 15) / 16) * ((T + 15) / 16);
         int S = 1;
-        while (S < 8 && tiles * S * 2 <= 640 && (E / (S * 2)) % 256 == 0) S *= 2;
+        while (S < 8 && tiles * S * 2 <= 2560 && (E / (S * 2)) % 256 == 0) S *= 2;
         double *part = nullptr;
         if (S > 1) {
             part = (double *)g53_router_part((size_t)S * T * NE * sizeof(double));
