@@ -8,11 +8,11 @@
  * does the same with every expert's weights read from HBM once per call:
  *
  *   1. router             the exact router kernels of g53h_ops.hip (top-k bit-exact).
- *   2. k_grp_plan         counting sort of the (token, slot) pairs by expert, stable in token
+ *   2. k_grp_prep         counting sort of the (token, slot) pairs by expert, stable in token
  *                         order; segment e holds expert e's tokens, segment NE the shared
  *                         expert's (every token); a tile is <= 64 consecutive positions of one
  *                         segment.
- *   3. k_grp_xq           each token's activations as NPX E4M3 planes with a power-of-two
+ *   3. (same launch)      each token's activations as NPX E4M3 planes with a power-of-two
  *                         token scale: x = 2^-k (q0 + q1 / 16 + q2 / 256 ...). For bf16-valued
  *                         inputs two planes hold x exactly (8 significant bits = 4 + 4).
  *   4. k_grp_gemm<true>   per (tile, 128-row block): gate and up rows of the expert times the
@@ -85,11 +85,10 @@ __device__ __forceinline__ int g53_grp_seg_cost(int n)
  * chunk c of 64 tokens and expert e, mask[c][e] has bit t%64 set when token t chose e; the
  * position of (t, e) is off[e] + (tokens of e in earlier chunks) + popcount(mask bits below
  * t). One workgroup of 1024 threads; dynamic LDS sized by the host. */
-__global__ void __launch_bounds__(1024)
-k_grp_plan(const int *__restrict__ idx, int T, int K, int NE, int has_sh, int *__restrict__ tok_of,
-           int *__restrict__ pos_of, int4 *__restrict__ tiles, int *__restrict__ meta, int mb_gu, int mb_dn)
+__device__ void g53_grp_plan(uint64_t *pl_lds, const int *__restrict__ idx, int T, int K, int NE, int has_sh,
+                             int *__restrict__ tok_of, int *__restrict__ pos_of, int4 *__restrict__ tiles,
+                             int *__restrict__ meta, int mb_gu, int mb_dn)
 {
-    extern __shared__ __attribute__((aligned(16))) uint64_t pl_lds[];
     const int nch = (T + 63) >> 6, nm = nch * NE, tid = threadIdx.x;
     uint64_t *mask = pl_lds;
     int *pre = (int *)(mask + nm);                 /* [nch][NE]                              */
@@ -233,42 +232,61 @@ __device__ __forceinline__ void g53_grp_st4(uint8_t *row, int c0, uint32_t q, in
     for (int k = 0; k < 4; k++) blk[g53_grp_tpos((c0 + k) & 127)] = (uint8_t)(q >> (8 * k));
 }
 
-/* Token t's row of x as NPX planes xq[p][t][E] with scale 2^k, k = 8 - exponent(absmax), so
- * every |x| * 2^k < 256; 2^-k goes to every position of the token (pos_of[t][ns], -1: none).
- * Grid T, 256 threads, E a multiple of 16. */
+typedef float g53_v4f __attribute__((ext_vector_type(4)));
+
+/* A token's row of x as NPX planes xq[p][t][E] with scale 2^k, k = 8 - exponent(absmax), so
+ * every |x| * 2^k < 256; xinv[t] = 2^-k. 256 threads a token, tg of them this one; the workgroup's
+ * four tokens share its barrier. E at most 4096, a multiple of 16: the row stays in registers. */
 template <int NP>
-__global__ void __launch_bounds__(256)
-k_grp_xq(const float *__restrict__ x, int E, int T, uint8_t *__restrict__ xq, float *__restrict__ xinvp,
-         const int *__restrict__ pos_of, int ps, int ns, int tiled)
+__device__ __forceinline__ void g53_grp_xq(float *red, const float *__restrict__ x, int E, int T, int t, int tg,
+                                           uint8_t *__restrict__ xq, float *__restrict__ xinv, int tiled)
 {
-    __shared__ float red[4];
-    const int t = blockIdx.x, tid = threadIdx.x;
-    const float *xr = x + (size_t)t * E;
+    const float *xr = x + (size_t)min(t, T - 1) * E;
+    g53_v4f v[4];
     float m = 0.0f;
-    for (int i = tid * 4; i < E; i += 1024) {
-        const float4 v = *(const float4 *)(xr + i);
-        m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int i = tg * 4 + q * 1024;
+        v[q] = i < E ? *(const g53_v4f *)(xr + i) : g53_v4f{0.f, 0.f, 0.f, 0.f};
+        m = fmaxf(m, fmaxf(fmaxf(fabsf(v[q][0]), fabsf(v[q][1])), fmaxf(fabsf(v[q][2]), fabsf(v[q][3]))));
     }
     for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    if ((tid & 63) == 0) red[tid >> 6] = m;
+    float *rt = red + (threadIdx.x >> 8) * 4;
+    if ((tg & 63) == 0) rt[tg >> 6] = m;
     __syncthreads();
-    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    if (t >= T) return;
+    m = fmaxf(fmaxf(rt[0], rt[1]), fmaxf(rt[2], rt[3]));
     int ex = 0;
     if (m > 0.0f && m <= 3.0e38f) (void)frexpf(m, &ex);          /* m < 2^ex */
     const int k = 8 - ex;
     const float sc = ldexpf(1.0f, k);
-    for (int j = tid; j < ns; j += 256) {
-        const int p = pos_of[t * ps + j];
-        if (p >= 0) xinvp[p] = ldexpf(1.0f, -k);
-    }
-    for (int i = tid * 4; i < E; i += 1024) {
-        const float4 v = *(const float4 *)(xr + i);
-        const float s[4] = {v.x * sc, v.y * sc, v.z * sc, v.w * sc};
-        uint32_t q[NP];
-        g53_split_planes<NP>(s, q);
+    if (tg == 0) xinv[t] = ldexpf(1.0f, -k);
 #pragma unroll
-        for (int p = 0; p < NP; p++) g53_grp_st4(xq + ((size_t)p * T + t) * E, i, q[p], tiled);
+    for (int q = 0; q < 4; q++) {
+        const int i = tg * 4 + q * 1024;
+        if (i >= E) break;
+        const float s[4] = {v[q][0] * sc, v[q][1] * sc, v[q][2] * sc, v[q][3] * sc};
+        uint32_t pq[NP];
+        g53_split_planes<NP>(s, pq);
+#pragma unroll
+        for (int p = 0; p < NP; p++) g53_grp_st4(xq + ((size_t)p * T + t) * E, i, pq[p], tiled);
     }
+}
+
+/* Workgroup 0 plans, the others take four tokens' planes each, in one launch: neither needs the
+ * other's result. Both are short chains of latencies (with 5 tokens 6.0 and 4.7 us, with 2048 25 and
+ * 17.5, one after the other before). Grid 1 + ceil(T / 4). */
+__global__ void __launch_bounds__(1024)
+k_grp_prep(const int *__restrict__ idx, int T, int K, int NE, int has_sh, int *__restrict__ tok_of,
+           int *__restrict__ pos_of, int4 *__restrict__ tiles, int *__restrict__ meta, int mb_gu, int mb_dn,
+           const float *__restrict__ x, int E, uint8_t *__restrict__ xq, float *__restrict__ xinv, int tiled)
+{
+    extern __shared__ __attribute__((aligned(16))) uint64_t pl_lds[];
+    if (blockIdx.x == 0)
+        g53_grp_plan(pl_lds, idx, T, K, NE, has_sh, tok_of, pos_of, tiles, meta, mb_gu, mb_dn);
+    else
+        g53_grp_xq<G53_GRP_NPX>((float *)pl_lds, x, E, T, ((int)blockIdx.x - 1) * 4 + (int)(threadIdx.x >> 8),
+                                threadIdx.x & 255, xq, xinv, tiled);
 }
 
 /* ------------------------------------------------------------- grouped GEMM ---- */
@@ -367,7 +385,7 @@ struct G53GrpArgs {
     int *meta_w;
     const int *tok_of;             /* position -> token (readable 8 past the last)       */
     const uint8_t *xq;             /* [NPX][T][E]                                        */
-    const float *xinvp;            /* [P]: the token scale of each position              */
+    const float *xinv;             /* [T]: the tokens' scales                            */
     uint8_t *aq;                   /* [NPA][P][I]                                        */
     float *contrib;                /* [P][E]                                             */
     int T, P, E, I, NE;
@@ -459,8 +477,9 @@ template <bool GATEUP>
 __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
 {
     __shared__ __attribute__((aligned(1024))) uint8_t ring[G53_GRP_NS * G53_GRP_SLOT];
-    __shared__ float xil[2][64];                             /* the items' token scales ...      */
-    __shared__ float scl[2][64];                             /* ... and block scales: two rows   */
+    /* the items' token scales (of position 32 h + 8 v + q at [2 v + h][8 q]) and block scales: two rows */
+    __shared__ float xil[2][8][64];
+    __shared__ float scl[2][64];
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i = lane & 31, g = lane >> 5;
     const int K = GATEUP ? a.E : a.I, MB = GATEUP ? a.I / 128 : a.E / 256, nkb = K / 128;
@@ -468,7 +487,7 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
     const int bhi = g53_sld(a.meta + bnd + 1);
     int loc = g53_sld(a.meta + bnd) + (int)(blockIdx.x >> 3);
     const uint32_t lring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)ring;
-    const uint32_t lxil = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float *)&xil[0][0];
+    const uint32_t lxil = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float *)&xil[0][0][0];
     const uint32_t lscl = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float *)&scl[0][0];
 
     /* this lane's part of a load instruction: row lane / 8 of eight, piece lane % 8 of LDS */
@@ -482,7 +501,7 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
                                          : a.tiled ? lr * 128 + c * 16 : lr * K + c * 16));
     }
     const uint32_t vox = (uint32_t)((lp ^ ((4 * (w & 1) + (lane >> 4)) & 7)) * 16);
-    const int kst = a.tiled ? 1024 : 128;
+    const int kst = a.tiled ? 1024 : 128, ksh = __builtin_ctz(K);    /* K: a power of two */
     const size_t xps = GATEUP ? (size_t)a.T * a.E : (size_t)a.P * a.I;
     auto item_at = [&](int n) {
         G53GrpItem it;
@@ -576,8 +595,11 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
         r.pa += kst;
         r.px += 128;
     };
-    auto scales = [&](const G53GrpItem &it, int par) {       /* the item's scales, by waves 0 and 1 */
-        if (GATEUP && w == 0) g53_dma4(a.xinvp + it.tl.y + min(lane, it.tl.z - 1), lxil + par * 256);
+    auto scales = [&](const G53GrpItem &it, const Bound &r, int par) {   /* the item's scales */
+        if (GATEUP && w < 4) {                               /* of the tokens whose first plane the wave requests */
+            g53_dma4(a.xinv + (r.vx[0] >> ksh), lxil + par * 2048 + w * 512);
+            g53_dma4(a.xinv + (r.vx[1] >> ksh), lxil + par * 2048 + w * 512 + 256);
+        }
         if (w == 1) {                                        /* rows: gate and up, or the item's two of down */
             const G53hExpert *ex = it.ex;
             const float *r0, *r1;
@@ -622,7 +644,7 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
     G53GrpOps ops[2];
     int par = 0;
     uint32_t so = 0;                                         /* slot of the step being multiplied */
-    scales(cur, 0);
+    scales(cur, bd, 0);
     request(bd, 0);
     request(bd, G53_GRP_SLOT);
     request(bd, 2 * G53_GRP_SLOT);
@@ -651,7 +673,7 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
             g53_grp_bar();
             if (kb == nkb - 3) {
                 bd = nb;
-                if (nx.tl.z) scales(nx, par ^ 1);
+                if (nx.tl.z) scales(nx, bd, par ^ 1);
             }
             const uint32_t rs = so;
             so = so == 2 * G53_GRP_SLOT ? 0u : so + G53_GRP_SLOT;
@@ -679,7 +701,7 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
              * whose operands have been read, in their final byte order (the tiled order within the 128-column
              * block when the pass is tiled), and leave as whole 16-byte pieces */
             uint8_t *ao = ring + so;
-            const float xi = xil[par][j];
+            const float xi = xil[par][2 * (i >> 3) + half][8 * (i & 7)];
             g53_grp_bar();                                   /* every wave is done with the slot */
 #pragma unroll
             for (int f = 0; f < 2; f++) {
@@ -846,19 +868,16 @@ static int g53_grp_plan_pass(const float *x, int tc, const G53hMoeLayer *L, cons
     int *pos_of = (int *)p;   p += al256((size_t)tc * (K + 1) * 4);
     int4 *tiles = (int4 *)p;  p += al256((size_t)maxtiles * 16);
     uint8_t *xq = (uint8_t *)p; p += al256((size_t)G53_GRP_NPX * tc * E);
-    float *xinvp = (float *)p; p += al256((size_t)P * 4);
+    float *xinv = (float *)p; p += al256((size_t)tc * 4);
     uint8_t *aq = (uint8_t *)p; p += al256((size_t)G53_GRP_NPA * P * I);
     float *contrib = (float *)p;
     const int nch = (tc + 63) / 64;
-    const size_t lds = (size_t)nch * NE * 12 + (size_t)(NE + 2) * 12;
+    const size_t lds = (size_t)nch * NE * 12 + (size_t)(NE + 2) * 12 + 64;   /* planes: 16 words */
     if (lds > 160 * 1024) return g53h_fail("g53h_moe_grouped: %zu bytes of planner LDS", lds);
-    if (lds > 65536) G53_TRY(hipFuncSetAttribute((const void *)k_grp_plan, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k_grp_plan, dim3(1), dim3(1024), lds, st, idx, tc, K, NE, hs, tok_of, pos_of, tiles, meta,
-                       I / 128, E / 256);
-    G53_LAUNCHED("k_grp_plan");
-    hipLaunchKernelGGL(k_grp_xq<G53_GRP_NPX>, dim3(tc), dim3(256), 0, st, x, E, tc, xq, xinvp, pos_of, K + 1, K + hs,
-                       layout == 1);
-    G53_LAUNCHED("k_grp_xq");
+    if (lds > 65536) G53_TRY(hipFuncSetAttribute((const void *)k_grp_prep, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_grp_prep, dim3(1 + (tc + 3) / 4), dim3(1024), lds, st, idx, tc, K, NE, hs, tok_of, pos_of, tiles,
+                       meta, I / 128, E / 256, x, E, xq, xinv, layout == 1);
+    G53_LAUNCHED("k_grp_prep");
     g53h_prof_mark(G53_PROF_GROUPED);
     float bound = L->swiglu_limit > 0.28f ? L->swiglu_limit : 0.28f;
     bound *= L->swiglu_limit;
@@ -866,7 +885,7 @@ static int g53_grp_plan_pass(const float *x, int tc, const G53hMoeLayer *L, cons
     (void)frexpf(bound, &ex);                      /* |act| <= bound < 2^ex */
     G53GrpArgs &a = g_pass.a;
     a.experts = L->experts; a.shared = L->shared; a.tiles = tiles; a.meta = meta; a.meta_w = meta;
-    a.tok_of = tok_of; a.xq = xq; a.xinvp = xinvp; a.aq = aq; a.contrib = contrib;
+    a.tok_of = tok_of; a.xq = xq; a.xinv = xinv; a.aq = aq; a.contrib = contrib;
     a.T = tc; a.P = P; a.E = E; a.I = I; a.NE = NE;
     a.limit = L->swiglu_limit; a.aq_scale = ldexpf(1.0f, 8 - ex); a.aq_inv = ldexpf(1.0f, ex - 8);
     a.partial = 0;
@@ -922,7 +941,7 @@ static size_t g53_grp_ws(const G53hMoeLayer *L, int tc)
     const size_t P = (size_t)tc * K + (size_t)hs * tc;
     const int maxtiles = (tc * K + G53_GRP_NT - 1) / G53_GRP_NT + NE + hs * ((tc + G53_GRP_NT - 1) / G53_GRP_NT);
     return al256(P * 4) + al256((size_t)tc * (K + 1) * 4) + al256((size_t)maxtiles * 16) +
-           al256((size_t)G53_GRP_NPX * tc * E) + al256(P * 4) + al256((size_t)G53_GRP_NPA * P * I) +
+           al256((size_t)G53_GRP_NPX * tc * E) + al256((size_t)tc * 4) + al256((size_t)G53_GRP_NPA * P * I) +
            al256(P * E * 4);
 }
 
