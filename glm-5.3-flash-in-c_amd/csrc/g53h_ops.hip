@@ -613,13 +613,17 @@ int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate
          * at most 10 workgroups per CU; the partial sums are added in column order after (288 experts x
          * 4096, both launches: 150 tokens 22.7 us at 640 workgroups, 20.2 at 2560; 256: 28.4, 24.4;
          * 5120 is no faster) */
-        const int tiles = ((NE + 15) / 16) * ((T + 15) / 16);
+        const int et = (NE + 15) / 16, tiles = et * ((T + 15) / 16);
         int S = 1;
         while (S < 8 && tiles * S * 2 <= 2560 && (E / (S * 2)) % 256 == 0) S *= 2;
         double *part = nullptr;
-        if (S > 1) {
-            part = (double *)g53_router_part((size_t)S * T * NE * sizeof(double));
+        if (E % 512 == 0) {
+            /* what any batch of at most T tokens may need (S T <= 16 * 2560 / et): a smaller batch after a
+             * larger one, a captured one for instance, allocates nothing */
+            const size_t rows = min((size_t)8 * T, (size_t)40960 / et);
+            part = (double *)g53_router_part(rows * NE * sizeof(double));
             if (!part) return -1;
+            if (S == 1) part = nullptr;
         }
         hipLaunchKernelGGL(k_router_mfma, dim3((NE + 15) / 16, (T + 15) / 16, S), dim3(256), 0, g53h_stream(),
                            score, choice, x, T, (const uint16_t *)gate, bias, NE, E, E / S, part);
