@@ -484,6 +484,18 @@ extern "C" int g53h_cache_slot_kind(const Glm53fExpertSrc *src)
     return !m ? 0 : m->tiled ? (m->mt ? 2 : 1) : m->i4t ? 3 : m->i4m ? 4 : 0;
 }
 
+extern "C" void g53h_cache_held(const Glm53fExpertSrc *src, int layer, int *own, int *others)
+{
+    *own = *others = 0;
+    if (!g53h_cache_is(src)) return;
+    const Glm53fCache *c = (const Glm53fCache *)src;
+    Impl *m = impl_of(c);
+    if (!m) return;
+    std::lock_guard<std::mutex> g(m->mu);
+    for (int s = 0; s < c->nslot; s++)
+        if (m->lru.pins[s] > 0) (m->lru.key_of[s] / c->n_experts == layer ? *own : *others) += 1;
+}
+
 extern "C" int g53h_cache_layer_table(Glm53fExpertSrc *src, int layer, const G53hExpert **table_d,
                                       const G53hExpert **table_h)
 {

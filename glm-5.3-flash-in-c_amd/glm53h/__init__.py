@@ -261,6 +261,7 @@ _SIGS = {
     "glm53f_cache_report": (None, [C.POINTER(Glm53fCache), C.c_char_p]),
     "glm53f_cache_sync": (C.c_int, [C.POINTER(Glm53fCache)]),
     "g53h_cache_is": (C.c_int, [C.POINTER(Glm53fExpertSrc)]),
+    "g53h_cache_held": (None, [C.POINTER(Glm53fExpertSrc), C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "g53h_cache_slot_kind": (C.c_int, [C.POINTER(Glm53fExpertSrc)]),
     "g53h_set_speculate": (C.c_int, [C.c_int]),
     "g53h_speculate_counts": (None, [C.c_void_p]),

@@ -1342,9 +1342,11 @@ static int *held_room(size_t n)
  * once, and the releases. Every expert stays held until the pass is queued, so the caller makes
  * sure that the cache has slots for all of them: what it evicts for a get is then the same as if
  * each had been released at once, since a held expert was used later than any that is not.
- * 150 tokens over 225 experts: 6.7 ms by chunks of 64 and batches of 8 experts with a wait for the
- * stream each, 1.36 ms so. */
-static void moe_cached(float *out, const float *x, const Glm53fMoeW *w, const Glm53fCfg *c, int T, int with_shared,
+ * 150 tokens over 225 experts: 8.4 ms by chunks of 64 and batches of 8 experts with a wait for the
+ * stream each, 1.31 ms so. Returns 0, or -1 with every expert released and nothing written when a get
+ * fails (an expert that cannot be read, or a slot that another holder took meanwhile): the chunks,
+ * which hold at most top-k at a time, then find a slot or report the drop. */
+static int moe_cached(float *out, const float *x, const Glm53fMoeW *w, const Glm53fCfg *c, int T, int with_shared,
                        int kind)
 {
     const int E = c->hidden, K = c->topk, NE = c->n_experts, nch = (T + G53_MOE_CHUNK - 1) / G53_MOE_CHUNK;
@@ -1370,8 +1372,7 @@ static void moe_cached(float *out, const float *x, const Glm53fMoeW *w, const Gl
     G53hExpert *table_d = (G53hExpert *)buf_get(&g_table, (size_t)(NE + 1) * sizeof(G53hExpert));
     G53hExpert *table = (G53hExpert *)pinned(&g_pin_tab, &g_pin_tab_n, (size_t)(NE + 1) * sizeof(G53hExpert));
     memset(table, 0, (size_t)(NE + 1) * sizeof(G53hExpert));
-    int *held = held_room((size_t)nch * NE), nh = 0, drops = 0;
-    unsigned char *dropped = NULL;                   /* [chunk][expert], once a get has failed */
+    int *held = held_room((size_t)nch * NE), nh = 0;
     for (int ch = 0; ch < nch; ch++) {
         const int c0 = ch * G53_MOE_CHUNK, m = T - c0 < G53_MOE_CHUNK ? T - c0 : G53_MOE_CHUNK;
         int uniq[1024], nu = 0;
@@ -1398,16 +1399,8 @@ static void moe_cached(float *out, const float *x, const Glm53fMoeW *w, const Gl
                 Glm53fExpertQ q;
                 memset(&q, 0, sizeof q);
                 if (src->get(src, w->layer, e, &q) != 0) {
-                    glm53f_expert_drops++;
-                    fprintf(stderr, "EXPERT DROP: layer %d expert %d failed to load; this output is CORRUPT\n",
-                            w->layer, e);
-                    if (!dropped && !(dropped = (unsigned char *)calloc((size_t)nch, (size_t)NE))) {
-                        fprintf(stderr, "glm53f: FATAL, out of host memory\n");
-                        abort();
-                    }
-                    dropped[(size_t)ch * NE + e] = 1;
-                    drops++;
-                    continue;
+                    for (int i = 0; i < nh; i++) src->release(src, w->layer, held[i]);
+                    return -1;
                 }
                 check_expert_shape(&q, c, w->layer, e);
                 held[nh++] = e;
@@ -1429,32 +1422,10 @@ static void moe_cached(float *out, const float *x, const Glm53fMoeW *w, const Gl
     L.experts = table_d; L.shared = with_shared ? table_d + NE : NULL; L.block_c = 128; L.tiled = kind;
     const int odev = g53h_is_device_ptr(out);
     float *od = odev ? out : (float *)buf_get(&g_out, (size_t)T * E * sizeof(float));
-    /* one pass over all tokens; chunk by chunk when a get failed, whose zero is its own chunk's */
-    const int step = drops ? G53_MOE_CHUNK : T;
-    for (int c0 = 0; c0 < T; c0 += step) {
-        const int m = T - c0 < step ? T - c0 : step;
-        G53hExpert *t = table;
-        if (drops) {
-            t = (G53hExpert *)malloc((size_t)(NE + 1) * sizeof *t);
-            if (!t) { fprintf(stderr, "glm53f: FATAL, out of host memory\n"); abort(); }
-            memcpy(t, table, (size_t)(NE + 1) * sizeof *t);
-            for (int e = 0; e < NE; e++)
-                if (dropped[(size_t)(c0 / G53_MOE_CHUNK) * NE + e]) {
-                    memset(&t[e], 0, sizeof t[e]);
-                    t[e].gate.flags = G53H_MAT_DROPPED;
-                }
-        }
-        if (drops ? g53h_h2d(table_d, t, (size_t)(NE + 1) * sizeof *t)
-                  : g53h_h2d_async(table_d, t, (size_t)(NE + 1) * sizeof *t))
-            g53_die("glm53f_moe");
-        if (drops) free(t);
-        if (g53h_grouped_begin_layout(xd + (size_t)c0 * E, m, &L, idx_d + (size_t)c0 * K, kind) ||
-            g53h_grouped_batch(&L) || g53h_grouped_end(od + (size_t)c0 * E, w_d + (size_t)c0 * K))
-            g53_die("glm53f_moe");
-    }
-    free(dropped);
-    if (src->release)
-        for (int i = 0; i < nh; i++) src->release(src, w->layer, held[i]);
+    if (g53h_h2d_async(table_d, table, (size_t)(NE + 1) * sizeof(G53hExpert)) ||
+        g53h_grouped_begin_layout(xd, T, &L, idx_d, kind) || g53h_grouped_batch(&L) || g53h_grouped_end(od, w_d))
+        g53_die("glm53f_moe");
+    for (int i = 0; i < nh; i++) src->release(src, w->layer, held[i]);
     int *errs = errors_enqueue();
     if (!odev) {
         if (g53h_d2h(out, od, (size_t)T * E * sizeof(float))) g53_die("glm53f_moe");
@@ -1462,13 +1433,15 @@ static void moe_cached(float *out, const float *x, const Glm53fMoeW *w, const Gl
         g53_die("glm53f_moe");
     }
     errors_check(errs, w->layer, K);
+    return 0;
 }
 
 /* How many of T tokens moe_cached takes at a time: 0 when it does not apply (another source, a cache
  * whose slots are row-major or int4, a layer the grouped kernels do not take, too few slots). Slots are
- * enough when, beside every expert that the pass may name, they have room for the reads that hints may
- * land meanwhile (in flight, queued, and of the next layer where the pass predicts it): then a get
- * always finds a slot that none of these holds, and all such slots were used before them. */
+ * enough when, beside every expert that the pass may name and what the caller holds already, they have
+ * room for the reads that hints may land meanwhile (in flight, queued, and of the next layer where the
+ * pass predicts it): then a get always finds a slot that none of these holds, and all such slots were
+ * used before them. */
 static int cached_tokens(const Glm53fMoeW *w, const Glm53fCfg *c, int T, int with_shared, int *kind)
 {
     *kind = g53h_cache_slot_kind(w->src);
@@ -1501,10 +1474,12 @@ static int cached_tokens(const Glm53fMoeW *w, const Glm53fCfg *c, int T, int wit
         if (need + ((size_t)64 << 20) <= free_b) { granted = need; break; }
         if (most <= G53_MOE_CHUNK) return 0;
     }
-    const long named = (long)most * c->topk < c->n_experts ? (long)most * c->topk : c->n_experts;
+    int own = 0, others = 0;
+    g53h_cache_held(w->src, w->layer, &own, &others);
+    const long named = (long)most * c->topk + own < c->n_experts ? (long)most * c->topk + own : c->n_experts;
     read_switches();
     const long next = w->next_gate && (w->prefill_next || g_prefill_pred >= 0) ? c->n_experts : 0;
-    return named + next + cache->n_io + cache->qlen <= cache->nslot ? most : 0;
+    return named + others + next + cache->n_io + cache->qlen <= cache->nslot ? most : 0;
 }
 
 static void moe_layer(float *out, const float *x, const Glm53fMoeW *w, const Glm53fCfg *c, int T, int with_shared)
@@ -1520,7 +1495,7 @@ static void moe_layer(float *out, const float *x, const Glm53fMoeW *w, const Glm
     while (pass && T - t0 > 1) {                     /* a last chunk of one token decodes below */
         int n = T - t0 < pass ? T - t0 : pass;
         if (n % G53_MOE_CHUNK == 1) n--;
-        moe_cached(out + (size_t)t0 * c->hidden, x + (size_t)t0 * c->hidden, w, c, n, with_shared, kind);
+        if (moe_cached(out + (size_t)t0 * c->hidden, x + (size_t)t0 * c->hidden, w, c, n, with_shared, kind)) break;
         t0 += n;
     }
     /* chunks of 64 tokens, as src/core/glm53f_ops.c:1344-1362 */

@@ -167,6 +167,9 @@ int  g53h_cache_layer_table(Glm53fExpertSrc *src, int layer, const G53hExpert **
  * MFMA-tiled FP8 (GLM53F_CACHE_MFMA set at its init), 3 int4-tiled (int4 mode 2), 4 int4
  * MFMA-tiled (int4 mode 3), 0 otherwise (row-major FP8 or int4, or src not a cache). */
 int  g53h_cache_slot_kind(const Glm53fExpertSrc *src);
+/* Slots held between get() and release() now (no counterpart in the reference): *own of them hold
+ * experts of layer, *others the rest; both 0 when src is not a cache. */
+void g53h_cache_held(const Glm53fExpertSrc *src, int layer, int *own, int *others);
 /* The drop-in's speculative cached decode (no counterpart in the reference): with a cache of
  * octet-tiled slots, glm53f_moe at T = 1 runs the one-launch decode over the layer's table
  * before the reference's hint/get/release calls, which it then makes in the reference's order,

@@ -31,7 +31,7 @@ def layer():
     return sp, pool, S.router_host(sp), S.bias_host(sp), S.expert_host(sp, "shared")
 
 
-def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True):
+def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True, hold=None):
     sp, pool, W, B, sh = layer
     cf = make_cfg(sp)
     cf.n_layers = 1
@@ -57,12 +57,15 @@ def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True):
     w.sh_down = fmat(dw, ds, sp.E, sp.I, 128, 128)
     drops = C.c_long.in_dll(L, "glm53f_expert_drops")
     was, outs = drops.value, []
+    done = hold(c) if hold else None
     try:
         for _ in range(2):                           # the second call finds what fits resident
             out = np.zeros(x.shape, np.float32)
             (L.glm53f_moe if shared else L.glm53f_moe_routed)(out.ctypes.data, x.ctypes.data, C.byref(w), C.byref(cf),
                                                               x.shape[0], None)
             outs.append(out)
+        if done:
+            done()
         check(L.glm53f_cache_sync(C.byref(c)), "sync")
         gets, pins = c.hits + c.misses, sum(c.pins[i] for i in range(c.nslot))
     finally:
@@ -100,4 +103,43 @@ def test_failed_get_is_the_chunks_drop(L, layer):
     want, _, lost = run(L, layer, x, sp.NE - 5, fails=(3, 17))
     got, _, lost1 = run(L, layer, x, sp.NE + 64, fails=(3, 17))
     assert lost1 == lost > 0
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+def holds(layer, expert, at_hint=False):
+    """A caller's own hold on an expert, as include/glm53f.h allows: taken before the calls, or by another
+    user of the cache while a call runs (in its first hint)."""
+    def hold(c):
+        ref, taken = C.pointer(c.src), []
+
+        def take(*_):
+            if not taken:
+                taken.append(c.src.get(ref, layer, expert, C.byref(glm53h.Glm53fExpertQ())))
+        hint = glm53h.HINT_FN(take)
+        if at_hint:
+            c.src.hint = hint
+        else:
+            take()
+
+        def release(_hint=hint):
+            assert taken == [0]
+            c.src.release(ref, layer, expert)
+        return release
+    return hold
+
+
+@pytest.mark.parametrize("mfma", [False, True])
+@pytest.mark.parametrize("where", ["other layer", "this layer", "during the call"])
+def test_held_slots_leave_room(L, layer, monkeypatch, where, mfma):
+    """As many slots as experts, one of them held by the caller: no expert is dropped and the output is that
+    of the chunks."""
+    say("cached prompt, a slot held", where, "mfma" if mfma else "octet")
+    if mfma:
+        monkeypatch.setenv("GLM53F_CACHE_MFMA", "1")
+    sp = layer[0]
+    x = np.ascontiguousarray(S.x_host(sp, 64, batch=7), np.float32)
+    want, _, _ = run(L, layer, x, sp.NE - 5)
+    hold = holds(0 if where == "this layer" else 1, 3, at_hint=where == "during the call")
+    got, _, lost = run(L, layer, x, sp.NE, prefetch_n=6, hold=hold)
+    assert lost == 0
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
