@@ -989,12 +989,12 @@ static int g53_grp_tcmax(int NE)
     return tcmax > G53_GRP_MAXT ? G53_GRP_MAXT : tcmax;
 }
 
-/* HBM that routing and one planning pass of T tokens may take (the workspace grows by a quarter more
- * than asked, the router's partial sums are at most 8 doubles a score). */
-extern "C" size_t g53h_grouped_bytes(const G53hMoeLayer *L, int T)
+/* HBM that g53h_router and one planning pass of T tokens would allocate now (each uses the workspace in
+ * turn): 0 when the library holds enough already. */
+extern "C" size_t g53h_grouped_growth(const G53hMoeLayer *L, int T)
 {
-    const size_t scores = (size_t)T * L->n_experts;
-    return g53_grp_ws(L, T) / 4 * 5 + scores * (2 * sizeof(float) + 8 * sizeof(double)) + (2u << 20);
+    const size_t ws = g53_grp_ws(L, T), scores = (size_t)2 * T * L->n_experts * sizeof(float);
+    return g53h_workspace_growth(ws > scores ? ws : scores) + g53h_router_growth(T, L->router_dt, L->n_experts, L->hidden);
 }
 
 extern "C" int g53h_grouped_max_tokens(const G53hMoeLayer *L)

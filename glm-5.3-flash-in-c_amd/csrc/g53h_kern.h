@@ -2,6 +2,8 @@
 #ifndef G53H_KERN_H
 #define G53H_KERN_H
 
+#include <stddef.h>
+
 #include "g53h.h"
 
 #define GLM53F_MAX_TOPK_DEV 64
@@ -17,6 +19,8 @@ int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate
                      const float *bias, int NE, int E, int K, int norm_topk, float routed_scale,
                      int *nan_flag, float *scratch, const G53hExpert *experts, const G53hExpert *shared,
                      G53hExpert *slots);
+/* HBM that the router would allocate for partial sums before a batch of T tokens. */
+size_t g53h_router_growth(int T, int gate_dt, int NE, int E);
 int g53h_decode_fused(float *out, const float *x, const G53hMoeLayer *L, int *idx_out, float *w_out);
 int g53h_decode_tiled(float *out, const float *x, const G53hMoeLayer *L, int *idx_out, float *w_out,
                       const int *idx_in, const float *w_in);

@@ -586,6 +586,32 @@ static void *g53_router_part(size_t bytes)
     return g_router_part;
 }
 
+/* A router of at most 128 KB, a workgroup per token: one launch where there were two (us; 16 experts x
+ * 256: 1 token 6.6 -> 5.5, 8 tokens 8.3 -> 5.2; 64 x 1024: 8 tokens 9.0 -> 7.9; 128 x 512, 256 tokens:
+ * 9.8 -> 8.8). One token of a larger one is faster over all its experts' workgroups (64 x 1024: 6.6,
+ * here 7.4), more than 256 tokens and more experts over the matrix cores (64 x 1024, 320 tokens: 10.2,
+ * here 11.7; 256 x 256, 64 tokens: 9.3, here 9.9). */
+static bool g53_router_small(int T, int gate_dt, int NE, int E)
+{
+    return gate_dt == 1 && E % 128 == 0 && (long)NE * E <= (T == 1 ? 8192 : 65536) &&
+           NE <= (T == 1 ? 32 : 128) && T <= 256;
+}
+
+/* Partial sums that a batch of at most T tokens may need, over the column ranges of g53h_router_into
+ * (S T <= 16 * 2560 / et): a smaller batch after a larger one, a captured one for instance, allocates
+ * nothing. */
+static size_t g53_router_part_need(int T, int NE, int E)
+{
+    const size_t et = (NE + 15) / 16, rows = min((size_t)8 * T, (size_t)40960 / et);
+    return E % 512 == 0 ? rows * NE * sizeof(double) : 0;
+}
+size_t g53h_router_growth(int T, int gate_dt, int NE, int E)
+{
+    if (T < 2 || gate_dt != 1 || g53_router_small(T, gate_dt, NE, E)) return 0;
+    const size_t n = g53_router_part_need(T, NE, E);
+    return n <= g_router_part_bytes ? 0 : n;
+}
+
 int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate, int gate_dt,
                      const float *bias, int NE, int E, int K, int norm_topk, float routed_scale,
                      int *nan_flag, float *scratch, const G53hExpert *experts, const G53hExpert *shared,
@@ -593,13 +619,7 @@ int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate
 {
     if (NE < 1 || NE > 1024) return g53h_fail("g53h_router: %d experts (max 1024)", NE);
     if (K < 1 || K > NE || K > GLM53F_MAX_TOPK_DEV) return g53h_fail("g53h_router: topk %d", K);
-    /* a router of at most 128 KB, a workgroup per token: one launch where there were two (us; 16 experts x
-     * 256: 1 token 6.6 -> 5.5, 8 tokens 8.3 -> 5.2; 64 x 1024: 8 tokens 9.0 -> 7.9; 128 x 512, 256 tokens:
-     * 9.8 -> 8.8). One token of a larger one is faster over all its experts' workgroups (64 x 1024: 6.6,
-     * here 7.4), more than 256 tokens and more experts over the matrix cores (64 x 1024, 320 tokens: 10.2,
-     * here 11.7; 256 x 256, 64 tokens: 9.3, here 9.9). */
-    if (gate_dt == 1 && E % 128 == 0 && (long)NE * E <= (T == 1 ? 8192 : 65536) && NE <= (T == 1 ? 32 : 128) &&
-        T <= 256 && (((uintptr_t)x | (uintptr_t)gate) & 15) == 0) {
+    if (g53_router_small(T, gate_dt, NE, E) && (((uintptr_t)x | (uintptr_t)gate) & 15) == 0) {
         hipLaunchKernelGGL(k_router_small<2>, dim3(T), dim3(NE > 32 ? 1024 : 512), 0, g53h_stream(), idx, w, x,
                            (const uint16_t *)gate, bias, NE, E, K, norm_topk, routed_scale, nan_flag, experts, shared, slots);
         G53_LAUNCHED("k_router_small");
@@ -613,15 +633,12 @@ int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate
          * at most 10 workgroups per CU; the partial sums are added in column order after (288 experts x
          * 4096, both launches: 150 tokens 22.7 us at 640 workgroups, 20.2 at 2560; 256: 28.4, 24.4;
          * 5120 is no faster) */
-        const int et = (NE + 15) / 16, tiles = et * ((T + 15) / 16);
+        const int tiles = ((NE + 15) / 16) * ((T + 15) / 16);
         int S = 1;
         while (S < 8 && tiles * S * 2 <= 2560 && (E / (S * 2)) % 256 == 0) S *= 2;
         double *part = nullptr;
         if (E % 512 == 0) {
-            /* what any batch of at most T tokens may need (S T <= 16 * 2560 / et): a smaller batch after a
-             * larger one, a captured one for instance, allocates nothing */
-            const size_t rows = min((size_t)8 * T, (size_t)40960 / et);
-            part = (double *)g53_router_part(rows * NE * sizeof(double));
+            part = (double *)g53_router_part(g53_router_part_need(T, NE, E));
             if (!part) return -1;
             if (S == 1) part = nullptr;
         }

@@ -41,6 +41,7 @@ int g53h_i4_from_f8_on(uint8_t *q_d, float *steps_d, const G53hMat *src, hipStre
  * Regions are carved from it per call; nothing in it survives between calls except the
  * counters region, which kernels leave zeroed. */
 void       *g53h_workspace(size_t bytes);
+size_t      g53h_workspace_growth(size_t bytes);    /* what g53h_workspace(bytes) would allocate: 0 when held */
 /* A zero-initialised region of 4096 ints that kernels use as arrival counters and flags and
  * always restore to zero before they exit. */
 int        *g53h_counters(void);

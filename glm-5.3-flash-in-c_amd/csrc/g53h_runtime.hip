@@ -347,16 +347,31 @@ extern "C" float g53h_elapsed_ms(void)
     return ms;
 }
 
+static size_t g_mem_cap = 0;
+extern "C" size_t g53h_set_mem_free(size_t bytes)
+{
+    const size_t old = g_mem_cap;
+    g_mem_cap = bytes;
+    return old;
+}
+
 extern "C" int g53h_mem_info(size_t *free_b, size_t *total_b)
 {
     if (g53h_ready()) return -1;
     G53_TRY(hipMemGetInfo(free_b, total_b));
+    if (g_mem_cap && *free_b > g_mem_cap) *free_b = g_mem_cap;
     return 0;
+}
+
+size_t g53h_workspace_growth(size_t bytes)
+{
+    return bytes <= g_ws_bytes ? 0 : (bytes + (bytes >> 2) + 0xfffff) & ~(size_t)0xfffff;
 }
 
 void *g53h_workspace(size_t bytes)
 {
-    if (bytes <= g_ws_bytes) return g_ws;
+    const size_t want = g53h_workspace_growth(bytes);
+    if (!want) return g_ws;
     if (g_ws) {
         if (g53h_check(hipStreamSynchronize(g_stream), "hipStreamSynchronize", __FILE__, __LINE__))
             return nullptr;
@@ -364,8 +379,6 @@ void *g53h_workspace(size_t bytes)
         g_ws = nullptr;
         g_ws_bytes = 0;
     }
-    size_t want = bytes + (bytes >> 2);
-    want = (want + 0xfffff) & ~(size_t)0xfffff;
     if (g53h_check(hipMalloc(&g_ws, want), "hipMalloc(workspace)", __FILE__, __LINE__)) return nullptr;
     g_ws_bytes = want;
     return g_ws;

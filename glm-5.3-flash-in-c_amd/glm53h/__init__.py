@@ -199,6 +199,7 @@ _SIGS = {
     "g53h_route_topn_batch": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_int,
                                         C.c_void_p, C.c_int, C.c_int]),
     "g53h_vote": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int]),
+    "g53h_set_mem_free": (C.c_size_t, [C.c_size_t]),
     "g53h_set_spin_limit": (C.c_int, [C.c_int]),
     "g53h_inject_errors": (C.c_int, [C.c_int, C.c_int]),
     "g53h_errors_peek_async": (C.c_int, [C.c_void_p]),

@@ -257,6 +257,8 @@ static void *buf_get(G53Buf *b, size_t n)
     return b->d;
 }
 
+static size_t buf_growth(const G53Buf *b, size_t n) { return n <= b->n ? 0 : n; }
+
 static G53Buf g_xin, g_out, g_idx, g_w, g_flag, g_table, g_pred, g_tmp, g_contrib;
 
 /* The same in the octet-tiled layout (for the tiled decode kernel), resident as well: uploaded
@@ -1318,7 +1320,7 @@ static void moe_chunk(float *out, const float *x, const Glm53fMoeW *w, const Glm
 }
 
 /* ------------------------------------------------ several tokens through the HBM cache ---- */
-size_t g53h_grouped_bytes(const G53hMoeLayer *L, int T);
+size_t g53h_grouped_growth(const G53hMoeLayer *L, int T);
 int g53h_grouped_begin_layout(const float *x_d, int T, const G53hMoeLayer *L, const int *idx_d, int layout);
 
 static void *g_pin_ids;
@@ -1442,7 +1444,8 @@ static int moe_cached(float *out, const float *x, const Glm53fMoeW *w, const Glm
  * room for the reads that hints may land meanwhile (in flight, queued, and of the next layer where the
  * pass predicts it): then a get always finds a slot that none of these holds, and all such slots were
  * used before them. */
-static int cached_tokens(const Glm53fMoeW *w, const Glm53fCfg *c, int T, int with_shared, int *kind)
+static int cached_tokens(const float *out, const float *x, const Glm53fMoeW *w, const Glm53fCfg *c, int T,
+                         int with_shared, int *kind)
 {
     *kind = g53h_cache_slot_kind(w->src);
     if (T < 2 || (*kind != 1 && *kind != 2)) return 0;
@@ -1461,25 +1464,28 @@ static int cached_tokens(const Glm53fMoeW *w, const Glm53fCfg *c, int T, int wit
     int most = g53h_grouped_max_tokens(&L) / G53_MOE_CHUNK * G53_MOE_CHUNK;
     if (most > T) most = T;
     if (most < T && most < G53_MOE_CHUNK) return 0;
-    /* a pass's buffers must fit beside what the caller keeps in HBM; shorter passes where they do not,
-     * chunks (which need the least) in the end. Asked once per size: the buffers are kept. */
-    static size_t granted = 0;
-    L.shared = with_shared ? (const G53hExpert *)&L : NULL;
-    for (;; most = most / 2 / G53_MOE_CHUNK * G53_MOE_CHUNK) {
-        if (most < 2) return 0;
-        const size_t need = g53h_grouped_bytes(&L, most) + (size_t)2 * most * c->hidden * sizeof(float);
-        if (need <= granted) break;
-        size_t free_b = 0, total_b = 0;
-        if (g53h_mem_info(&free_b, &total_b)) return 0;
-        if (need + ((size_t)64 << 20) <= free_b) { granted = need; break; }
-        if (most <= G53_MOE_CHUNK) return 0;
-    }
     int own = 0, others = 0;
     g53h_cache_held(w->src, w->layer, &own, &others);
     const long named = (long)most * c->topk + own < c->n_experts ? (long)most * c->topk + own : c->n_experts;
     read_switches();
     const long next = w->next_gate && (w->prefill_next || g_prefill_pred >= 0) ? c->n_experts : 0;
-    return named + others + next + cache->n_io + cache->qlen <= cache->nslot ? most : 0;
+    if (named + others + next + cache->n_io + cache->qlen > cache->nslot) return 0;
+    /* what a pass has to allocate must fit beside what the caller keeps in HBM; shorter passes where it
+     * does not, chunks (which need the least) in the end. Nothing is asked when every buffer is held. */
+    L.shared = with_shared ? (const G53hExpert *)&L : NULL;
+    resident_router(w->gate, (size_t)c->n_experts * c->hidden, &L.router_dt);
+    for (;; most = most / 2 / G53_MOE_CHUNK * G53_MOE_CHUNK) {
+        if (most < 2) return 0;
+        const size_t act = (size_t)most * c->hidden * sizeof(float), routed = (size_t)most * c->topk * sizeof(int);
+        size_t need = g53h_grouped_growth(&L, most) + buf_growth(&g_idx, routed + sizeof(int)) + buf_growth(&g_w, routed);
+        if (buf_growth(&g_xin, act) && !g53h_is_device_ptr(x)) need += act;
+        if (buf_growth(&g_out, act) && !g53h_is_device_ptr(out)) need += act;
+        if (!need) return most;
+        size_t free_b = 0, total_b = 0;
+        if (g53h_mem_info(&free_b, &total_b)) return 0;
+        if (need + ((size_t)64 << 20) <= free_b) return most;
+        if (most <= G53_MOE_CHUNK) return 0;
+    }
 }
 
 static void moe_layer(float *out, const float *x, const Glm53fMoeW *w, const Glm53fCfg *c, int T, int with_shared)
@@ -1491,7 +1497,7 @@ static void moe_layer(float *out, const float *x, const Glm53fMoeW *w, const Glm
         abort();
     }
     int t0 = 0, kind = 0;
-    const int pass = cached_tokens(w, c, T, with_shared, &kind);
+    const int pass = cached_tokens(out, x, w, c, T, with_shared, &kind);
     while (pass && T - t0 > 1) {                     /* a last chunk of one token decodes below */
         int n = T - t0 < pass ? T - t0 : pass;
         if (n % G53_MOE_CHUNK == 1) n--;

@@ -323,6 +323,9 @@ int   g53h_decode_publish(int slot, unsigned seq, size_t route_off, const int *i
  * decode kernels gives up (and sets bit 1 of their error flags); 0 restores the default.
  * Returns the previous setting. Waits between the waves of one workgroup are not affected. */
 int g53h_set_spin_limit(int polls);
+/* Test hook: the most free HBM that g53h_mem_info reports, for callers that ask it before they allocate;
+ * 0 restores the device's own figure. Returns the previous setting. */
+size_t g53h_set_mem_free(size_t bytes);
 /* Test hook: ORs bits into error word `word` (0 .. G53H_NERR-1) on the compute stream, as a
  * kernel that hit that condition would; the caller's next read of the flags sees them. */
 int g53h_inject_errors(int word, int bits);

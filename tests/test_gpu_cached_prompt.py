@@ -106,6 +106,33 @@ def test_failed_get_is_the_chunks_drop(L, layer):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+def test_pass_needs_memory_only_for_what_is_not_held(L):
+    """A call that cannot take the pass (too few slots) leaves no claim on memory: when HBM is full at the
+    next call, which could take it, the chunks run; with room again the pass does. Same output each time."""
+    say("cached prompt, HBM full")
+    sp = S.spec(2, NE=24, K=16, seed=8)              # the largest workspace: 2000 tokens, top-16
+    layer = sp, [S.expert_host(sp, p) for p in range(NP)], S.router_host(sp), S.bias_host(sp), S.expert_host(sp, "shared")
+    x = np.ascontiguousarray(S.x_host(sp, 2000, batch=9), np.float32)
+    one = glm53h.G53hExpert()
+    g = glm53h.G53hMoeLayer(hidden=sp.E, inter=sp.I, n_experts=sp.NE, topk=sp.K, router_dt=1, block_c=128,
+                            shared=C.addressof(one))
+    growth = L.g53h_grouped_growth
+    growth.argtypes, growth.restype = [C.POINTER(glm53h.G53hMoeLayer), C.c_int], C.c_size_t
+    if growth(C.byref(g), x.shape[0]) == 0:
+        pytest.skip("the library holds a larger workspace already")
+    want, _, _ = run(L, layer, x, sp.NE - 5)
+    was = L.g53h_set_mem_free(32 << 20)
+    try:
+        got, _, _ = run(L, layer, x, sp.NE + 64)
+    finally:
+        L.g53h_set_mem_free(was)
+    assert growth(C.byref(g), x.shape[0]) > 0        # no pass of all tokens was made
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    got, _, _ = run(L, layer, x, sp.NE + 64)
+    assert growth(C.byref(g), x.shape[0]) == 0
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def holds(layer, expert, at_hint=False):
     """A caller's own hold on an expert, as include/glm53f.h allows: taken before the calls, or by another
     user of the cache while a call runs (in its first hint)."""
