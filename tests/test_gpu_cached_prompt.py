@@ -31,7 +31,7 @@ def layer():
     return sp, pool, S.router_host(sp), S.bias_host(sp), S.expert_host(sp, "shared")
 
 
-def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True, hold=None):
+def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True, hold=None, reads=None):
     sp, pool, W, B, sh = layer
     cf = make_cfg(sp)
     cf.n_layers = 1
@@ -39,14 +39,20 @@ def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True, hold=No
     def view(_st, _layer, e, out):
         if e in fails:
             return -1
+        if reads is not None:                        # started and not handed back yet
+            reads.append(e)
+            most[0] = max(most[0], len(reads))
         q = out.contents
         q.gate, q.up, q.down = [fmat(w, s, r, c, 128, 128) for (w, s), (r, c) in
                                 zip(pool[e % NP], [(sp.I, sp.E), (sp.I, sp.E), (sp.E, sp.I)])]
         return 0
 
-    st = glm53h.G53hStore(glm53h.VIEW_FN(view), glm53h.DONE_FN(), None)
+    most = [0]
+    back = glm53h.DONE_FN(lambda _st, _layer, e: reads.remove(e)) if reads is not None else glm53h.DONE_FN()
+    st = glm53h.G53hStore(glm53h.VIEW_FN(view), back, None)
     c, probe = glm53h.Glm53fCache(), glm53h.Glm53fCache()
     check(L.g53h_cache_init_store(C.byref(probe), C.byref(st), C.byref(cf), 1 << 30, 0, 0), "cache")
+    most[0] = 0
     budget = probe.slot_bytes * slots
     L.glm53f_cache_free(C.byref(probe))
     check(L.g53h_cache_init_store(C.byref(c), C.byref(st), C.byref(cf), budget, n_io, 0), "cache")
@@ -74,7 +80,7 @@ def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True, hold=No
     assert pins == 0                                 # everything was released
     lost, drops.value = drops.value - was, was
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
-    return outs[0], gets, lost
+    return (outs[0], gets, lost) if reads is None else (outs[0], most[0])
 
 
 @pytest.mark.parametrize("T,mfma,n_io,prefetch_n,shared", [
@@ -103,6 +109,30 @@ def test_failed_get_is_the_chunks_drop(L, layer):
     want, _, lost = run(L, layer, x, sp.NE - 5, fails=(3, 17))
     got, _, lost1 = run(L, layer, x, sp.NE + 64, fails=(3, 17))
     assert lost1 == lost > 0
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+def test_gets_wait_for_hinted_reads(L, layer):
+    """A cold cache with hints: at most top-k reads of the call's own are under way at a time beside the
+    prefetch's n_io, so that the hinted reads are not overtaken."""
+    say("cached prompt, cold with hints")
+    sp, pool = layer[:2]
+    x = np.ascontiguousarray(S.x_host(sp, 64, batch=10), np.float32)
+    want, _, _ = run(L, layer, x, sp.NE - 5)
+    mem = []
+
+    def pinned(a):                                   # copies from other memory are not asynchronous
+        mem.append(L.g53h_host_alloc(a.nbytes))
+        b = np.frombuffer((C.c_uint8 * a.nbytes).from_address(mem[-1]), a.dtype)
+        b[:] = a
+        return b
+    try:
+        pool = [[(pinned(w), pinned(s)) for w, s in mats] for mats in pool]
+        got, most = run(L, (sp, pool) + layer[2:], x, sp.NE + 64, n_io=2, prefetch_n=6, reads=[])
+    finally:
+        for m in mem:
+            L.g53h_host_free(m)
+    assert 0 < most <= sp.K + 2
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
