@@ -1378,8 +1378,8 @@ static int moe_cached(float *out, const float *x, const Glm53fMoeW *w, const Glm
     /* Hinted reads go ahead on the prefetch stream, n_io at a time, as long as the gets do not overtake
      * them: a get of an expert that is still queued reads it on the demand stream, and the two streams
      * together move less than either alone (20 of 46 GB/s). So, as the chunks do, top-k gets, then a
-     * wait for what they had to read (64 tokens, 87 experts to read, n_io 4: 103 ms without the wait, 65
-     * with it; nothing resident is waited for, and without hints all reads queue up: 48 ms). */
+     * wait for what they had to read (64 tokens, 87 experts to read, n_io 4: 103 ms without the wait, 54
+     * with it, 65 by chunks; nothing resident is waited for, and without hints all reads queue up: 48). */
     const Glm53fCache *cache = (const Glm53fCache *)src;
     const int behind = prefetch && cache->n_io > 0, B = K < G53_MOE_BATCH ? K : G53_MOE_BATCH;
     uint64_t missed = cache->misses;
