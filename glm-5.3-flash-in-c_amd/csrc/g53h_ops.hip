@@ -597,12 +597,17 @@ static bool g53_router_small(int T, int gate_dt, int NE, int E)
            NE <= (T == 1 ? 32 : 128) && T <= 256;
 }
 
-/* Partial sums that a batch of at most T tokens may need, over the column ranges of g53h_router_into
- * (S T <= 16 * 2560 / et): a smaller batch after a larger one, a captured one for instance, allocates
- * nothing. */
+/* Workgroups up to which a batch with few tiles splits its columns: 10 a CU where the selection takes every
+ * range's sums in one flight of loads (288 experts x 4096, both launches, us: 150 tokens 22.7 at 640
+ * workgroups, 20.2 at 2560; 256: 28.4, 24.4; 5120 is no faster), 2.5 a CU above 320 experts, where it takes
+ * them range by range (1024 x 2048: 64 tokens 37.7 at 640, 66.5 at 2560; 512 x 4096, 150: 45.0, 59.0). */
+static int g53_router_split_wgs(int NE) { return NE <= 320 ? 2560 : 640; }
+
+/* Partial sums that a batch of at most T tokens may need over the column ranges (S T <= 16 workgroups /
+ * et): a smaller batch after a larger one, a captured one for instance, allocates nothing. */
 static size_t g53_router_part_need(int T, int NE, int E)
 {
-    const size_t et = (NE + 15) / 16, rows = min((size_t)8 * T, (size_t)40960 / et);
+    const size_t et = (NE + 15) / 16, rows = min((size_t)8 * T, (size_t)16 * g53_router_split_wgs(NE) / et);
     return E % 512 == 0 ? rows * NE * sizeof(double) : 0;
 }
 size_t g53h_router_growth(int T, int gate_dt, int NE, int E)
@@ -629,13 +634,11 @@ int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate
     const double *psum = nullptr;                            /* split logits, summed by the selection */
     int nsum = 1;
     if (T >= 2 && gate_dt == 1 && E % 256 == 0) {           /* batches: the matrix-core form */
-        /* few tiles (small T): the columns are split over up to 8 workgroups per tile while that gives
-         * at most 10 workgroups per CU; the partial sums are added in column order after (288 experts x
-         * 4096, both launches: 150 tokens 22.7 us at 640 workgroups, 20.2 at 2560; 256: 28.4, 24.4;
-         * 5120 is no faster) */
+        /* few tiles (small T): the columns are split over up to 8 workgroups per tile; the partial sums are
+         * added in column order after */
         const int tiles = ((NE + 15) / 16) * ((T + 15) / 16);
         int S = 1;
-        while (S < 8 && tiles * S * 2 <= 2560 && (E / (S * 2)) % 256 == 0) S *= 2;
+        while (S < 8 && tiles * S * 2 <= g53_router_split_wgs(NE) && (E / (S * 2)) % 256 == 0) S *= 2;
         double *part = nullptr;
         if (E % 512 == 0) {
             part = (double *)g53_router_part(g53_router_part_need(T, NE, E));

@@ -89,7 +89,7 @@ def test_small_layer_descriptors(L, T):
 @pytest.mark.parametrize("T,NE,E,K,shift", [
     (1, 1, 128, 1, 0), (1, 32, 256, 8, 0), (2, 65, 384, 8, 0), (3, 16, 4096, 16, 0), (512, 128, 512, 4, 0),
     (200, 320, 128, 10, 0), (512, 129, 128, 3, 0), (5, 33, 256, 8, 1),
-    (257, 64, 256, 8, 0), (17, 129, 768, 8, 0), (700, 300, 2048, 8, 0), (2000, 288, 512, 8, 0)])
+    (257, 64, 256, 8, 0), (64, 321, 2048, 8, 0), (33, 1024, 1024, 8, 0), (17, 129, 768, 8, 0), (700, 300, 2048, 8, 0), (2000, 288, 512, 8, 0)])
 def test_small_router(L, T, NE, E, K, shift):
     """Either side of the rule, and the matrix-core form over one and several column ranges of one and
     more chunks; shift moves x off 16-byte alignment."""
