@@ -269,8 +269,8 @@ __global__ void __launch_bounds__(64) k_router_scores(float *__restrict__ score,
 
 /* The same scores for many tokens on the FP64 matrix cores (v_mfma_f64_16x16x4f64). Every
  * product (double)bf16 * (double)x is exact in double, as in k_router_scores; the instruction
- * adds them with double FMAs, in an order of its own. A workgroup computes the 16 x 16 tile of
- * experts e0 = 16 * blockIdx.x .. +15 and tokens t0 = 16 * blockIdx.y .. +15; its four waves
+ * adds them with double FMAs, in an order of its own. A workgroup computes the 16 x 16 tile (bx, by) of
+ * experts e0 = 16 * bx .. +15 and tokens t0 = 16 * by .. +15 over column range bz; its four waves
  * split the columns (wave w takes columns 64w .. 64w+63 of every 256-column chunk) and their
  * partial sums are added in LDS at the end. Operands: lane l gives A[l % 16][l / 16] (an
  * expert's weight) and B[l / 16][l % 16] (a token's x); step s uses column 64w + 16(l/16) + s
@@ -279,26 +279,36 @@ __global__ void __launch_bounds__(64) k_router_scores(float *__restrict__ score,
  * 256. The double instruction's rate bounds it from some hundred tokens on, below that the wait for
  * a chunk, so the next chunk's operands are requested before this one is multiplied (288 experts x
  * 4096 with the selection, us: 150 tokens 26.3 -> 20.2, 384: 47.3 -> 32.7, 2048: 109.8 -> 103.5, where a
- * 32 x 32 tile per wave over eight column ranges had been faster than the unpipelined loop). */
+ * 32 x 32 tile per wave over eight column ranges had been faster than the unpipelined loop).
+ * The grid is (bx, by, bz), or flat (S column ranges) with a contiguous run of tiles, experts fastest, on
+ * each of the 8 XCDs that workgroups are dealt to in turn, so that a token tile is fetched into one L2
+ * instead of into as many as it meets experts. */
 typedef double g53_v4d __attribute__((ext_vector_type(4)));
 typedef float g53_v4f __attribute__((ext_vector_type(4)));
 #define G53_RM_XST 260                                  /* LDS floats per token row       */
 __global__ void __launch_bounds__(256) k_router_mfma(float *__restrict__ score, float *__restrict__ choice,
                                                      const float *__restrict__ x, int T,
                                                      const uint16_t *__restrict__ gate,
-                                                     const float *__restrict__ bias, int NE, int E, int klen,
+                                                     const float *__restrict__ bias, int NE, int E, int klen, int S,
                                                      double *__restrict__ psum)
 {
+    int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+    if (S) {                                                 /* flat */
+        const int ET = (NE + 15) >> 4, TT = (T + 15) >> 4;
+        const int j = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
+        if (j >= ET * TT * S) return;
+        bx = j % ET; by = (j / ET) % TT; bz = j / (ET * TT);
+    }
     __shared__ __attribute__((aligned(16))) float xs[16 * G53_RM_XST];
     __shared__ g53_v4d part[3][64];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int t0 = blockIdx.y * 16, e0 = blockIdx.x * 16;
+    const int t0 = by * 16, e0 = bx * 16;
     const int i = lane & 15, g = lane >> 4;
     const int er = e0 + i < NE ? e0 + i : NE - 1;          /* rows past NE: discarded       */
     const uint16_t *wrow = gate + (size_t)er * E + w * 64 + g * 16;
     const float *xl = xs + i * G53_RM_XST + w * 64 + g * 16;
     g53_v4d acc = {0.0, 0.0, 0.0, 0.0};
-    const int kb = blockIdx.z * klen;                        /* this workgroup's column range */
+    const int kb = bz * klen;                                /* this workgroup's column range */
     /* the next chunk's operands come to registers while this one's are multiplied */
     g53_u4 wv[2];
     g53_v4f xv[4];
@@ -334,7 +344,7 @@ __global__ void __launch_bounds__(256) k_router_mfma(float *__restrict__ score, 
     for (int r = 0; r < 4; r++) {
         const int e = e0 + 4 * r + g;
         if (t < T && e < NE && psum) {                        /* a column range: its sum */
-            psum[((size_t)blockIdx.z * T + t) * NE + e] = acc[r];
+            psum[((size_t)bz * T + t) * NE + e] = acc[r];
         } else if (t < T && e < NE) {
             const float s = g53_sigmoidf((float)acc[r]);
             score[(size_t)t * NE + e] = s;
@@ -645,8 +655,15 @@ int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate
             if (!part) return -1;
             if (S == 1) part = nullptr;
         }
-        hipLaunchKernelGGL(k_router_mfma, dim3((NE + 15) / 16, (T + 15) / 16, S), dim3(256), 0, g53h_stream(),
-                           score, choice, x, T, (const uint16_t *)gate, bias, NE, E, E / S, part);
+        /* The flat order with few expert tiles and activations that fill the 32 MB of L2 (experts x hidden, both
+         * launches, us, grid / flat: 64 x 4096, 4096 tokens 64.0 / 56.8; 128 x 4096, 2048: 58.7 / 54.0; 24 x 2048,
+         * 8192: 47.9 / 43.9; the 32 x 32 kernel before: 54.8, 52.1, 43.8), and where a grid has too few rows for
+         * the tokens. More expert tiles gain nothing (288 x 4096, 2048: 102.3 / 102.7; 192 x 4096, 8192: 255.1 /
+         * 254.9), smaller batches lose the index arithmetic's time (288 x 4096, 5: 11.7 / 12.0). */
+        const int tt = (T + 15) / 16, flat = (NE <= 160 && (long)T * E >= (8 << 20)) || tt > 65535;
+        const dim3 grid = flat ? dim3((unsigned)(tiles * S + 7) / 8 * 8) : dim3((NE + 15) / 16, tt, S);
+        hipLaunchKernelGGL(k_router_mfma, grid, dim3(256), 0, g53h_stream(), score, choice, x, T,
+                           (const uint16_t *)gate, bias, NE, E, E / S, flat ? S : 0, part);
         G53_LAUNCHED("k_router_mfma");
         if (S > 1) { psum = part; nsum = S; }
     } else {

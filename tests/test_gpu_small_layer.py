@@ -89,10 +89,11 @@ def test_small_layer_descriptors(L, T):
 @pytest.mark.parametrize("T,NE,E,K,shift", [
     (1, 1, 128, 1, 0), (1, 32, 256, 8, 0), (2, 65, 384, 8, 0), (3, 16, 4096, 16, 0), (512, 128, 512, 4, 0),
     (200, 320, 128, 10, 0), (512, 129, 128, 3, 0), (5, 33, 256, 8, 1),
-    (257, 64, 256, 8, 0), (64, 321, 2048, 8, 0), (33, 1024, 1024, 8, 0), (17, 129, 768, 8, 0), (700, 300, 2048, 8, 0), (2000, 288, 512, 8, 0)])
+    (257, 64, 256, 8, 0), (64, 321, 2048, 8, 0), (33, 1024, 1024, 8, 0), (17, 129, 768, 8, 0), (700, 300, 2048, 8, 0), (2000, 288, 512, 8, 0),
+    (4100, 30, 2048, 8, 0), (16400, 100, 512, 4, 0)])
 def test_small_router(L, T, NE, E, K, shift):
     """Either side of the rule, and the matrix-core form over one and several column ranges of one and
-    more chunks; shift moves x off 16-byte alignment."""
+    more chunks, in either order of its tiles; shift moves x off 16-byte alignment."""
     say("small router", T, NE, E, K, shift)
     sp = S.LayerSpec(E=E, I=128, NE=NE, K=K, router_sigma=0.05)
     rf, bias = S.router_host(sp), S.bias_host(sp)
@@ -108,6 +109,31 @@ def test_small_router(L, T, NE, E, K, shift):
     assert np.array_equal(idx.download(np.int32).reshape(T, K), wi)
     assert np.array_equal(bits(w.download(np.float32).reshape(T, K)), bits(ww))
     assert flag.download(np.int32)[0] == 0
+
+
+def test_router_more_tokens_than_grid_rows(L):
+    """1,048,592 tokens, 65,537 tiles of 16: a block of tokens repeated gives its result repeated."""
+    say("router, a million tokens")
+    E, NE, K, n, reps = 256, 20, 4, 4096, 256
+    T = n * reps + 16
+    sp = S.LayerSpec(E=E, I=128, NE=NE, K=K, router_sigma=0.05)
+    rf, bias = S.router_host(sp), S.bias_host(sp)
+    x = S.x_host(sp, n, batch=7)
+    xd = DevBuf(T * E * 4)
+    check(L.g53h_h2d(xd.ptr, x.ctypes.data, x.nbytes), "h2d")
+    have = n
+    while have < T:                                  # doubling copies
+        m = min(have, T - have)
+        check(L.g53h_d2d(xd.ptr + have * E * 4, xd.ptr, m * E * 4), "d2d")
+        have += m
+    g, b = DevBuf.from_array((rf.view(np.uint32) >> 16).astype(np.uint16)), DevBuf.from_array(bias)
+    idx, w = DevBuf(T * K * 4), DevBuf(T * K * 4)
+    check(L.g53h_router(idx.ptr, w.ptr, xd.ptr, T, g.ptr, 1, b.ptr, NE, E, K, sp.norm_topk,
+                        C.c_float(sp.routed_scale), None), "router")
+    wi, ww = O.router(O.oracle(), x, sp, rf, bias)
+    at = np.arange(T) % n
+    assert np.array_equal(idx.download(np.int32).reshape(T, K), wi[at])
+    assert np.array_equal(bits(w.download(np.float32).reshape(T, K)), bits(ww)[at])
 
 
 def test_small_router_nan(L):
