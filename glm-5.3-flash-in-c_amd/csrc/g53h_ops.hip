@@ -181,15 +181,23 @@ extern "C" int g53h_mm_f8(float *y, const float *x, int T, const G53hMat *m)
         return g53h_fail("g53h_mm_f8: bad geometry %dx%d block %dx%d scols %d", m->rows, m->cols,
                          m->br, m->bc, m->scols);
     if (m->flags & G53H_MAT_TILED) return g53h_fail("g53h_mm_f8: octet-tiled codes are read by the decode kernel only");
-    if (m->flags == 0 && m->bc == 128) {
-        /* Two tokens a workgroup share each weight's decode; while single tokens leave every CU at
-         * most one workgroup the call is a chain of latencies instead, and 16 waves, each with its
-         * block's codes in flight, shorten it. Measured, (1 token, 16 waves) against (2, 8): 4096 x
-         * 4096 1 token 10.5 against 14.8 us, 2048 x 4096 4 tokens 12.6 against 15.4; 4096 x 2048 24
-         * tokens 28.6 against 19.1, 4096 x 4096 64 tokens 123 against 64. (3 and 4 tokens: 20 and 31
-         * us at 24, the chains' registers spill.) */
-        const long tiles = (m->rows + 63) / 64;
-        const int al = m->cols % 16 == 0 && ((uintptr_t)m->w & 15) == 0, one = tiles * T <= g53h_num_cus();
+    /* FP8 with 128-column blocks: a row tile. Two tokens a workgroup share each weight's decode; while single
+     * tokens leave every CU at most one workgroup the call is a chain of latencies instead, and 16 waves, each
+     * with its block's codes in flight, shorten it. Measured, (1 token, 16 waves) against (2, 8): 4096 x 4096 1
+     * token 10.5 against 14.8 us, 2048 x 4096 4 tokens 12.6 against 15.4; 4096 x 2048 24 tokens 28.6 against
+     * 19.1, 4096 x 4096 64 tokens 123 against 64. (3 and 4 tokens: 20 and 31 us at 24, the chains' registers
+     * spill.) Codes and columns that are not in multiples of 16 bytes load by words: 4096 x 1030, 24 tokens
+     * 36.5 us with a thread per (row, token), 19.0 here; 333 x 2047, 5: 55.0, 12.1.
+     * A thread per (row, token) is the faster one where the only block, or the second of two, is partial and
+     * its columns, taken 8 at a time, are most of the work: below 128 columns (us, thread / tile: 4096 x 100, 1
+     * token 3.8 / 4.9, 24 tokens 4.3 / 10.3; 4096 x 17, 300: 8.2 / 62.4; 2048 x 112, 64: 4.7 / 7.3; aligned and
+     * one workgroup a CU, 4096 x 112, 1: 3.7 / 3.6), and unaligned rows of 136 to 207 in whole tiles (4096 x 136,
+     * 24: 5.0 / 8.2; 4096 x 200, 64: 13.8 / 16.6; 129 columns, 64: 20.3 / 16.3; 250, 64: 23.8 / 20.6). */
+    const long tiles = (m->rows + 63) / 64;
+    const int al = m->cols % 16 == 0 && ((uintptr_t)m->w & 15) == 0, one = tiles * T <= g53h_num_cus();
+    const int narrow = m->cols < 128 ? !(al && one)
+                                     : !al && !one && m->rows % 64 == 0 && m->cols >= 136 && m->cols < 208;
+    if (m->flags == 0 && m->bc == 128 && !narrow) {
         const long wgs = tiles * (one ? T : (T + 1) / 2);
         if (wgs > 0x7fffffffL) return g53h_fail("g53h_mm_f8: %d rows x %d tokens", m->rows, T);
         const dim3 g((unsigned)wgs);

@@ -22,7 +22,9 @@ def L():
 @pytest.mark.parametrize("rows,cols,br,T,shift", [
     (1, 5, 128, 1, 0), (64, 128, 128, 1, 0), (63, 127, 128, 2, 0), (65, 129, 16, 3, 0), (128, 136, 128, 4, 8),
     (200, 1030, 16, 5, 0), (130, 1024, 128, 9, 3), (300, 4096, 128, 2, 1), (4096, 2048, 128, 24, 0),
-    (100, 1152, 128, 7, 0), (64, 2047, 64, 13, 16), (256, 2176, 128, 130, 0), (4100, 131, 128, 5, 0)])
+    (100, 1152, 128, 7, 0), (64, 2047, 64, 13, 16), (256, 2176, 128, 130, 0), (4100, 131, 128, 5, 0),
+    (200, 64, 128, 3, 0), (4000, 112, 128, 4, 0), (4096, 112, 128, 5, 0), (4096, 100, 16, 24, 0), (2048, 136, 128, 24, 0),
+    (2048, 207, 128, 9, 1), (2048, 208, 128, 9, 1), (2047, 180, 128, 24, 0), (2048, 135, 128, 9, 0)])
 def test_mm_f8_rows(L, rows, cols, br, T, shift):
     say("mm rows", rows, cols, br, T, shift)
     rng = np.random.default_rng(rows * 7 + cols)
