@@ -394,7 +394,7 @@ struct G53GrpArgs {
                                       2: experts MFMA-tiled, planes in column order        */
     int partial;                   /* 1: experts without weights are outside this batch and
                                       left alone, unless marked dropped (gate.flags & G53H_MAT_DROPPED)    */
-    uint64_t *trace;               /* optional: [items][32] timestamps of each gate/up item  */
+    uint64_t *trace;               /* optional: [items][8] timestamps of each gate/up item   */
 };
 
 /* The clamped SwiGLU of src/core/glm53f_ops.c:486-494 (gate clamped from above, up both ways)
@@ -654,7 +654,7 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
     for (;;) {
         const int n = cur.tl.z, pos0 = cur.tl.y;
         if (GATEUP && a.trace && tid == 0) {
-            uint64_t *tr = a.trace + (size_t)cur.num * 32;
+            uint64_t *tr = a.trace + (size_t)cur.num * 8;
             tr[0] = __builtin_amdgcn_s_memrealtime();
             tr[4] = (uint64_t)__smid() << 32 | (uint32_t)(pos0 << 8 | n);
             tr[5] = (uint64_t)blockIdx.x << 32 | (uint32_t)(cur.tl.x << 8 | cur.mb);
@@ -694,7 +694,7 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
             step(kb, ops[0], ops[1]);
             step(kb + 1, ops[1], ops[0]);
         }
-        if (GATEUP && a.trace && tid == 0) a.trace[(size_t)cur.num * 32 + 2] = __builtin_amdgcn_s_memrealtime();
+        if (GATEUP && a.trace && tid == 0) a.trace[(size_t)cur.num * 8 + 2] = __builtin_amdgcn_s_memrealtime();
         const int j = half * 32 + i;                         /* this lane's position */
         if (GATEUP) {
             /* SwiGLU; the activation planes of the item's 128 rows are put together in the slot
@@ -739,7 +739,7 @@ __global__ void __launch_bounds__(64 * G53_GRP_NW, 1) k_grp_gemm(G53GrpArgs a)
                 *(g53_v4i *)(a.aq + ((size_t)p * a.P + pos0 + jj) * a.I + cur.mb * 128 + piece * 16) =
                     *(const g53_v4i *)(ao + (p * G53_GRP_NT + jj) * 128 + piece * 16);
             }
-            if (a.trace && tid == 0) a.trace[(size_t)cur.num * 32 + 3] = __builtin_amdgcn_s_memrealtime();
+            if (a.trace && tid == 0) a.trace[(size_t)cur.num * 8 + 3] = __builtin_amdgcn_s_memrealtime();
         } else {
 #pragma unroll
             for (int f = 0; f < 2; f++) {

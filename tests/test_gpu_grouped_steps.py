@@ -59,3 +59,22 @@ def test_grouped_unaligned_codes(L, shift, T, tiled):
     out, idx, _ = run(layer, x, 1, "g53h_moe_grouped")
     assert np.array_equal(idx, wi)
     assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
+
+
+def test_trace_stays_in_its_buffer(L):
+    """g53h_set_grouped_trace writes 8 words for each gate/up item and nothing after them."""
+    say("grouped trace")
+    sp = S.LayerSpec(E=512, I=512, NE=3, K=3, router_sigma=0.02)
+    layer = S.DeviceLayer.build(sp)
+    items = (sp.NE + 1) * sp.I // 128                # five tokens: a tile of each expert and the shared one
+    buf = DevBuf(items * 32 * 8)
+    buf.zero()
+    check(L.g53h_set_grouped_trace(buf.ptr), "trace")
+    try:
+        run(layer, S.x_host(sp, 5, batch=3), 1, "g53h_moe_grouped")
+    finally:
+        check(L.g53h_set_grouped_trace(None), "trace")
+    got = buf.download(np.uint64)
+    t = got[:items * 8].reshape(items, 8)
+    assert (t[:, 0] > 0).all() and (t[:, 2] >= t[:, 0]).all() and (t[:, 3] >= t[:, 2]).all()
+    assert not got[items * 8:].any()
