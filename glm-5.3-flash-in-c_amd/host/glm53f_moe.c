@@ -849,6 +849,7 @@ static void decode_cached(float *out, const float *x, const Glm53fMoeW *w, const
             i4m = 0;
     }
     if (!nh) i4r = i4t = i4m = mt = 0;
+    const int mviews = mt;
     HP(3);
     if (spec) {                  /* every chosen expert was in the kernel's table: the output is done */
         g_spec_n[0]++;
@@ -882,21 +883,23 @@ static void decode_cached(float *out, const float *x, const Glm53fMoeW *w, const
     const int one_i4t = i4t && (!with_shared || (tab[K].gate.flags & G53H_MAT_TILED));
     const int one_i4m = i4m && (!with_shared || (tab[K].gate.flags & G53H_MAT_MTILED));
     const int one_mt = mt && (!with_shared || (tab[K].gate.flags & G53H_MAT_MTILED));
-    if ((i4t && !one_i4t) || (i4m && !one_i4m)) {
-        /* the row kernels read row-major levels (and steps) */
-        static G53Buf g_i4u[GLM53F_MAX_TOPK];
+    if ((i4t && !one_i4t) || (i4m && !one_i4m) || (mviews && !one_mt)) {
+        /* the row kernels read row-major levels (and steps), and row-major or octet-tiled codes */
+        static G53Buf g_unt[GLM53F_MAX_TOPK];
         for (int j = 0; j < K; j++) {
             G53hMat *ms[3] = {&tab[j].gate, &tab[j].up, &tab[j].down};
             if (!ms[0]->w) continue;
             size_t need = 0;
             for (int i = 0; i < 3; i++)
-                need += ((((size_t)ms[i]->rows * (ms[i]->cols / 2)) + 255) & ~(size_t)255) +
+                need += ((((size_t)ms[i]->rows * (mviews ? ms[i]->cols : ms[i]->cols / 2)) + 255) & ~(size_t)255) +
                         (i4m ? (((size_t)ms[i]->rows * ms[i]->scols * 4 + 255) & ~(size_t)255) : 0);
-            uint8_t *b = (uint8_t *)buf_get(&g_i4u[j], need);
+            uint8_t *b = (uint8_t *)buf_get(&g_unt[j], need);
             for (int i = 0; i < 3; i++) {
                 uint8_t *lv = b;
-                b += (((size_t)ms[i]->rows * (ms[i]->cols / 2)) + 255) & ~(size_t)255;
-                if (i4m) {
+                b += (((size_t)ms[i]->rows * (mviews ? ms[i]->cols : ms[i]->cols / 2)) + 255) & ~(size_t)255;
+                if (mviews) {
+                    if (g53h_mtile_f8(lv, ms[i]->w, ms[i]->rows, ms[i]->cols, 1)) g53_die("converting an expert view");
+                } else if (i4m) {
                     float *st = (float *)b;
                     b += ((size_t)ms[i]->rows * ms[i]->scols * 4 + 255) & ~(size_t)255;
                     if (g53h_mtile_i4(lv, st, ms[i]->w, ms[i]->s, ms[i]->rows, ms[i]->cols, 1))
@@ -906,7 +909,7 @@ static void decode_cached(float *out, const float *x, const Glm53fMoeW *w, const
                     g53_die("converting an int4 expert view");
                 }
                 ms[i]->w = lv;
-                ms[i]->flags = G53H_MAT_I4;
+                ms[i]->flags = mviews ? 0 : G53H_MAT_I4;
             }
         }
     }

@@ -13,6 +13,7 @@ import oracle_lib as O
 from glm53h import check
 from test_gpu_cache import make_cfg
 from test_gpu_grouped import within
+from test_gpu_i4 import dev_quant, imat
 from test_gpu_parity import fmat, say
 
 pytestmark = pytest.mark.gpu
@@ -58,9 +59,8 @@ def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True, hold=No
     check(L.g53h_cache_init_store(C.byref(c), C.byref(st), C.byref(cf), budget, n_io, 0), "cache")
     w = glm53h.Glm53fMoeW()
     w.gate, w.bias, w.src, w.prefetch_n = W.ctypes.data, B.ctypes.data, C.pointer(c.src), prefetch_n
-    (gw, gs), (uw, us), (dw, ds) = sh
-    w.sh_gate, w.sh_up = fmat(gw, gs, sp.I, sp.E, 128, 128), fmat(uw, us, sp.I, sp.E, 128, 128)
-    w.sh_down = fmat(dw, ds, sp.E, sp.I, 128, 128)
+    w.sh_gate, w.sh_up, w.sh_down = [m if isinstance(m, glm53h.Glm53fMat) else fmat(*m, r, c, 128, 128) for m, (r, c) in
+                                     zip(sh, [(sp.I, sp.E), (sp.I, sp.E), (sp.E, sp.I)])]
     drops = C.c_long.in_dll(L, "glm53f_expert_drops")
     was, outs = drops.value, []
     done = hold(c) if hold else None
@@ -199,4 +199,22 @@ def test_held_slots_leave_room(L, layer, monkeypatch, where, mfma):
     hold = holds(0 if where == "this layer" else 1, 3, at_hint=where == "during the call")
     got, _, lost = run(L, layer, x, sp.NE, prefetch_n=6, hold=hold)
     assert lost == 0
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("T", [1, 3])
+def test_int4_shared_expert_beside_mfma_slots(L, layer, monkeypatch, T):
+    """A shared expert that cannot be kept tiled: the row kernels read the MFMA-tiled views as rows, and the
+    output is that of row-major slots."""
+    say("cached, int4 shared expert", T)
+    sp, pool, W, B, sh = layer
+    keep = [dev_quant(w, s, r, c, 128, 128) + (r, c) for (w, s), (r, c) in
+            zip(sh, [(sp.I, sp.E), (sp.I, sp.E), (sp.E, sp.I)])]
+    layer = sp, pool, W, B, [imat(*k) for k in keep]
+    x = np.ascontiguousarray(S.x_host(sp, T, batch=11), np.float32)
+    monkeypatch.setenv("GLM53F_CACHE_ROWMAJOR", "1")
+    want, _, _ = run(L, layer, x, sp.NE)
+    monkeypatch.delenv("GLM53F_CACHE_ROWMAJOR")
+    monkeypatch.setenv("GLM53F_CACHE_MFMA", "1")
+    got, _, _ = run(L, layer, x, sp.NE)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
