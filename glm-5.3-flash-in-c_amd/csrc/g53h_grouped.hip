@@ -355,13 +355,12 @@ __device__ __forceinline__ void g53_grp_bar()
     asm volatile("" ::: "memory");
 }
 
-/* A descriptor with the layout the grouped kernels assume: octet-tiled iff the pass is, or
- * MFMA-tiled in an MFMA-tiled pass. */
+/* A descriptor with the layout the grouped kernels assume: exactly the pass's. */
 __device__ __forceinline__ bool g53_grp_mat_ok(const G53hMat *m, int rows, int cols, int tiled)
 {
     const int fl = g53_sld(&m->flags);
     const int want = tiled == 2 ? G53H_MAT_MTILED : tiled ? G53H_MAT_TILED : 0;
-    return !(fl & G53H_MAT_I4) && (fl & (tiled == 2 ? G53H_MAT_MTILED : G53H_MAT_TILED)) == want && g53_sld(&m->br) == 128 &&
+    return (fl & (G53H_MAT_I4 | G53H_MAT_I4T | G53H_MAT_TILED | G53H_MAT_MTILED)) == want && g53_sld(&m->br) == 128 &&
            g53_sld(&m->bc) == 128 && g53_sld(&m->rows) == rows && g53_sld(&m->cols) == cols &&
            g53_sld(&m->scols) >= cols / 128;
 }

@@ -180,7 +180,8 @@ extern "C" int g53h_mm_f8(float *y, const float *x, int T, const G53hMat *m)
         m->scols != (m->cols + m->bc - 1) / m->bc || ((m->flags & G53H_MAT_I4) && (m->cols & 1)))
         return g53h_fail("g53h_mm_f8: bad geometry %dx%d block %dx%d scols %d", m->rows, m->cols,
                          m->br, m->bc, m->scols);
-    if (m->flags & G53H_MAT_TILED) return g53h_fail("g53h_mm_f8: octet-tiled codes are read by the decode kernel only");
+    if (m->flags & (G53H_MAT_TILED | G53H_MAT_MTILED | G53H_MAT_I4T))
+        return g53h_fail("g53h_mm_f8: tiled codes are read by the layer kernels only (flags %d)", m->flags);
     /* FP8 with 128-column blocks: a row tile. Two tokens a workgroup share each weight's decode; while single
      * tokens leave every CU at most one workgroup the call is a chain of latencies instead, and 16 waves, each
      * with its block's codes in flight, shorten it. Measured, (1 token, 16 waves) against (2, 8): 4096 x 4096 1

@@ -100,10 +100,12 @@ __device__ inline float g53_row_dot_tiled(const G53hMat &m, int o, const float *
     return (float)acc;
 }
 
-/* A usable octet-tiled matrix: 128-column blocks and whole row octets (the tiled format's
- * definition); anything else marked tiled is not read. */
+/* A matrix the row kernels read: row-major FP8 or int4, or a usable octet-tiled one, of 128-column
+ * blocks and whole row octets (the tiled format's definition). The matrix-core layouts and int4-tiled
+ * levels are not read. */
 __device__ __forceinline__ bool g53_rows_ok(const G53hMat &m)
 {
+    if (m.flags & (G53H_MAT_MTILED | G53H_MAT_I4T)) return false;
     if (!(m.flags & G53H_MAT_TILED) || (m.flags & G53H_MAT_I4)) return true;
     return m.bc == 128 && m.cols == 128 * m.scols && (m.rows & 7) == 0 && ((uintptr_t)m.w & 15) == 0;
 }

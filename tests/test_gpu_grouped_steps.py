@@ -78,3 +78,25 @@ def test_trace_stays_in_its_buffer(L):
     t = got[:items * 8].reshape(items, 8)
     assert (t[:, 0] > 0).all() and (t[:, 2] >= t[:, 0]).all() and (t[:, 3] >= t[:, 2]).all()
     assert not got[items * 8:].any()
+
+
+@pytest.mark.parametrize("tiled,flags", [(False, 8), (True, 8), (True, 2 | 8), (False, 16), (False, 2), (True, 0)])
+def test_grouped_other_layouts_are_unusable(L, tiled, flags):
+    """A descriptor marked with any layout but the pass's: flag 8, and the expert's share is zero, as that of
+    a layer without it."""
+    say("grouped, other layout", tiled, flags)
+    sp = S.LayerSpec(E=512, I=512, NE=3, K=3, router_sigma=0.02)
+    x = S.x_host(sp, 5, batch=4)
+    outs = []
+    for missing in (False, True):
+        layer = S.DeviceLayer.build(sp, tiled=tiled)
+        e = layer.experts[1]
+        layer.experts[1] = G53hExpert() if missing else G53hExpert(
+            *[G53hMat(m.w, m.s, m.rows, m.cols, m.br, m.bc, m.scols, flags) for m in (e.gate, e.up, e.down)])
+        layer.table.upload(np.frombuffer(bytes(layer.experts), np.uint8))
+        L.g53h_grouped_errors()
+        xd, od = DevBuf.from_array(x), DevBuf(x.nbytes)
+        check(L.g53h_moe_grouped(od.ptr, xd.ptr, 5, C.byref(layer.layer), None, None), "grouped")
+        assert L.g53h_grouped_errors() == (0 if missing else 8)
+        outs.append(od.download(np.uint32))
+    assert np.array_equal(*outs)

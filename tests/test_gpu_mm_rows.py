@@ -41,3 +41,11 @@ def test_mm_f8_rows(L, rows, cols, br, T, shift):
     got = yd.download(np.float32)
     assert got[-1] == 7.0                            # nothing past the last row
     assert same(got[:-1].reshape(T, rows), O.mm_f8(O.oracle(), x, w, s, rows, cols, br, 128))
+
+
+@pytest.mark.parametrize("flags", [2, 8, 4 | 8, 4 | 16])
+def test_mm_f8_refuses_tiled_codes(L, flags):
+    say("mm, tiled codes", flags)
+    buf = DevBuf(1 << 16)
+    m = G53hMat(buf.ptr, buf.ptr, 64, 128, 1 if flags & 4 else 128, 64 if flags & 4 else 128, 2 if flags & 4 else 1, flags)
+    assert L.g53h_mm_f8(buf.ptr, buf.ptr, 1, C.byref(m)) == -1

@@ -86,6 +86,28 @@ def test_small_layer_descriptors(L, T):
     assert np.array_equal(got[1], want[1]) and np.array_equal(bits(got[0]), bits(want[0]))
 
 
+@pytest.mark.parametrize("block_c", [128, 0])
+@pytest.mark.parametrize("flags", [8, 4 | 8, 4 | 16])
+def test_unreadable_layouts_give_nan(L, flags, block_c):
+    """A descriptor in a layout that the small-layer and row kernels do not read (MFMA-tiled, int4-tiled):
+    NaN for the tokens that chose the expert, not a misread one; the other tokens as before."""
+    say("small layer, unreadable layout", flags, block_c)
+    sp = S.LayerSpec(E=384, I=256, NE=8, K=2, router_sigma=0.05)
+    layer = S.DeviceLayer.build(sp)
+    layer.layer.block_c = block_c
+    x = S.x_host(sp, 9, batch=8)
+    want, idx, _ = run(layer, x, 0)
+    d = layer.experts[3]
+    layer.experts[3] = G53hExpert(*[G53hMat(m.w, m.s, m.rows, m.cols, 1 if flags & 4 else m.br, 64 if flags & 4 else m.bc,
+                                            m.cols // (64 if flags & 4 else 128), flags) for m in (d.gate, d.up, d.down)])
+    layer.table.upload(np.frombuffer(bytes(layer.experts), np.uint8))
+    got, idx1, _ = run(layer, x, 0)
+    assert np.array_equal(idx, idx1)
+    hit = (idx == 3).any(axis=1)
+    assert hit.any() and not hit.all()
+    assert np.isnan(got[hit]).all() and np.array_equal(bits(got[~hit]), bits(want[~hit]))
+
+
 @pytest.mark.parametrize("T,NE,E,K,shift", [
     (1, 1, 128, 1, 0), (1, 32, 256, 8, 0), (2, 65, 384, 8, 0), (3, 16, 4096, 16, 0), (512, 128, 512, 4, 0),
     (200, 320, 128, 10, 0), (512, 129, 128, 3, 0), (5, 33, 256, 8, 1),
