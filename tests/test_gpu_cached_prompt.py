@@ -32,7 +32,8 @@ def layer():
     return sp, pool, S.router_host(sp), S.bias_host(sp), S.expert_host(sp, "shared")
 
 
-def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True, hold=None, reads=None):
+def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True, hold=None, reads=None,
+        predict=False):
     sp, pool, W, B, sh = layer
     cf = make_cfg(sp)
     cf.n_layers = 1
@@ -61,6 +62,8 @@ def run(L, layer, x, slots, n_io=0, prefetch_n=0, fails=(), shared=True, hold=No
     w.gate, w.bias, w.src, w.prefetch_n = W.ctypes.data, B.ctypes.data, C.pointer(c.src), prefetch_n
     w.sh_gate, w.sh_up, w.sh_down = [m if isinstance(m, glm53h.Glm53fMat) else fmat(*m, r, c, 128, 128) for m, (r, c) in
                                      zip(sh, [(sp.I, sp.E), (sp.I, sp.E), (sp.E, sp.I)])]
+    if predict:
+        w.next_gate, w.next_bias, w.prefill_next = W.ctypes.data, B.ctypes.data, 1
     drops = C.c_long.in_dll(L, "glm53f_expert_drops")
     was, outs = drops.value, []
     done = hold(c) if hold else None
@@ -100,6 +103,32 @@ def test_one_pass_is_the_chunks(L, layer, monkeypatch, T, mfma, n_io, prefetch_n
     idx, _ = O.router(O.oracle(), x[sel], sp, W, B)
     mats = {int(e): pool[int(e) % NP] for e in np.unique(idx)}
     within(got[sel], O.moe(O.oracle(), x[sel], sp, W, B, mats, sh if shared else None)[0], f"T={T}")
+
+
+def test_several_passes_are_the_chunks(L, layer):
+    """More tokens than one planning pass takes: two passes, then one token that decodes."""
+    say("cached prompt, several passes")
+    sp = layer[0]
+    x = np.ascontiguousarray(S.x_host(sp, 2048 + 129, batch=12), np.float32)
+    want, gets, _ = run(L, layer, x, sp.NE - 5)
+    got, gets1, lost = run(L, layer, x, sp.NE + 64)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    assert gets1 == gets and lost == 0
+
+
+@pytest.mark.parametrize("mfma", [False, True])
+def test_next_layer_prediction_in_a_pass(L, layer, monkeypatch, mfma):
+    """Hints for the next layer from each chunk's own prediction, made inside the pass: the reads they start
+    change nothing."""
+    say("cached prompt, next layer predicted", "mfma" if mfma else "octet")
+    if mfma:
+        monkeypatch.setenv("GLM53F_CACHE_MFMA", "1")
+    sp = layer[0]
+    x = np.ascontiguousarray(S.x_host(sp, 130, batch=13), np.float32)
+    want, gets, _ = run(L, layer, x, sp.NE - 5, n_io=2, prefetch_n=6, predict=True)
+    got, gets1, lost = run(L, layer, x, 2 * sp.NE + 64, n_io=2, prefetch_n=6, predict=True)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    assert gets1 == gets and lost == 0
 
 
 def test_failed_get_is_the_chunks_drop(L, layer):

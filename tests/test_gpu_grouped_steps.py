@@ -61,6 +61,25 @@ def test_grouped_unaligned_codes(L, shift, T, tiled):
     assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("E,inter,T", [(512, 512, 2), (512, 4096, 33), (4096, 512, 65), (1024, 2048, 130), (2048, 1024, 5)])
+def test_grouped_mfma_tiled(L, E, inter, T):
+    """MFMA-tiled experts (the drop-in's cache may hold them), whose addresses depend on both sizes: bit for
+    bit the row-major layer."""
+    say("grouped, MFMA-tiled", E, inter, T)
+    sp = S.LayerSpec(E=E, I=inter, NE=4, K=3, router_sigma=0.02)
+    x = S.x_host(sp, T, batch=5)
+    want, wi, ww = run(S.DeviceLayer.build(sp), x, 1, "g53h_moe_grouped")
+    layer = S.DeviceLayer.build(sp, mfma=True)
+    begin = L.g53h_grouped_begin_layout
+    begin.argtypes, begin.restype = [C.c_void_p, C.c_int, C.POINTER(glm53h.G53hMoeLayer), C.c_void_p, C.c_int], C.c_int
+    xd, od, id_, wd = DevBuf.from_array(x), DevBuf(x.nbytes), DevBuf.from_array(wi), DevBuf.from_array(ww)
+    check(begin(xd.ptr, T, C.byref(layer.layer), id_.ptr, 2), "begin")
+    check(L.g53h_grouped_batch(C.byref(layer.layer)), "batch")
+    check(L.g53h_grouped_end(od.ptr, wd.ptr), "end")
+    assert L.g53h_grouped_errors() == 0
+    assert np.array_equal(od.download(np.uint32).reshape(x.shape), want.view(np.uint32))
+
+
 def test_trace_stays_in_its_buffer(L):
     """g53h_set_grouped_trace writes 8 words for each gate/up item and nothing after them."""
     say("grouped trace")

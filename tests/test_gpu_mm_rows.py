@@ -1,6 +1,7 @@
 """The row-tile matrix product (g53h_mm_f8 on FP8 matrices with 128-column blocks, replaces
 src/core/glm53f_ops.c:185-228): bit-exact with the oracle at the edges of its tiles of 64 rows,
-128 columns and up to four tokens, and for matrices that are not 16-byte aligned."""
+128 columns and up to two tokens, for matrices that are not 16-byte aligned, and either side of the
+line to a thread per row for narrow ones."""
 import ctypes as C
 
 import numpy as np
