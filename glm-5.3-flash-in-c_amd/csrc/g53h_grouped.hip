@@ -293,7 +293,7 @@ k_grp_prep(const int *__restrict__ idx, int T, int K, int NE, int has_sh, int *_
 /* Both GEMMs share one pipeline. A workgroup is 8 waves and stays for the whole launch, one per
  * CU; it walks its items (256 weight rows x one tile) as one stream of steps of 128 weight columns.
  * A step's operands - 256 rows x 128 codes, and the tile's positions x 128 codes x 2 planes - go
- * straight to LDS (global_load_lds, 1 KB a wave instruction), into a ring of three slots, two steps
+ * straight to LDS (global_load_lds, 1 KB a wave instruction), into a ring of three slots, three steps
  * ahead, across item boundaries: no registers hold loads in flight, every code is fetched as part
  * of a whole 128-byte run, and one barrier per step hands a slot over. The waits count loads by
  * hand, so the loads are inline assembly: the compiler would wait for every LDS load before any
@@ -382,7 +382,7 @@ struct G53GrpArgs {
                                       segment | tiles of the segment << 16}                */
     const int *meta;               /* [0] tile count, [1] error flags                    */
     int *meta_w;
-    const int *tok_of;             /* position -> token (readable 8 past the last)       */
+    const int *tok_of;             /* [P]: position -> token                             */
     const uint8_t *xq;             /* [NPX][T][E]                                        */
     const float *xinv;             /* [T]: the tokens' scales                            */
     uint8_t *aq;                   /* [NPA][P][I]                                        */
@@ -827,7 +827,7 @@ static int g53_grp_shapes_ok(const G53hMoeLayer *L)
 
 extern "C" int g53h_grouped_ok(const G53hMoeLayer *L)
 {
-    /* the grouped kernels read row-major or octet-tiled experts, not MFMA-tiled ones */
+    /* MFMA-tiled experts are taken through g53h_grouped_begin_layout only */
     return L && L->router && L->bias && (L->tiled == 0 || L->tiled == 1) && g53_grp_shapes_ok(L);
 }
 

@@ -34,8 +34,9 @@ __global__ void k_mm_f8_generic(float *__restrict__ y, const float *__restrict__
 /* The same product for FP8 matrices with 128-column blocks (row-major codes, any rows, columns,
  * alignment and scale rows), TG tokens at a time. A workgroup owns 64 rows x TG tokens; wave w
  * takes column blocks w, w + NW, ... and lane r row r, so a weight is decoded once for TG tokens
- * and x is the same for every lane: scalar loads, requested a group ahead of its products, and no
- * LDS traffic in the inner loop. A wave loads its block's 64 x 128 codes as whole 128-byte runs (8
+ * and x is the same for every lane: scalar loads, two groups a request and asked for one group's
+ * products ahead (they return in any order, so a wait is for all of them), and no LDS traffic in
+ * the inner loop. A wave loads its block's 64 x 128 codes as whole 128-byte runs (8
  * lanes a row), a round ahead, and turns them through 4 KB of LDS, 32 rows at a time; 16-byte
  * pieces are swizzled by row pairs, so that 16 lanes meet no bank twice. Each block's scaled
  * double sum goes to LDS, and the thread that owns (row, token) adds a round's NW sums in block
@@ -125,7 +126,8 @@ __global__ void __launch_bounds__(64 * NW, 4) k_mm_f8_rows(float *__restrict__ y
             }
             if (b + NW < nb) load(b + NW);
             if (W == 128) {
-                /* a group's x is requested while the group before it is multiplied */
+                /* a group's x is requested while the group before it is multiplied (the compiler asks for two
+                 * groups at once, every other time) */
                 xload(xv[0], b * 128);
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
