@@ -196,28 +196,34 @@ extern "C" int g53h_mm_f8(float *y, const float *x, int T, const G53hMat *m)
      * token 3.8 / 4.9, 24 tokens 4.3 / 10.3; 4096 x 17, 300: 8.2 / 62.4; 2048 x 112, 64: 4.7 / 7.3; aligned and
      * one workgroup a CU, 4096 x 112, 1: 3.7 / 3.6), and unaligned rows of 136 to 207 in whole tiles (4096 x 136,
      * 24: 5.0 / 8.2; 4096 x 200, 64: 13.8 / 16.6; 129 columns, 64: 20.3 / 16.3; 250, 64: 23.8 / 20.6). */
-    const long tiles = (m->rows + 63) / 64;
+    const long tiles = ((long)m->rows + 63) / 64;
     const int al = m->cols % 16 == 0 && ((uintptr_t)m->w & 15) == 0, one = tiles * T <= g53h_num_cus();
     const int narrow = m->cols < 128 ? !(al && one)
                                      : !al && !one && m->rows % 64 == 0 && m->cols >= 136 && m->cols < 208;
-    if (m->flags == 0 && m->bc == 128 && !narrow) {
-        const long wgs = tiles * (one ? T : (T + 1) / 2);
-        if (wgs > 0x7fffffffL) return g53h_fail("g53h_mm_f8: %d rows x %d tokens", m->rows, T);
-        const dim3 g((unsigned)wgs);
-        hipStream_t st = g53h_stream();
-#define G53_MM(TG, NW, AL) hipLaunchKernelGGL((k_mm_f8_rows<TG, NW, AL>), g, dim3(64 * NW), 0, st, y, x, T, *m)
+    const long per_tile = 0xffffffffL / (one ? 1024 : 512) / tiles * (one ? 1 : 2);
+    const int tile = m->flags == 0 && m->bc == 128 && !narrow && per_tile > 0;
+    /* a launch holds fewer than 2^32 threads (more are cut off without an error): tokens in slices */
+    const long per = tile ? per_tile : 0xffffff00L / m->rows;
+    hipStream_t st = g53h_stream();
+    for (long t0 = 0; t0 < T; t0 += per) {
+        const int n = (int)(T - t0 < per ? T - t0 : per);
+        float *ys = y + (size_t)t0 * m->rows;
+        const float *xs = x + (size_t)t0 * m->cols;
+        if (!tile) {
+            hipLaunchKernelGGL(k_mm_f8_generic, dim3((unsigned)(((long)n * m->rows + 127) / 128)), dim3(128), 0, st, ys, xs,
+                               n, *m);
+            G53_LAUNCHED("k_mm_f8_generic");
+            continue;
+        }
+        const dim3 g((unsigned)(tiles * (one ? n : (n + 1) / 2)));
+#define G53_MM(TG, NW, AL) hipLaunchKernelGGL((k_mm_f8_rows<TG, NW, AL>), g, dim3(64 * NW), 0, st, ys, xs, n, *m)
         if (one && al) G53_MM(1, 16, true);
         else if (one) G53_MM(1, 16, false);
         else if (al) G53_MM(2, 8, true);
         else G53_MM(2, 8, false);
 #undef G53_MM
         G53_LAUNCHED("k_mm_f8_rows");
-        return 0;
     }
-    const long n = (long)T * m->rows;
-    hipLaunchKernelGGL(k_mm_f8_generic, dim3((unsigned)((n + 127) / 128)), dim3(128), 0,
-                       g53h_stream(), y, x, T, *m);
-    G53_LAUNCHED("k_mm_f8_generic");
     return 0;
 }
 

@@ -44,6 +44,32 @@ def test_mm_f8_rows(L, rows, cols, br, T, shift):
     assert same(got[:-1].reshape(T, rows), O.mm_f8(O.oracle(), x, w, s, rows, cols, br, 128))
 
 
+@pytest.mark.parametrize("cols,T", [(128, 262151), (16, 1048583)])
+def test_mm_f8_more_outputs_than_a_grid_holds(L, cols, T):
+    """So many tokens x 4096 rows that one launch has too few threads for them, by row tiles and by threads. A
+    block of tokens repeated gives its result repeated, at both ends and on both sides of every multiple of
+    2^16 tokens."""
+    say("mm, more than a grid", cols, T)
+    rows, n = 4096, 4099
+    rng = np.random.default_rng(11)
+    w = rng.integers(0, 256, rows * cols).astype(np.uint8)
+    w[(w & 0x7f) == 0x7f] ^= 1
+    s = rng.uniform(1e-3, 1e-1, rows // 128).astype(np.float32)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    wd, sd, xd, yd = DevBuf.from_array(w), DevBuf.from_array(s), DevBuf(T * cols * 4), DevBuf(T * rows * 4)
+    for t in range(0, T, n):
+        check(L.g53h_h2d(xd.ptr + t * cols * 4, x.ctypes.data, min(n, T - t) * cols * 4), "h2d")
+    m = G53hMat(wd.ptr, sd.ptr, rows, cols, 128, 128, 1, 0)
+    check(L.g53h_mm_f8(yd.ptr, xd.ptr, T, C.byref(m)), "mm")
+    check(L.g53h_sync(), "sync")
+    at = sorted({t for e in range(0, T, 1 << 16) for t in range(e - 2, e + 3) if t >= 0} | {T - 2, T - 1})
+    want = O.mm_f8(O.oracle(), np.ascontiguousarray(x[[t % n for t in at]]), w, s, rows, cols, 128, 128)
+    got = np.empty((len(at), rows), np.float32)
+    for i, t in enumerate(at):
+        check(L.g53h_d2h(got[i].ctypes.data, yd.ptr + t * rows * 4, rows * 4), "d2h")
+    assert same(got, want)
+
+
 @pytest.mark.parametrize("flags", [2, 8, 4 | 8, 4 | 16])
 def test_mm_f8_refuses_tiled_codes(L, flags):
     say("mm, tiled codes", flags)
