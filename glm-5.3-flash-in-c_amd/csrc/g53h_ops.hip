@@ -677,7 +677,8 @@ int g53h_router_into(int *idx, float *w, const float *x, int T, const void *gate
          * 8192: 47.9 / 43.9; the 32 x 32 kernel before: 54.8, 52.1, 43.8), and where a grid has too few rows for
          * the tokens. More expert tiles gain nothing (288 x 4096, 2048: 102.3 / 102.7; 192 x 4096, 8192: 255.1 /
          * 254.9), smaller batches lose the index arithmetic's time (288 x 4096, 5: 11.7 / 12.0). */
-        const int tt = (T + 15) / 16, flat = (NE <= 160 && (long)T * E >= (8 << 20)) || tt > 65535;
+        const int tt = (T + 15) / 16, fits = (long)tiles * S < (1 << 24) - 8;        /* 2^32 threads a launch */
+        const int flat = fits && ((NE <= 160 && (long)T * E >= (8 << 20)) || tt > 65535);
         const dim3 grid = flat ? dim3((unsigned)(tiles * S + 7) / 8 * 8) : dim3((NE + 15) / 16, tt, S);
         hipLaunchKernelGGL(k_router_mfma, grid, dim3(256), 0, g53h_stream(), score, choice, x, T,
                            (const uint16_t *)gate, bias, NE, E, E / S, flat ? S : 0, part);
